@@ -33,19 +33,17 @@ namespace dmv {
 // (block masses and their prefix) and allocates nothing.
 int sample_to_device(dmv_state *s, int64_t k, uint64_t seed, const double *d_u, int64_t *d_out)
 {
+    prof_begin(DMV_KC_SAMPLE);
+    DMV_TRY(launch_sample(s->dtype, s->amp, s->n, s->layout, k, seed, d_u, s->cum, s->ws, d_out));
+    prof_end(DMV_KC_SAMPLE, (double)s->bytes);
     // the reference panics when it cannot sample (circuit.rs:478-482): refuse a zero state
     const int bb = s->n < 12 ? s->n : 12;
-    DMV_TRY(launch_block_norms(s->dtype, s->amp, s->n, s->layout, bb, s->ws));
-    DMV_TRY(launch_sum(s->ws, uint64_t(1) << (s->n - bb), s->scalars));
     double total = 0.0;
-    DMV_TRY(copy_d2h(&total, s->scalars, sizeof(double)));
+    DMV_TRY(copy_d2h(&total, s->cum + ((uint64_t(1) << (s->n - bb)) - 1), sizeof(double)));
     if (!(total > 0.0 && std::isfinite(total))) {
         set_error("could not sample from output distribution (total probability %g)", total);
         return DMV_ERR_STATE;
     }
-    prof_begin(DMV_KC_SAMPLE);
-    DMV_TRY(launch_sample(s->dtype, s->amp, s->n, s->layout, k, seed, d_u, s->cum, s->ws, d_out));
-    prof_end(DMV_KC_SAMPLE, (double)s->bytes);
     return DMV_OK;
 }
 }  // namespace dmv

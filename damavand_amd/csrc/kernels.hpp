@@ -76,8 +76,9 @@ int launch_join(int dtype, void *state, StateLayout L, uint64_t begin, uint64_t 
 int launch_probs(int dtype, const void *state, StateLayout L, uint64_t begin, uint64_t count, double *out);
 // Partial sums of |a|^2 over blocks of 2^block_bits amplitudes.
 int launch_block_norms(int dtype, const void *state, int n, StateLayout L, int block_bits, double *partials);
-// Deterministic single-workgroup sum of `count` doubles into *out (device).
-int launch_sum(const double *in, uint64_t count, double *out);
+// Deterministic sum of `count` doubles into *out (device); above 4096 of them
+// the 256 doubles behind are used too.
+int launch_sum(double *in, uint64_t count, double *out);
 int launch_expect_z(int dtype, const void *state, int n, StateLayout L, double *partials, double *out);
 int launch_expect_zz(int dtype, const void *state, int n, StateLayout L, const double *a, int n_pairs,
                      const int *pi, const int *pj, const double *b, double *partials, double *out);
@@ -97,6 +98,8 @@ int launch_obs_table(int dtype, const void *psi, void *lam, int n, StateLayout L
 // Row sums: out[slot_map ? slot_map[b] : b] = sum_t partials[b * n_tiles + t]
 // for b < n_rows.
 int launch_slot_sums(const double *partials, int n_rows, uint64_t n_tiles, const int *slot_map, double *out);
+// Samples; every out[i] is -1 where the total probability is not positive and
+// finite.
 int launch_sample(int dtype, const void *state, int n, StateLayout L, int64_t k, uint64_t seed, const double *u,
                   double *block_cum, double *partials, int64_t *out);
 
