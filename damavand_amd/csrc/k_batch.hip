@@ -56,23 +56,25 @@ __device__ __forceinline__ double chain_h(uint64_t x, uint32_t n, const double *
 
 // At most 168 VGPRs, so that three 256-thread workgroups share a CU.
 // STREAM: streaming loads and stores of the tile path's scratch states.
-template <class R, int RLOG, int TLOG, bool STREAM>
+// complex64 (S = float) is computed in FP64 as in the other tile kernels.
+template <class S, class R, int RLOG, int TLOG, bool STREAM>
 __global__ void __launch_bounds__(1 << TLOG) __attribute__((amdgpu_waves_per_eu(3)))
 k_batch(const BatchCircuit *__restrict__ circ, const uint32_t *__restrict__ order, uint32_t count,
         uint32_t *__restrict__ counter, const DevPass *__restrict__ passes, const DevPhase *__restrict__ phases,
         const DevOp *__restrict__ ops, const DevOp *__restrict__ sops, const double *__restrict__ coef,
-        typename Cplx<R>::T *__restrict__ scratch, uint64_t slot_amps, double *__restrict__ energy,
+        typename Cplx<S>::T *__restrict__ scratch, uint64_t slot_amps, double *__restrict__ energy,
         double *__restrict__ grad)
 {
     using V = typename Cplx<R>::T;
+    using ST = typename Cplx<S>::T;
     constexpr int K = RLOG + TLOG, NT = 1 << TLOG;
     __shared__ V lds[1 << K];
     __shared__ double red[NT / 64];
     __shared__ double acc[kBatchMaxIp * (NT / 64)];
     __shared__ uint32_t s_idx;
     const uint32_t tid = threadIdx.x;
-    V *psi = scratch + (uint64_t)blockIdx.x * 2 * slot_amps;
-    V *lam = psi + slot_amps;
+    ST *psi = scratch + (uint64_t)blockIdx.x * 2 * slot_amps;
+    ST *lam = psi + slot_amps;
     for (;;) {
         if (tid == 0)
             s_idx = atomicAdd(counter, 1u);
@@ -132,7 +134,7 @@ k_batch(const BatchCircuit *__restrict__ circ, const uint32_t *__restrict__ orde
         }
         // tile path over the workgroup's scratch states
         for (uint64_t i = tid; i < n_amp; i += NT) {
-            V z;
+            ST z;
             z.x = i == 0 ? 1 : 0;
             z.y = 0;
             psi[i] = z;
@@ -141,17 +143,17 @@ k_batch(const BatchCircuit *__restrict__ circ, const uint32_t *__restrict__ orde
         const uint64_t n_tiles = n_amp >> K;
         for (uint32_t p = C.fwd_begin; p < C.fwd_end; p++) {
             for (uint64_t t = 0; t < n_tiles; t++)
-                tile_body<R, RLOG, TLOG, STREAM>(psi, passes + p, phases, ops, t, lds, kPlainLayout);
+                tile_body<S, R, RLOG, TLOG, STREAM>(psi, passes + p, phases, ops, t, lds, kPlainLayout);
             __syncthreads();
         }
         double e = 0.0;
         for (uint64_t i = tid; i < n_amp; i += NT) {
             const double h = chain_h(i, n, a, b);
-            const V v = psi[i];
+            const ST v = psi[i];
             e += h * norm2(v);
-            V w2;
-            w2.x = v.x * (R)h;
-            w2.y = v.y * (R)h;
+            ST w2;
+            w2.x = v.x * h;
+            w2.y = v.y * h;
             lam[i] = w2;
         }
         e = block_sum<NT>(e, red);
@@ -160,7 +162,7 @@ k_batch(const BatchCircuit *__restrict__ circ, const uint32_t *__restrict__ orde
         __syncthreads();
         for (uint32_t p = C.adj_begin; p < C.adj_end; p++) {
             for (uint64_t t = 0; t < n_tiles; t++)
-                tile_body_adjoint<R, RLOG, TLOG, STREAM>(psi, lam, passes + p, phases, ops, t, lds, red,
+                tile_body_adjoint<S, R, RLOG, TLOG, STREAM>(psi, lam, passes + p, phases, ops, t, lds, red,
                                                  WaveAccSink{acc, NT / 64, t == 0}, kPlainLayout);
             __syncthreads();
             if (tid == 0)
@@ -172,14 +174,14 @@ k_batch(const BatchCircuit *__restrict__ circ, const uint32_t *__restrict__ orde
 
 __global__ void k_zero_u32(uint32_t *p) { *p = 0u; }
 
-template <class R, int RLOG, int TLOG, bool STREAM = false>
+template <class S, int RLOG, int TLOG, bool STREAM = false>
 static int run_batch(const BatchLaunch &L)
 {
-    using V = typename Cplx<R>::T;
+    using ST = typename Cplx<S>::T;
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, stream(), L.counter);
     DMV_TRY(check_launch("batch queue reset"));
-    hipLaunchKernelGGL((k_batch<R, RLOG, TLOG, STREAM>), dim3(L.grid), dim3(1 << TLOG), 0, stream(), L.circ, L.order, L.count,
-                       L.counter, L.passes, L.phases, L.ops, L.sops, L.coef, (V *)L.scratch, L.slot_amps, L.energy,
+    hipLaunchKernelGGL((k_batch<S, double, RLOG, TLOG, STREAM>), dim3(L.grid), dim3(1 << TLOG), 0, stream(), L.circ, L.order, L.count,
+                       L.counter, L.passes, L.phases, L.ops, L.sops, L.coef, (ST *)L.scratch, L.slot_amps, L.energy,
                        L.grad);
     return check_launch("batch kernel");
 }

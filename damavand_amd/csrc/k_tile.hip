@@ -14,7 +14,7 @@ namespace dmv {
 
 bool tile_half_exists(int dtype, int rlog, int tlog)
 {
-    return tlog == 8 && rlog == (dtype == DMV_C64 ? 5 : 4);
+    return tlog == 8 && (rlog == 4 || (rlog == 5 && dtype == DMV_C64));
 }
 
 int launch_tile(int dtype, int rlog, int tlog, bool nt, bool half, void *state, int n, StateLayout L,

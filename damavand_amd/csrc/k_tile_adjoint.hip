@@ -19,9 +19,9 @@ struct PartialSink {
     }
 };
 
-template <class R, int RLOG, int TLOG, bool NT>
+template <class S, class R, int RLOG, int TLOG, bool NT>
 __global__ void __launch_bounds__(1 << TLOG)
-k_tile_adjoint(typename Cplx<R>::T *__restrict__ psi, typename Cplx<R>::T *__restrict__ lam,
+k_tile_adjoint(typename Cplx<S>::T *__restrict__ psi, typename Cplx<S>::T *__restrict__ lam,
                const DevPass *__restrict__ passes, const DevPhase *__restrict__ phases,
                const DevOp *__restrict__ ops, uint32_t pass_idx, double *__restrict__ partials, StateLayout L)
 {
@@ -30,17 +30,18 @@ k_tile_adjoint(typename Cplx<R>::T *__restrict__ psi, typename Cplx<R>::T *__res
     __shared__ double red[(1 << TLOG) / 64];
     constexpr uint32_t W = (1u << TLOG) / 64;
     PartialSink sink{partials, (uint64_t)gridDim.x * W, (uint64_t)blockIdx.x * W};
-    tile_body_adjoint<R, RLOG, TLOG, NT>(psi, lam, passes + pass_idx, phases, ops, blockIdx.x, lds, red, sink, L);
+    tile_body_adjoint<S, R, RLOG, TLOG, NT>(psi, lam, passes + pass_idx, phases, ops, blockIdx.x, lds, red, sink, L);
 }
 
-template <class R, int RLOG, int TLOG, bool NT = false>
+// complex64 states are computed in FP64 as in the forward passes (tile_body).
+template <class S, int RLOG, int TLOG, bool NT = false>
 static int run_tile_adj(void *psi, void *lam, int n, StateLayout L, const DevPass *passes, const DevPhase *phases,
                         const DevOp *ops, uint32_t pass_idx, double *partials)
 {
-    using V = typename Cplx<R>::T;
+    using ST = typename Cplx<S>::T;
     const uint64_t tiles = uint64_t(1) << (n - (RLOG + TLOG));
-    hipLaunchKernelGGL((k_tile_adjoint<R, RLOG, TLOG, NT>), dim3((uint32_t)tiles), dim3(1 << TLOG), 0, stream(),
-                       (V *)psi, (V *)lam, passes, phases, ops, pass_idx, partials, L);
+    hipLaunchKernelGGL((k_tile_adjoint<S, double, RLOG, TLOG, NT>), dim3((uint32_t)tiles), dim3(1 << TLOG), 0, stream(),
+                       (ST *)psi, (ST *)lam, passes, phases, ops, pass_idx, partials, L);
     return check_launch("adjoint tile pass");
 }
 

@@ -8,9 +8,9 @@ namespace dmv {
 
 // HALF: half a tile of LDS (split transposes), so that three workgroups of
 // the 64 KiB tiles share a CU instead of two.
-template <class R, int RLOG, int TLOG, bool NT, bool HALF>
+template <class S, class R, int RLOG, int TLOG, bool NT, bool HALF>
 __global__ void __launch_bounds__(1 << TLOG)
-k_tile(typename Cplx<R>::T *__restrict__ state, const DevPass *__restrict__ passes,
+k_tile(typename Cplx<S>::T *__restrict__ state, const DevPass *__restrict__ passes,
        const DevPhase *__restrict__ phases, const DevOp *__restrict__ ops, uint32_t pass_idx, uint32_t xcd_log2,
        StateLayout L)
 {
@@ -22,24 +22,24 @@ k_tile(typename Cplx<R>::T *__restrict__ state, const DevPass *__restrict__ pass
     const uint32_t b = blockIdx.x;
     const uint64_t tile = xcd_log2 ? (uint64_t)(b & ((1u << xcd_log2) - 1)) * (gridDim.x >> xcd_log2) + (b >> xcd_log2)
                                    : (uint64_t)b;
-    tile_body<R, RLOG, TLOG, NT, HALF>(state, passes + pass_idx, phases, ops, tile, lds, L);
+    tile_body<S, R, RLOG, TLOG, NT, HALF>(state, passes + pass_idx, phases, ops, tile, lds, L);
 }
 
 // ------------------------------------------------------------- launchers --
-template <class R, int RLOG, int TLOG, bool HALF>
+template <class S, class R, int RLOG, int TLOG, bool HALF>
 static int run_tile(bool nt, void *state, int n, StateLayout L, const DevPass *passes, const DevPhase *phases, const DevOp *ops,
                     uint32_t pass_idx)
 {
-    using V = typename Cplx<R>::T;
+    using ST = typename Cplx<S>::T;
     const uint64_t tiles = uint64_t(1) << (n - (RLOG + TLOG));
     const int64_t xl = tune_value("tile_xcd_log2", 3);  // 8 XCDs per MI355X
     const uint32_t xcd_log2 = (xl > 0 && xl <= 4 && tiles >= (uint64_t(1) << xl)) ? (uint32_t)xl : 0u;
     if (nt)
-        hipLaunchKernelGGL((k_tile<R, RLOG, TLOG, true, HALF>), dim3((uint32_t)tiles), dim3(1 << TLOG), 0, stream(),
-                           (V *)state, passes, phases, ops, pass_idx, xcd_log2, L);
+        hipLaunchKernelGGL((k_tile<S, R, RLOG, TLOG, true, HALF>), dim3((uint32_t)tiles), dim3(1 << TLOG), 0, stream(),
+                           (ST *)state, passes, phases, ops, pass_idx, xcd_log2, L);
     else
-        hipLaunchKernelGGL((k_tile<R, RLOG, TLOG, false, HALF>), dim3((uint32_t)tiles), dim3(1 << TLOG), 0,
-                           stream(), (V *)state, passes, phases, ops, pass_idx, xcd_log2, L);
+        hipLaunchKernelGGL((k_tile<S, R, RLOG, TLOG, false, HALF>), dim3((uint32_t)tiles), dim3(1 << TLOG), 0,
+                           stream(), (ST *)state, passes, phases, ops, pass_idx, xcd_log2, L);
     return check_launch("tile pass");
 }
 
@@ -54,5 +54,8 @@ int launch_tile_c128_wave(int rlog, int tlog, bool nt, void *state, int n, State
                           const DevPhase *phases, const DevOp *ops, uint32_t pass_idx);
 int launch_tile_c64(int rlog, int tlog, bool nt, bool half, void *state, int n, StateLayout L, const DevPass *passes,
                     const DevPhase *phases, const DevOp *ops, uint32_t pass_idx);
+
+int launch_tile_c64_wide(int rlog, int tlog, bool nt, bool half, void *state, int n, StateLayout L,
+                         const DevPass *passes, const DevPhase *phases, const DevOp *ops, uint32_t pass_idx);
 
 }  // namespace dmv

@@ -311,9 +311,9 @@ PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const
     if (runs > pp.low_bits && runs <= 6)
         pp.low_bits = (int)runs;
     pp.swz_bits = dtype == DMV_C64 ? 4 : 3;
-    // defaults: 256 threads; k = 12 (complex128) / 13 (complex64) forward,
-    // 11 for reverse sweeps, which hold psi and lambda in registers together
-    int k = dtype == DMV_C64 ? (adjoint ? 11 : 13) : (adjoint ? 11 : 12);
+    // defaults: 256 threads; k = 12 forward, 11 for reverse sweeps, which hold
+    // psi and lambda in registers together
+    int k = adjoint ? 11 : 12;
     // streaming (nontemporal) loads and stores: forward passes from 2 GiB
     // states up (measured 1.5-3.5% faster per pass at 27, 30 and 33 qubits,
     // complex128, and slower at 24 qubits, where much of the state stays in

@@ -38,22 +38,26 @@ template <int TLOG> __device__ __forceinline__ uint64_t thread_global_offset(con
 // Moves the tile through LDS: register p of thread t is written at
 // swz(thread part in A) ^ src[p] and register r is read back from
 // swz(thread part in B) ^ dst[r].  The swizzle is linear, so these are
-// the swizzled local indices of (t, p) in A and (t, r) in B.
-template <class V, int NR, int TLOG>
+// the swizzled local indices of (t, p) in A and (t, r) in B.  The plan's
+// offsets count amplitudes of the state's storage type ST; complex64
+// amplitudes are complex128 ones in registers and LDS (see tile_body), at twice
+// the offset.
+template <class V, class ST, int NR, int TLOG>
 __device__ __forceinline__ void transpose(V (&v)[NR], V *lds, const DevLayout *A, const uint32_t *src,
                                           const DevLayout *B, const uint32_t *dst, uint32_t tid)
 {
-    constexpr int G = sizeof(V) == 16 ? 3 : 4;
+    constexpr int G = sizeof(ST) == 16 ? 3 : 4;
+    constexpr uint32_t SC = sizeof(V) / sizeof(ST);
     char *base = reinterpret_cast<char *>(lds);
-    const uint32_t la = swz_index<G>(thread_local_offset<TLOG>(A, tid)) * (uint32_t)sizeof(V);
+    const uint32_t la = swz_index<G>(thread_local_offset<TLOG>(A, tid)) * (uint32_t)sizeof(ST);
 #pragma unroll
     for (int r = 0; r < NR; r++)
-        *reinterpret_cast<V *>(base + (la ^ src[r])) = v[r];
+        *reinterpret_cast<V *>(base + (la ^ src[r]) * SC) = v[r];
     __syncthreads();
-    const uint32_t lb = swz_index<G>(thread_local_offset<TLOG>(B, tid)) * (uint32_t)sizeof(V);
+    const uint32_t lb = swz_index<G>(thread_local_offset<TLOG>(B, tid)) * (uint32_t)sizeof(ST);
 #pragma unroll
     for (int r = 0; r < NR; r++)
-        v[r] = *reinterpret_cast<const V *>(base + (lb ^ dst[r]));
+        v[r] = *reinterpret_cast<const V *>(base + (lb ^ dst[r]) * SC);
     __syncthreads();
 }
 
@@ -64,31 +68,32 @@ __device__ __forceinline__ void transpose(V (&v)[NR], V *lds, const DevLayout *A
 // from the host with that bit already removed, and removing a bit is linear,
 // so drop(la ^ src[p]) = drop(la) ^ src[p].  Every wave passes the same four
 // barriers; the rounds are uniform branches on the wave's half.
-template <class V, int NR, int TLOG>
+template <class V, class ST, int NR, int TLOG>
 __device__ __forceinline__ void transpose_half(V (&v)[NR], V *lds, const DevLayout *A, const uint32_t *src,
                                                const DevLayout *B, const uint32_t *dst, uint32_t split,
                                                uint32_t tid)
 {
     static_assert(TLOG >= 7, "the split bit must be a wave bit");
-    constexpr int G = sizeof(V) == 16 ? 3 : 4;
+    constexpr int G = sizeof(ST) == 16 ? 3 : 4;
+    constexpr uint32_t SC = sizeof(V) / sizeof(ST);
     char *base = reinterpret_cast<char *>(lds);
     const uint32_t la =
-        drop_bit(swz_index<G>(thread_local_offset<TLOG>(A, tid)) * (uint32_t)sizeof(V), split);
+        drop_bit(swz_index<G>(thread_local_offset<TLOG>(A, tid)) * (uint32_t)sizeof(ST), split);
     const uint32_t lb =
-        drop_bit(swz_index<G>(thread_local_offset<TLOG>(B, tid)) * (uint32_t)sizeof(V), split);
+        drop_bit(swz_index<G>(thread_local_offset<TLOG>(B, tid)) * (uint32_t)sizeof(ST), split);
     const uint32_t half = __builtin_amdgcn_readfirstlane(tid >> (TLOG - 1));
 #pragma unroll
     for (uint32_t h = 0; h < 2; h++) {
         if (half == h) {
 #pragma unroll
             for (int r = 0; r < NR; r++)
-                *reinterpret_cast<V *>(base + (la ^ src[r])) = v[r];
+                *reinterpret_cast<V *>(base + (la ^ src[r]) * SC) = v[r];
         }
         __syncthreads();
         if (half == h) {
 #pragma unroll
             for (int r = 0; r < NR; r++)
-                v[r] = *reinterpret_cast<const V *>(base + (lb ^ dst[r]));
+                v[r] = *reinterpret_cast<const V *>(base + (lb ^ dst[r]) * SC);
         }
         __syncthreads();
     }
@@ -457,36 +462,47 @@ template <int K> __device__ __forceinline__ uint64_t tile_base(const DevPass *P,
 // g (tile base and thread offset) and the register offsets have disjoint
 // bits, so the element of amplitude g | reg is elem(g) ^ elem(reg); greg holds
 // the register offsets already mapped to elements by the planner.
-template <bool NT, class V, int NR>
-__device__ __forceinline__ void load_tile(V (&v)[NR], const V *__restrict__ state, uint64_t g, const uint64_t *greg,
+template <bool NT, class V, class ST, int NR>
+__device__ __forceinline__ void load_tile(V (&v)[NR], const ST *__restrict__ state, uint64_t g, const uint64_t *greg,
                                           StateLayout L)
 {
     const uint64_t eg = elem(g, L);
+    ST w[NR];
 #pragma unroll
     for (int r = 0; r < NR; r++)
-        v[r] = ld<NT>(state + (eg ^ greg[r]));
+        w[r] = ld<NT>(state + (eg ^ greg[r]));
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        v[r].x = w[r].x;
+        v[r].y = w[r].y;
+    }
 }
 
-template <bool NT, class V, int NR>
-__device__ __forceinline__ void store_tile(const V (&v)[NR], V *__restrict__ state, uint64_t g, const uint64_t *greg,
+template <bool NT, class V, class ST, int NR>
+__device__ __forceinline__ void store_tile(const V (&v)[NR], ST *__restrict__ state, uint64_t g, const uint64_t *greg,
                                            StateLayout L)
 {
     const uint64_t eg = elem(g, L);
 #pragma unroll
-    for (int r = 0; r < NR; r++)
-        st<NT>(state + (eg ^ greg[r]), v[r]);
+    for (int r = 0; r < NR; r++) {
+        ST w;
+        w.x = v[r].x;
+        w.y = v[r].y;
+        st<NT>(state + (eg ^ greg[r]), w);
+    }
 }
 
 // Runs the phases of a pass on a loaded tile and leaves it in the store
 // layout.  HALF: lds holds half a tile and every transpose of the pass is
 // split (the host runs only such passes, or passes without transposes, on
 // these kernels).
-template <class R, int RLOG, int TLOG, bool HALF>
+template <class S, class R, int RLOG, int TLOG, bool HALF>
 __device__ __forceinline__ void process_tile(typename Cplx<R>::T (&v)[1 << RLOG], const DevPass *P,
                                              const DevPhase *__restrict__ phases, const DevOp *__restrict__ ops,
                                              typename Cplx<R>::T *lds)
 {
     using V = typename Cplx<R>::T;
+    using ST = typename Cplx<S>::T;
     constexpr int NR = 1 << RLOG;
     const uint32_t tid = threadIdx.x;
     const DevLayout *cur = &P->lay_ld;
@@ -494,24 +510,29 @@ __device__ __forceinline__ void process_tile(typename Cplx<R>::T (&v)[1 << RLOG]
         const DevPhase *D = phases + ph;
         if (D->transpose_in) {
             if constexpr (HALF)
-                transpose_half<V, NR, TLOG>(v, lds, cur, D->src_lswz, &D->lay, D->dst_lswz, P->split, tid);
+                transpose_half<V, ST, NR, TLOG>(v, lds, cur, D->src_lswz, &D->lay, D->dst_lswz, P->split, tid);
             else
-                transpose<V, NR, TLOG>(v, lds, cur, D->src_lswz, &D->lay, D->dst_lswz, tid);
+                transpose<V, ST, NR, TLOG>(v, lds, cur, D->src_lswz, &D->lay, D->dst_lswz, tid);
         }
         cur = &D->lay;
         run_ops<V, R, RLOG>(v, ops, D->op_begin, D->op_end, tid);
     }
     if (P->transpose_st) {
         if constexpr (HALF)
-            transpose_half<V, NR, TLOG>(v, lds, cur, P->st_src_lswz, &P->lay_st, P->st_dst_lswz, P->split, tid);
+            transpose_half<V, ST, NR, TLOG>(v, lds, cur, P->st_src_lswz, &P->lay_st, P->st_dst_lswz, P->split, tid);
         else
-            transpose<V, NR, TLOG>(v, lds, cur, P->st_src_lswz, &P->lay_st, P->st_dst_lswz, tid);
+            transpose<V, ST, NR, TLOG>(v, lds, cur, P->st_src_lswz, &P->lay_st, P->st_dst_lswz, tid);
     }
 }
 
-// One tile of a forward pass: load, run the phases, store.
-template <class R, int RLOG, int TLOG, bool NT, bool HALF = false>
-__device__ __forceinline__ void tile_body(typename Cplx<R>::T *__restrict__ state, const DevPass *P,
+// One tile of a forward pass: load, run the phases, store.  S: the state's
+// real type, R: the type it is computed in.  complex64 states are computed in
+// FP64: without packed FP32 instructions an FP32 operation takes a vector
+// instruction as an FP64 one does, so this costs registers and LDS only (16
+// amplitudes per thread instead of 32), a pass then rounds each amplitude once,
+// at its store, and the matrices are not rounded at all.
+template <class S, class R, int RLOG, int TLOG, bool NT, bool HALF = false>
+__device__ __forceinline__ void tile_body(typename Cplx<S>::T *__restrict__ state, const DevPass *P,
                                           const DevPhase *__restrict__ phases, const DevOp *__restrict__ ops,
                                           uint64_t tile, typename Cplx<R>::T *lds, StateLayout L)
 {
@@ -521,7 +542,7 @@ __device__ __forceinline__ void tile_body(typename Cplx<R>::T *__restrict__ stat
     const uint64_t g = tile_base<K>(P, tile);
     V v[NR];
     load_tile<NT>(v, state, g | thread_global_offset<TLOG>(P->gthr_ld, tid), P->greg_ld, L);
-    process_tile<R, RLOG, TLOG, HALF>(v, P, phases, ops, lds);
+    process_tile<S, R, RLOG, TLOG, HALF>(v, P, phases, ops, lds);
     store_tile<NT>(v, state, g | thread_global_offset<TLOG>(P->gthr_st, tid), P->greg_st, L);
 }
 
@@ -601,14 +622,15 @@ __device__ __forceinline__ void ip_sums(const V (&p)[1 << RLOG], const V (&l)[1 
 // two states (four register arrays, or three with one run of ops per state
 // between IP ops) needed more registers or twice the code and ran slower.
 // STREAM: streaming (nontemporal) loads and stores of both states.
-template <class R, int RLOG, int TLOG, bool STREAM = false, class Sink>
-__device__ __forceinline__ void tile_body_adjoint(typename Cplx<R>::T *__restrict__ psi,
-                                                  typename Cplx<R>::T *__restrict__ lam, const DevPass *P,
+template <class S, class R, int RLOG, int TLOG, bool STREAM = false, class Sink>
+__device__ __forceinline__ void tile_body_adjoint(typename Cplx<S>::T *__restrict__ psi,
+                                                  typename Cplx<S>::T *__restrict__ lam, const DevPass *P,
                                                   const DevPhase *__restrict__ phases,
                                                   const DevOp *__restrict__ ops, uint64_t tile,
                                                   typename Cplx<R>::T *lds, double *red, Sink sink, StateLayout L)
 {
     using V = typename Cplx<R>::T;
+    using ST = typename Cplx<S>::T;
     constexpr int NR = 1 << RLOG, K = RLOG + TLOG, NT = 1 << TLOG;
     const uint32_t tid = threadIdx.x;
     const uint64_t g = tile_base<K>(P, tile);
@@ -621,8 +643,8 @@ __device__ __forceinline__ void tile_body_adjoint(typename Cplx<R>::T *__restric
     for (uint32_t ph = P->phase_begin; ph < P->phase_end; ph++) {
         const DevPhase *D = phases + ph;
         if (D->transpose_in) {
-            transpose<V, NR, TLOG>(p, lds, cur, D->src_lswz, &D->lay, D->dst_lswz, tid);
-            transpose<V, NR, TLOG>(l, lds, cur, D->src_lswz, &D->lay, D->dst_lswz, tid);
+            transpose<V, ST, NR, TLOG>(p, lds, cur, D->src_lswz, &D->lay, D->dst_lswz, tid);
+            transpose<V, ST, NR, TLOG>(l, lds, cur, D->src_lswz, &D->lay, D->dst_lswz, tid);
         }
         cur = &D->lay;
         for (uint32_t o = D->op_begin; o < D->op_end; o++) {
@@ -659,8 +681,8 @@ __device__ __forceinline__ void tile_body_adjoint(typename Cplx<R>::T *__restric
         }
     }
     if (P->transpose_st) {
-        transpose<V, NR, TLOG>(p, lds, cur, P->st_src_lswz, &P->lay_st, P->st_dst_lswz, tid);
-        transpose<V, NR, TLOG>(l, lds, cur, P->st_src_lswz, &P->lay_st, P->st_dst_lswz, tid);
+        transpose<V, ST, NR, TLOG>(p, lds, cur, P->st_src_lswz, &P->lay_st, P->st_dst_lswz, tid);
+        transpose<V, ST, NR, TLOG>(l, lds, cur, P->st_src_lswz, &P->lay_st, P->st_dst_lswz, tid);
     }
     const uint64_t gs = g | thread_global_offset<TLOG>(P->gthr_st, tid);
     store_tile<STREAM>(p, psi, gs, P->greg_st, L);
