@@ -6,8 +6,10 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <string>
 #include <thread>
+#include <unordered_map>
 #include <vector>
 
 #include "device.hpp"
@@ -75,16 +77,19 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
     DMV_CHECK_ARG(per_cu >= 1 && per_cu <= 16, "batch_wgs_per_cu must be in [1, 16], got %d", per_cu);
     const int small_max = K - 1;
 
-    // Per-circuit plans are independent: build them on host threads, then
-    // concatenate in circuit order (the result does not depend on threading).
+    // Circuits with the same gates on the same qubits share one plan: their
+    // ops differ in matrices only.  Lowering (matrices), planning and filling
+    // in run on host threads; the result does not depend on threading.
     struct Built {
         int rc = DMV_OK;
         std::string err;
         int np = 0;
         double cost = 0.0;
         bool small = false;
-        std::vector<DevOp> fo, ao;
-        Plan pf, pa;
+        int like = -1;                 // the first circuit of the same structure (perhaps itself)
+        std::vector<HostOp> f, a;      // merged ops
+        Plan pf, pa;                   // tile path, where like is the circuit itself
+        uint32_t fwd = 0, adj = 0;     // ... its first passes among all
     };
     std::vector<Built> built(count);
     PlanParams pp0;
@@ -93,11 +98,15 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
     pp0.tlog = tlog;
     pp0.low_bits = coalesce_bits(dtype);
     pp0.swz_bits = dtype == DMV_C64 ? 4 : 3;
-    pp0.max_gen_per_pass = (int)tune_value("max_gen_per_pass", 8);
-    auto build_one = [&](int i, Built &B) -> int {
+    const int64_t gen = tune_value("max_gen_per_pass", -1);
+    pp0.max_gen_per_pass = gen > 0 ? (int)gen : 8;
+    pp0.gen_auto = gen > 0 ? 0 : 1;
+    pp0.max_ip_per_pass = (int)kBatchMaxIp;
+    auto lower = [&](int i, Built &B) -> int {
         const int ni = n[i];
         DMV_CHECK_ARG(ni >= 2 && ni <= 24, "batch circuit %d: qubits must be in [2, 24], got %d", i, ni);
         std::vector<Gate> gates;
+        gates.reserve((size_t)(gate_offset[i + 1] - gate_offset[i]));
         for (int g = gate_offset[i]; g < gate_offset[i + 1]; g++) {
             Gate G;
             G.kind = gate_kind[g];
@@ -119,35 +128,31 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
         for (const Gate &G : gates)
             if (gate_is_parametric(G.kind))
                 B.np++;
-        std::vector<HostOp> f = merge_ops(forward_ops(gates));
-        std::vector<HostOp> a = merge_ops(adjoint_ops(gates));
-        B.cost = (double)(f.size() + a.size()) * std::ldexp(1.0, ni);
+        B.f = merge_ops(forward_ops(gates));
+        B.a = merge_ops(adjoint_ops(gates));
+        B.cost = (double)(B.f.size() + B.a.size()) * std::ldexp(1.0, ni);
         B.small = ni <= small_max;
-        if (B.small) {
-            B.fo = global_dev_ops(f);
-            B.ao = global_dev_ops(a);
-            return DMV_OK;
-        }
+        return DMV_OK;
+    };
+    auto plan_one = [&](int i, Built &B) -> int {
         PlanParams pp = pp0;
-        pp.n = ni;
-        DMV_TRY(build_plan(f, pp, &B.pf));
-        DMV_TRY(build_plan(a, pp, &B.pa));
+        pp.n = n[i];
+        DMV_TRY(build_plan(B.f, pp, &B.pf));
+        DMV_TRY(build_plan(B.a, pp, &B.pa));
         for (size_t p = 0; p + 1 < B.pa.ip_begin.size(); p++)
             DMV_CHECK_ARG(B.pa.ip_begin[p + 1] - B.pa.ip_begin[p] <= kBatchMaxIp,
                           "batch circuit %d: %u parameters in one reverse pass (at most %u)", i,
                           B.pa.ip_begin[p + 1] - B.pa.ip_begin[p], kBatchMaxIp);
         return DMV_OK;
     };
-    {
+    // fn(i) for i < total, on up to 16 threads taking `grain` at a time or more
+    auto on_threads = [](int total, int grain, const std::function<void(int)> &fn) {
         const int hw = (int)std::max(1u, std::thread::hardware_concurrency());
-        const int nthreads = std::max(1, std::min({hw, 16, (count + 31) / 32}));
+        const int nthreads = std::max(1, std::min({hw, 16, total / grain}));
         std::atomic<int> next{0};
         auto worker = [&]() {
-            for (int i = next.fetch_add(1); i < count; i = next.fetch_add(1)) {
-                built[i].rc = build_one(i, built[i]);
-                if (built[i].rc != DMV_OK)
-                    built[i].err = last_error();
-            }
+            for (int i = next.fetch_add(1); i < total; i = next.fetch_add(1))
+                fn(i);
         };
         std::vector<std::thread> pool;
         for (int t = 1; t < nthreads; t++)
@@ -155,15 +160,55 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
         worker();
         for (std::thread &t : pool)
             t.join();
+    };
+    on_threads(count, 16, [&](int i) {
+        built[i].rc = lower(i, built[i]);
+        if (built[i].rc != DMV_OK)
+            built[i].err = last_error();
+    });
+    for (int i = 0; i < count; i++)
+        if (built[i].rc != DMV_OK) {
+            set_error("%s", built[i].err.c_str());
+            return built[i].rc;
+        }
+    std::vector<int> firsts;  // circuits of a new structure, tile path
+    {
+        std::unordered_multimap<uint64_t, int> seen;
+        for (int i = 0; i < count; i++) {
+            Built &B = built[i];
+            if (B.small)
+                continue;
+            uint64_t h = (uint64_t)n[i];
+            for (const std::vector<HostOp> *v : {&B.f, &B.a})
+                for (const HostOp &op : *v)
+                    h = (h ^ (op.kind + 16 * (uint64_t)op.target + 1024 * (op.ctrl + 1))) * 0x9E3779B97F4A7C15ull;
+            const auto range = seen.equal_range(h);
+            for (auto it = range.first; it != range.second && B.like < 0; ++it) {
+                const Built &O = built[it->second];
+                if (n[it->second] == n[i] && same_structure(O.f, B.f) && same_structure(O.a, B.a))
+                    B.like = it->second;
+            }
+            if (B.like < 0) {
+                B.like = i;
+                seen.emplace(h, i);
+                firsts.push_back(i);
+            }
+        }
     }
+    on_threads((int)firsts.size(), 2, [&](int j) {
+        Built &B = built[firsts[(size_t)j]];
+        B.rc = plan_one(firsts[(size_t)j], B);
+        if (B.rc != DMV_OK)
+            B.err = last_error();
+    });
 
     std::vector<BatchCircuit> circ(count);
     std::vector<DevPass> passes;
     std::vector<DevPhase> phases;
-    std::vector<DevOp> ops, sops;
     std::vector<double> cost(count);
     int nmax = 1;
     int64_t total_params = 0;
+    uint64_t n_ops = 0, n_sops = 0;
     for (int i = 0; i < count; i++) {
         Built &B = built[i];
         if (B.rc != DMV_OK) {
@@ -183,43 +228,59 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
         C.coef = (uint32_t)coef_offset[i];
         C.grad = (uint32_t)param_offset[i];
         cost[i] = B.cost;
+        C.small = B.small ? 1u : 0u;
         if (B.small) {
-            C.small = 1;
-            C.fwd_begin = (uint32_t)sops.size();
-            sops.insert(sops.end(), B.fo.begin(), B.fo.end());
-            C.fwd_end = (uint32_t)sops.size();
-            C.adj_begin = (uint32_t)sops.size();
-            sops.insert(sops.end(), B.ao.begin(), B.ao.end());
-            C.adj_end = (uint32_t)sops.size();
-        } else {
-            C.small = 0;
+            C.fwd_begin = (uint32_t)n_sops;
+            C.fwd_end = C.adj_begin = C.fwd_begin + (uint32_t)B.f.size();
+            C.adj_end = C.adj_begin + (uint32_t)B.a.size();
+            C.fwd_ops = C.adj_ops = 0;
+            n_sops = C.adj_end;
+            continue;
+        }
+        if (B.like == i) {
             for (int which = 0; which < 2; which++) {
                 const Plan &plan = which == 0 ? B.pf : B.pa;
-                const uint32_t pbase = (uint32_t)passes.size();
+                (which == 0 ? B.fwd : B.adj) = (uint32_t)passes.size();
                 const uint32_t phbase = (uint32_t)phases.size();
-                const uint32_t obase = (uint32_t)ops.size();
                 for (DevPass P : plan.passes) {
                     P.phase_begin += phbase;
                     P.phase_end += phbase;
                     passes.push_back(P);
                 }
-                for (DevPhase D : plan.phases) {
-                    D.op_begin += obase;
-                    D.op_end += obase;
-                    phases.push_back(D);
-                }
-                ops.insert(ops.end(), plan.ops.begin(), plan.ops.end());
-                if (which == 0) {
-                    C.fwd_begin = pbase;
-                    C.fwd_end = (uint32_t)passes.size();
-                } else {
-                    C.adj_begin = pbase;
-                    C.adj_end = (uint32_t)passes.size();
-                }
+                phases.insert(phases.end(), plan.phases.begin(), plan.phases.end());
             }
         }
-        B = Built();  // release the per-circuit copies early
+        const Built &T = built[B.like];
+        C.fwd_begin = T.fwd;
+        C.fwd_end = T.fwd + (uint32_t)T.pf.passes.size();
+        C.adj_begin = T.adj;
+        C.adj_end = T.adj + (uint32_t)T.pa.passes.size();
+        C.fwd_ops = n_ops;
+        C.adj_ops = n_ops + T.pf.ops.size();
+        n_ops += T.pf.ops.size() + T.pa.ops.size();
     }
+    std::vector<DevOp> ops((size_t)n_ops), sops((size_t)n_sops);
+    on_threads(count, 16, [&](int i) {
+        const Built &B = built[i];
+        const BatchCircuit &C = circ[i];
+        std::vector<DevOp> dev;
+        if (B.small) {
+            dev = global_dev_ops(B.f);
+            std::copy(dev.begin(), dev.end(), sops.begin() + C.fwd_begin);
+            dev = global_dev_ops(B.a);
+            std::copy(dev.begin(), dev.end(), sops.begin() + C.adj_begin);
+            return;
+        }
+        const Built &T = built[B.like];
+        dev = T.pf.ops;
+        refresh_ops(B.f, T.pf.op_src, &dev);
+        std::copy(dev.begin(), dev.end(), ops.begin() + (int64_t)C.fwd_ops);
+        dev = T.pa.ops;
+        refresh_ops(B.a, T.pa.op_src, &dev);
+        std::copy(dev.begin(), dev.end(), ops.begin() + (int64_t)C.adj_ops);
+    });
+    built.clear();
+    built.shrink_to_fit();
     std::vector<uint32_t> order(count);
     for (int i = 0; i < count; i++)
         order[i] = (uint32_t)i;

@@ -988,11 +988,9 @@ int dmv_circuit_tile_shape(dmv_circuit *c, int dtype, int adjoint, int *tile_qub
         *threads_log2 = pp.tlog;
     if (max_gen_per_pass) {
         *max_gen_per_pass = pp.max_gen_per_pass;
-        if (pp.gen_auto && c->n > pp.k) {
-            // chosen per circuit: the budget its forward plan takes
-            Plan plan;
-            DMV_TRY(build_plan(merge_ops(forward_ops(c->gates)), pp, &plan));
-            *max_gen_per_pass = plan.max_gen;
+        if (pp.gen_auto && !adjoint && c->n > pp.k) {
+            // no budget is set: the one that would suit the forward's gates in their order
+            DMV_TRY(in_order_budget(merge_ops(forward_ops(c->gates)), pp, max_gen_per_pass));
         }
     }
     if (nontemporal)

@@ -83,7 +83,7 @@ constexpr uint32_t kNoReg = 0xFFFFFFFFu;
 //  * ctrl_thr: controls that are thread bits (mask over the thread id);
 //  * plain: a GEN op acting on every register (en = all) whose first pair
 //    members (registers with the partner mask's highest bit clear) all hold
-//    target bit 0, so the matrix applies without per-pair selects; for a
+//    target bit 0; for a
 //    DIAG op: the diagonal is exactly diag(1, -1) (Z, CZ), so the op only
 //    flips the signs of the amplitudes whose target bit is 1; for an IP
 //    op: the previous op of the phase is an IP op of the same kind, target
@@ -99,7 +99,8 @@ struct alignas(16) DevOp {
     uint32_t ctrl_thr;
     uint64_t ctrl;     // every bit of ctrl must be 1 for the op to act
     uint32_t plain;
-    uint32_t ip_pos;   // IP op of a tile plan: its index among the IP ops of its pass
+    uint32_t aux;      // tile plans; an IP op: its index among the IP ops of its pass;
+                       // a GEN: 1 if m is special unitary (m11 = m00*, m01 = -m10*)
     double m[8];       // re/im of m00, m01, m10, m11
 };
 static_assert(sizeof(DevOp) == 112, "DevOp layout");

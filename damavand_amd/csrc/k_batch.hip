@@ -19,7 +19,7 @@ struct WaveAccSink {
     bool first;
     __device__ void operator()(const DevOp *op, double v, uint32_t wave) const
     {
-        double *a = acc + op->ip_pos * waves + wave;
+        double *a = acc + op->aux * waves + wave;
         *a = first ? v : *a + v;
     }
 };
@@ -36,7 +36,7 @@ __device__ __forceinline__ void flush_pass_grads(const DevPass *P, const DevPhas
                 continue;
             double s = 0.0;
             for (uint32_t w = 0; w < waves; w++)
-                s += acc[op->ip_pos * waves + w];
+                s += acc[op->aux * waves + w];
             g[op->slot] = s;
         }
 }
@@ -133,6 +133,7 @@ k_batch(const BatchCircuit *__restrict__ circ, const uint32_t *__restrict__ orde
             continue;
         }
         // tile path over the workgroup's scratch states
+        const DevOp *fops = ops + C.fwd_ops, *aops = ops + C.adj_ops;
         for (uint64_t i = tid; i < n_amp; i += NT) {
             ST z;
             z.x = i == 0 ? 1 : 0;
@@ -143,7 +144,7 @@ k_batch(const BatchCircuit *__restrict__ circ, const uint32_t *__restrict__ orde
         const uint64_t n_tiles = n_amp >> K;
         for (uint32_t p = C.fwd_begin; p < C.fwd_end; p++) {
             for (uint64_t t = 0; t < n_tiles; t++)
-                tile_body<S, R, RLOG, TLOG, STREAM>(psi, passes + p, phases, ops, t, lds, kPlainLayout);
+                tile_body<S, R, RLOG, TLOG, STREAM>(psi, passes + p, phases, fops, t, lds, kPlainLayout);
             __syncthreads();
         }
         double e = 0.0;
@@ -162,11 +163,11 @@ k_batch(const BatchCircuit *__restrict__ circ, const uint32_t *__restrict__ orde
         __syncthreads();
         for (uint32_t p = C.adj_begin; p < C.adj_end; p++) {
             for (uint64_t t = 0; t < n_tiles; t++)
-                tile_body_adjoint<S, R, RLOG, TLOG, STREAM>(psi, lam, passes + p, phases, ops, t, lds, red,
+                tile_body_adjoint<S, R, RLOG, TLOG, STREAM>(psi, lam, passes + p, phases, aops, t, lds, red,
                                                  WaveAccSink{acc, NT / 64, t == 0}, kPlainLayout);
             __syncthreads();
             if (tid == 0)
-                flush_pass_grads(passes + p, phases, ops, acc, NT / 64, g);
+                flush_pass_grads(passes + p, phases, aops, acc, NT / 64, g);
             __syncthreads();  // the next pass's first tile overwrites acc
         }
     }

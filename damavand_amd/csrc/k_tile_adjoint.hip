@@ -15,7 +15,7 @@ struct PartialSink {
     uint64_t per_ip, base;  // per_ip = tiles x waves, base = tile x waves
     __device__ void operator()(const DevOp *op, double v, uint32_t wave) const
     {
-        partials[(uint64_t)op->ip_pos * per_ip + base + wave] = v;
+        partials[(uint64_t)op->aux * per_ip + base + wave] = v;
     }
 };
 

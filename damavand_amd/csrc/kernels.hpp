@@ -39,6 +39,7 @@ struct BatchCircuit {
     uint32_t adj_begin, adj_end;
     uint32_t coef;                // a_q at coef[coef + q], b_q at coef[coef + n + q]
     uint32_t grad;                // gradient of parameter k at grad[grad + k]
+    uint64_t fwd_ops, adj_ops;    // tile path: the circuit's ops; phases count from there
 };
 struct BatchLaunch {
     const BatchCircuit *circ;

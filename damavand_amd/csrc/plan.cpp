@@ -312,6 +312,71 @@ std::vector<HostOp> merge_ops(const std::vector<HostOp> &ops)
     return out;
 }
 
+void special_unitary(std::vector<HostOp> *ops)
+{
+    double gr = 1.0, gi = 0.0;  // product of the phases taken out
+    double drop = 0.0;          // ... and the sum of the small ones
+    HostOp *general = nullptr;
+    for (HostOp &op : *ops) {
+        if (op.kind != OP_GEN || op.ctrl)
+            continue;
+        double *m = op.m;
+        double dr = m[0] * m[6] - m[1] * m[7] - m[2] * m[4] + m[3] * m[5];
+        double di = m[0] * m[7] + m[1] * m[6] - m[2] * m[5] - m[3] * m[4];
+        const double abs = std::hypot(dr, di);
+        if (!(std::abs(abs - 1.0) < 1e-12))
+            continue;  // not unitary: stays as it is
+        dr /= abs;
+        di /= abs;
+        // p = sqrt(det) by half angles (no cancellation), m / p is special unitary
+        const bool unit = std::abs(dr - 1.0) < 1e-13 && std::abs(di) < 1e-13;
+        double pr = 1.0, pi = 0.0;
+        if (!unit && dr >= 0.0) {
+            pr = std::sqrt(0.5 * (1.0 + dr));
+            pi = 0.5 * di / pr;
+        } else if (!unit) {
+            pi = std::sqrt(0.5 * (1.0 - dr));
+            pr = 0.5 * di / pi;
+        }
+        auto over = [&](double x, double y, double *re, double *im) {
+            *re = x * pr + y * pi;
+            *im = y * pr - x * pi;
+        };
+        // the mean of what m00 and m11*, m10 and -m01* say (equal up to rounding)
+        double ar, ai, cr, ci, br, bi, er, ei;
+        over(m[0], m[1], &ar, &ai);
+        over(m[6], m[7], &cr, &ci);
+        over(m[4], m[5], &br, &bi);
+        over(m[2], m[3], &er, &ei);
+        const double sr = 0.5 * (ar + cr), si = 0.5 * (ai - ci), tr = 0.5 * (br - er), ti = 0.5 * (bi + ei);
+        // the phase that the mean drops (about the rounding of p) goes with p
+        const double d = 0.5 * (sr * ai - si * ar + sr * ci + si * cr + tr * bi - ti * br - tr * ei - ti * er);
+        m[0] = sr; m[1] = si; m[2] = -tr; m[3] = ti;
+        m[4] = tr; m[5] = ti; m[6] = sr; m[7] = -si;
+        op.su2 = true;
+        // kept apart from p's product, which would round it away
+        drop += d;
+        if (!unit) {
+            const double t = gr * pr - gi * pi;
+            gi = gr * pi + gi * pr;
+            gr = t;
+        }
+        if (!general || !unit)
+            general = &op;
+    }
+    if (!general || (gr == 1.0 && gi == 0.0 && std::abs(drop) < 1e-16))
+        return;
+    const double t = gr - gi * drop;
+    gi += gr * drop;
+    gr = t;
+    general->su2 = false;
+    for (int i = 0; i < 4; i++) {
+        const double x = general->m[2 * i], y = general->m[2 * i + 1];
+        general->m[2 * i] = x * gr - y * gi;
+        general->m[2 * i + 1] = x * gi + y * gr;
+    }
+}
+
 static uint64_t op_qubits(const HostOp &op) { return (uint64_t(1) << op.target) | op.ctrl; }
 
 // Local index of a global bit mask: bit j of the result is qubit qpos[j].
@@ -435,66 +500,372 @@ static uint32_t first_members(uint32_t m, int nr)
     return f;
 }
 
-static int make_pass(uint64_t Q, const std::vector<HostOp> &taken, const PlanParams &pp, Plan *plan)
-{
-    DevPass P;
-    std::memset(&P, 0, sizeof(P));
-    P.k = (uint32_t)pp.k;
-    int nq = 0;
-    for (int q = 0; q < pp.n; q++)
-        if ((Q >> q) & 1)
-            P.qpos[nq++] = (uint32_t)q;
-    if (nq != pp.k) {
-        set_error("internal: pass has %d qubits, expected %d", nq, pp.k);
-        return DMV_ERR_STATE;
-    }
-    std::vector<HostOp> loc(taken.size());
-    for (size_t i = 0; i < taken.size(); i++) {
-        loc[i] = taken[i];
-        const uint64_t lt = to_local(uint64_t(1) << taken[i].target, P.qpos, pp.k);
-        loc[i].target = __builtin_ctzll(lt);
-        loc[i].ctrl = to_local(taken[i].ctrl, P.qpos, pp.k);
-    }
+// ------------------------------------------------------------- scheduling --
+// Ops as the scheduler sees them: which bits an op touches, and which bit must
+// be in registers.  Two ops that share a bit keep their order; ops on
+// disjoint bits commute.
+struct SchedOp {
+    uint64_t bits;     // target and controls
+    uint64_t ctrl;     // controls
+    int target;
+    uint32_t kind;
+    int weight;        // progress that running it counts for
+    int group;         // an IP op: how many its run of IP ops on the target has from here on
+};
 
-    // Register phases: greedy, keeping op order wherever ops share a qubit.
-    struct Ph {
-        uint32_t rs;
-        std::vector<int> ops;
-    };
-    std::vector<Ph> phs;
+// Every bit's ops in order, and how far each bit has got.  An op can run once
+// it is the next one of all its bits.
+struct Frontier {
+    const std::vector<SchedOp> *ops;
+    std::vector<int> list;      // op indices, bit after bit
+    int begin[kMaxQubits], end[kMaxQubits];  // each bit's range in `list`
+    int at[kMaxQubits];                      // ... and its next op
+
+    void build(const std::vector<SchedOp> &o, int n)
+    {
+        ops = &o;
+        int count[kMaxQubits] = {};
+        for (const SchedOp &op : o)
+            for (uint64_t m = op.bits; m; m &= m - 1)
+                count[__builtin_ctzll(m)]++;
+        int total = 0;
+        for (int q = 0; q < kMaxQubits; q++) {
+            begin[q] = end[q] = at[q] = total;
+            total += q < n ? count[q] : 0;
+        }
+        list.resize((size_t)total);
+        for (size_t i = 0; i < o.size(); i++)
+            for (uint64_t m = o[i].bits; m; m &= m - 1)
+                list[(size_t)end[__builtin_ctzll(m)]++] = (int)i;
+    }
+    int next(const int *pos, int q) const { return pos[q] < end[q] ? list[(size_t)pos[q]] : -1; }
+};
+
+// What a pass or phase may hold.
+struct SchedLimits {
+    int max_gen = 1 << 30;      // general 2x2 ops
+    int max_ip = 1 << 30;       // IP ops (an op of a run is counted with the rest of its run)
+    int max_high_targets = 64;  // register targets outside `low`
+    uint64_t low = 0;
+};
+
+// A trial: the bits it may use, how far it has got, and what it holds.
+struct Trial {
+    uint64_t bits = 0;      // pass: the tile's qubits; phase: the register bits
+    int pos[kMaxQubits];
+    int score = 0, gen = 0, ip = 0;
+    uint64_t targets = 0;   // bits that need a register
+};
+
+// Whether op i, the next one of bit q, can run now.  Passes: all its bits must
+// be in the tile.  Phases: the target of a pair op must be a register bit, and
+// with `renames_only` an X or CNOT also needs its control in registers (it
+// then only relabels registers).
+template <bool PHASE>
+static bool can_run(const Frontier &F, const SchedLimits &lim, bool renames_only, const Trial &t, int i)
+{
+    const SchedOp &op = (*F.ops)[(size_t)i];
+    if constexpr (PHASE) {
+        if (op_needs_register(op.kind) &&
+            (!((t.bits >> op.target) & 1) || (renames_only && op.kind == OP_SWAP && (op.ctrl & ~t.bits))))
+            return false;
+    } else {
+        if (op.bits & ~t.bits)
+            return false;
+    }
+    for (uint64_t m = op.bits; m; m &= m - 1)
+        if (F.next(t.pos, __builtin_ctzll(m)) != i)
+            return false;
+    if constexpr (!PHASE) {
+        const uint64_t targets = op_needs_register(op.kind) ? t.targets | (uint64_t(1) << op.target) : t.targets;
+        return !(op.kind == OP_GEN && t.gen >= lim.max_gen) &&
+               !(op.group > 0 && t.ip > 0 && t.ip + op.group > lim.max_ip) &&
+               popcount64(targets & ~lim.low) <= lim.max_high_targets;
+    }
+    return true;
+}
+
+// Runs every op that the trial's bits allow.  `dirty`: the bits to look at first.
+template <bool PHASE>
+static void run_trial(const Frontier &F, const SchedLimits &lim, bool renames_only, uint64_t dirty, Trial &t,
+                      std::vector<int> *taken)
+{
+    while (dirty) {
+        const int q = __builtin_ctzll(dirty);
+        const int i = F.next(t.pos, q);
+        if (i < 0 || !can_run<PHASE>(F, lim, renames_only, t, i)) {
+            dirty &= dirty - 1;
+            continue;
+        }
+        const SchedOp &op = (*F.ops)[(size_t)i];
+        for (uint64_t m = op.bits; m; m &= m - 1)
+            t.pos[__builtin_ctzll(m)]++;
+        t.score += op.weight;
+        t.gen += op.kind == OP_GEN;
+        t.ip += op_is_ip(op.kind);
+        if (op_needs_register(op.kind))
+            t.targets |= uint64_t(1) << op.target;
+        if (taken)
+            taken->push_back(i);
+        dirty |= op.bits;
+    }
+}
+
+// Grows a trial by one bit at a time, each time by the bit that lets it run
+// the most; where none lets it run anything, by the bit whose next op is the
+// oldest.  `width`: how many bits it may have; `allowed`: which.
+template <bool PHASE>
+static void grow_trial(const Frontier &F, const SchedLimits &lim, bool renames_only, int n, uint64_t allowed, int width,
+                       Trial &t)
+{
+    run_trial<PHASE>(F, lim, renames_only, PHASE ? ((uint64_t(1) << n) - 1) : t.bits, t, nullptr);
+    Trial best, u;
+    while (popcount64(t.bits) < width) {
+        int best_gain = -1, best_old = 0;
+        uint64_t best_bit = 0;
+        for (uint64_t m = allowed & ~t.bits; m; m &= m - 1) {
+            const uint64_t bit = m & -m;
+            const int q = __builtin_ctzll(m);
+            const int first = F.next(t.pos, q);
+            if (first < 0)
+                continue;
+            // whatever the new bit lets run starts with its own next op
+            t.bits |= bit;
+            const bool runs = can_run<PHASE>(F, lim, renames_only, t, first);
+            int gain = 0;
+            if (runs) {
+                u = t;
+                run_trial<PHASE>(F, lim, renames_only, bit, u, nullptr);
+                gain = u.score - t.score;
+            }
+            t.bits &= ~bit;
+            if (gain > best_gain || (gain == best_gain && first < best_old)) {
+                if (runs)
+                    best = u;
+                best_gain = gain;
+                best_old = first;
+                best_bit = bit;
+            }
+        }
+        if (best_gain < 0 || (PHASE && best_gain == 0))
+            break;
+        if (best_gain > 0)
+            t = best;
+        else
+            t.bits |= best_bit;
+    }
+}
+
+// The bits of the next pass (PHASE = false) or phase: trials grown from
+// `start` alone and from the bits of the next few two-bit ops, the one that
+// gets furthest.
+template <bool PHASE>
+static Trial pick_bits(const Frontier &F, const SchedLimits &lim, bool renames_only, int n, uint64_t start,
+                       uint64_t allowed, int width)
+{
+    constexpr int kSeeds = PHASE ? 2 : 4;
+    uint64_t seeds[kSeeds + 1] = {0};
+    int n_seeds = 1;
+    const std::vector<SchedOp> &ops = *F.ops;
+    int cand[kMaxQubits], nc = 0;
+    for (int q = 0; q < n; q++)
+        for (int p = F.at[q]; p < F.end[q]; p++) {
+            const int i = F.list[(size_t)p];
+            if (ops[(size_t)i].ctrl) {
+                cand[nc++] = i;
+                break;
+            }
+        }
+    std::sort(cand, cand + nc);
+    for (int c = 0; c < nc && n_seeds <= kSeeds; c++) {
+        const uint64_t b = ops[(size_t)cand[c]].bits & allowed & ~start;
+        bool fresh = b != 0 && popcount64(start | b) <= width;
+        for (int j = 0; j < n_seeds && fresh; j++)
+            fresh = seeds[j] != b;
+        if (fresh)
+            seeds[n_seeds++] = b;
+    }
+    Trial best;
+    for (int j = 0; j < n_seeds; j++) {
+        Trial t;
+        t.bits = start | seeds[j];
+        std::memcpy(t.pos, F.at, sizeof(t.pos));
+        grow_trial<PHASE>(F, lim, renames_only, n, allowed, width, t);
+        if (j == 0 || t.score > best.score)
+            best = t;
+    }
+    return best;
+}
+
+static int op_weight(const HostOp &op) { return op.kind == OP_GEN ? 2 : 1; }
+
+// A register phase of a pass: its register bits and its ops in order.
+struct Ph {
+    uint32_t rs;
+    std::vector<int> ops;
+};
+
+// Cost of a pass's phases in hundredths of an HBM pass (see plan_cost): each
+// phase, a load or store transpose where the low qubits must leave the
+// registers, and an X or CNOT whose control is a thread bit (per-lane selects
+// of every register).
+static int phases_cost(const std::vector<Ph> &phs, const std::vector<HostOp> &loc, uint32_t lowmask)
+{
+    int c = 0;
+    for (const Ph &ph : phs) {
+        c += 13;
+        for (int i : ph.ops)
+            if (loc[(size_t)i].kind == OP_SWAP && (loc[(size_t)i].ctrl & ~(uint64_t)ph.rs))
+                c += 6;
+    }
+    if (phs.front().rs & lowmask)
+        c += 13;
+    if (phs.back().rs & lowmask)
+        c += 13;
+    return c;
+}
+
+// Phases in op order: registers go to the first targets that come along.
+static void first_fit_phases(const std::vector<HostOp> &loc, const PlanParams &pp, std::vector<Ph> *out)
+{
+    out->clear();
     std::vector<char> used(loc.size(), 0);
-    size_t left = loc.size();
+    size_t left = loc.size(), first = 0;
     while (left > 0) {
         Ph ph{0u, {}};
         uint64_t blocked = 0;
-        for (size_t i = 0; i < loc.size(); i++) {
+        for (size_t i = first; i < loc.size(); i++) {
             if (used[i])
                 continue;
-            const uint64_t qs = (uint64_t(1) << loc[i].target) | loc[i].ctrl;
-            if (qs & blocked) {
+            const uint64_t qs = op_qubits(loc[i]), tb = uint64_t(1) << loc[i].target;
+            const bool reg = op_needs_register(loc[i].kind);
+            if ((qs & blocked) || (reg && !(ph.rs & tb) && popcount64(ph.rs) >= pp.rlog)) {
                 blocked |= qs;
                 continue;
             }
-            if (op_needs_register(loc[i].kind)) {
-                const uint32_t tb = 1u << loc[i].target;
-                if (!(ph.rs & tb)) {
-                    if (popcount64(ph.rs) >= pp.rlog) {
-                        blocked |= qs;
-                        continue;
-                    }
-                    ph.rs |= tb;
-                }
-            }
+            if (reg)
+                ph.rs |= (uint32_t)tb;
             ph.ops.push_back((int)i);
             used[i] = 1;
             left--;
         }
-        if (ph.ops.empty()) {
-            set_error("internal: scheduler made no progress");
-            return DMV_ERR_STATE;
-        }
-        phs.push_back(std::move(ph));
+        while (first < loc.size() && used[first])
+            first++;
+        out->push_back(std::move(ph));
     }
+}
+
+static bool split_phases(const std::vector<HostOp> &loc, const PlanParams &pp, bool renames_only, bool high_first,
+                         std::vector<Ph> *out)
+{
+    std::vector<SchedOp> so(loc.size());
+    for (size_t i = 0; i < loc.size(); i++)
+        so[i] = SchedOp{op_qubits(loc[i]), loc[i].ctrl, loc[i].target, loc[i].kind, op_weight(loc[i]), 0};
+    Frontier F;
+    F.build(so, pp.k);
+    const SchedLimits none;
+    const uint64_t all = (uint64_t(1) << pp.k) - 1, low = (uint64_t(1) << pp.low_bits) - 1;
+    size_t left = loc.size();
+    out->clear();
+    while (left > 0) {
+        const uint64_t allowed = out->empty() && high_first ? all & ~low : all;
+        Trial t = pick_bits<true>(F, none, renames_only, pp.k, 0, allowed, pp.rlog);
+        bool only = renames_only;
+        if (t.score == 0 && only) {
+            only = false;  // only swaps with controls far away are left to run
+            t = pick_bits<true>(F, none, false, pp.k, 0, allowed, pp.rlog);
+        }
+        if (t.score == 0) {
+            if (high_first && out->empty())
+                return false;
+            set_error("internal: scheduler made no progress");
+            return false;
+        }
+        Ph ph{(uint32_t)t.bits, {}};
+        Trial done;
+        done.bits = t.bits;
+        std::memcpy(done.pos, F.at, sizeof(done.pos));
+        run_trial<true>(F, none, only, all, done, &ph.ops);
+        std::memcpy(F.at, done.pos, sizeof(F.at));
+        left -= ph.ops.size();
+        // register bits that no pair op of the phase needs are free again
+        uint32_t used = 0;
+        for (int i : ph.ops)
+            if (op_needs_register(loc[(size_t)i].kind))
+                used |= (uint32_t)(op_qubits(loc[(size_t)i]) & t.bits);
+        ph.rs = used;
+        out->push_back(std::move(ph));
+    }
+    return true;
+}
+
+// One HBM pass: its qubits, its ops on tile bits in order, and its phases.
+struct PassCut {
+    uint32_t qpos[16];
+    std::vector<HostOp> loc;
+    std::vector<int> src;  // which op of the circuit each is
+    std::vector<Ph> phs;
+    int cost = 0;  // of the phases
+};
+
+static int cut_pass(uint64_t Q, const std::vector<HostOp> &ops, const std::vector<int> &order, const PlanParams &pp,
+                    bool first_fit, std::vector<PassCut> *out)
+{
+    out->emplace_back();
+    PassCut &C = out->back();
+    int nq = 0, local[64];
+    for (int q = 0; q < pp.n; q++)
+        if ((Q >> q) & 1) {
+            if (nq < 16)
+                C.qpos[nq] = (uint32_t)q;
+            local[q] = nq++;
+        }
+    if (nq != pp.k) {
+        set_error("internal: pass has %d qubits, expected %d", nq, pp.k);
+        return DMV_ERR_STATE;
+    }
+    C.loc.reserve(order.size());
+    for (int i : order) {
+        HostOp op = ops[(size_t)i];
+        op.target = local[op.target];
+        uint64_t ctrl = 0;
+        for (uint64_t m = op.ctrl; m; m &= m - 1)
+            ctrl |= uint64_t(1) << local[__builtin_ctzll(m)];
+        op.ctrl = ctrl;
+        C.loc.push_back(op);
+    }
+    C.src = order;
+    // Register phases: the cheapest of the ways to cut the pass into them: in
+    // op order, or searched for (swaps with thread-bit controls kept until
+    // they only relabel, or done in place; the first phase's registers off the
+    // low bits, which saves the load's transpose, or anywhere).
+    const uint32_t lowmask = (1u << pp.low_bits) - 1;
+    first_fit_phases(C.loc, pp, &C.phs);
+    C.cost = phases_cost(C.phs, C.loc, lowmask);
+    std::vector<Ph> trial;
+    for (int way = 0; way < 4 && !first_fit; way++) {
+        if (!split_phases(C.loc, pp, (way & 1) == 0, (way & 2) != 0, &trial))
+            continue;
+        const int c = phases_cost(trial, C.loc, lowmask);
+        if (c < C.cost) {
+            C.cost = c;
+            C.phs.swap(trial);
+        }
+    }
+    return DMV_OK;
+}
+
+static void set_values(const HostOp &h, DevOp *op);
+
+static int make_pass(const PassCut &C, const PlanParams &pp, Plan *plan)
+{
+    DevPass P;
+    std::memset(&P, 0, sizeof(P));
+    P.k = (uint32_t)pp.k;
+    for (int j = 0; j < pp.k; j++)
+        P.qpos[j] = C.qpos[j];
+    const std::vector<HostOp> &loc = C.loc;
+    std::vector<Ph> phs = C.phs;
     const uint32_t lowmask = (1u << pp.low_bits) - 1;
     // Split transposes: the highest local bit above the lane-coalesced and
     // swizzle-group bits that no op of the pass needs in a register stays a
@@ -602,7 +973,7 @@ static int make_pass(uint64_t Q, const std::vector<HostOp> &taken, const PlanPar
             op.ctrl = h.ctrl;
             op.slot = h.slot;
             op.ctrl_thr = cthr;
-            std::memcpy(op.m, h.m, sizeof(op.m));
+            set_values(h, &op);
             op.tbit = J == kNoReg ? thread_bit(D.lay, pp, (uint32_t)h.target) : kNoReg;
             op.en = 0;
             for (int q = 0; q < NR; q++)
@@ -623,8 +994,6 @@ static int make_pass(uint64_t Q, const std::vector<HostOp> &taken, const PlanPar
             }
             if (h.kind == OP_GEN && J != kNoReg)
                 op.plain = (op.en == all_regs && (op.fl & first_members(op.rmask, NR)) == 0) ? 1u : 0u;
-            if (h.kind == OP_DIAG)
-                op.plain = diag_is_sign_flip(op.m) ? 1u : 0u;
             if (op_is_ip(h.kind) && h.slot + 1 > plan->n_slots)
                 plan->n_slots = h.slot + 1;
             if (op_is_ip(h.kind) && plan->ops.size() > D.op_begin) {
@@ -637,6 +1006,7 @@ static int make_pass(uint64_t Q, const std::vector<HostOp> &taken, const PlanPar
             }
             plan->ops.push_back(op);
             plan->op_pass.push_back(pass_index);
+            plan->op_src.push_back(C.src[(size_t)i]);
         }
         D.op_end = (uint32_t)plan->ops.size();
         plan->phases.push_back(D);
@@ -675,79 +1045,46 @@ static int make_pass(uint64_t Q, const std::vector<HostOp> &taken, const PlanPar
     return DMV_OK;
 }
 
-// Plan cost in units of a plain pass: every pass moves the state once, and
-// every phase beyond a pass's first adds compute between barriers (measured
-// on MI355X: the 30-qubit layered circuit at budget 12 adds one phase to
-// every pass for 1.29x the time; the 33-qubit random circuit saves 7 of 58
-// passes for 0.93x).
-static double plan_cost(const Plan &plan)
+// Cost of a plan in hundredths of an HBM pass.  Fitted to the 30-qubit layered
+// circuit in complex128 (745 gates, 6 to 19 passes, 35 to 48 phases): 2.6 ms a
+// pass plus 0.33 ms a phase on top of the ops' own time.
+static int plan_cost(const std::vector<PassCut> &cuts)
 {
-    return (double)plan.passes.size() + 0.6 * (double)(plan.phases.size() - plan.passes.size());
+    int c = 0;
+    for (const PassCut &C : cuts)
+        c += 100 + C.cost;
+    return c;
 }
 
-int build_plan(const std::vector<HostOp> &ops, const PlanParams &pp, Plan *out)
+// Passes in op order: a pass takes every op that still fits, and what it
+// cannot take blocks its qubits.
+static int first_fit_passes(const std::vector<HostOp> &ops, const std::vector<SchedOp> &so, const SchedLimits &lim,
+                            const PlanParams &pp, std::vector<PassCut> *out)
 {
-    if (pp.gen_auto) {
-        // the GEN budget per pass depends on the circuit: plan with 8 and 12
-        // and keep the cheaper plan (the smaller budget on a tie)
-        PlanParams a = pp, b = pp;
-        a.gen_auto = b.gen_auto = 0;
-        a.max_gen_per_pass = 8;
-        b.max_gen_per_pass = 12;
-        Plan pa, pb;
-        DMV_TRY(build_plan(ops, a, &pa));
-        DMV_TRY(build_plan(ops, b, &pb));
-        *out = plan_cost(pb) < plan_cost(pa) ? std::move(pb) : std::move(pa);
-        return DMV_OK;
-    }
-    DMV_CHECK_ARG(pp.k == pp.rlog + pp.tlog, "tile qubits %d != %d + %d", pp.k, pp.rlog, pp.tlog);
-    DMV_CHECK_ARG(pp.n >= pp.k && pp.k <= kMaxTileQubits && pp.rlog >= 1 &&
-                      (1 << pp.rlog) <= kMaxRegs && pp.tlog <= kMaxThreadBits &&
-                      pp.low_bits <= pp.tlog && pp.low_bits + pp.rlog <= pp.k,
-                  "invalid tile shape n=%d k=%d rlog=%d tlog=%d", pp.n, pp.k, pp.rlog, pp.tlog);
-    Plan plan;
-    const uint64_t all = (pp.n >= 64) ? ~uint64_t(0) : ((uint64_t(1) << pp.n) - 1);
-    const uint64_t lowmask = (uint64_t(1) << pp.low_bits) - 1;
-    for (const HostOp &op : ops) {
-        DMV_CHECK_ARG(op.target >= 0 && op.target < pp.n, "target %d out of range", op.target);
-        DMV_CHECK_ARG((op.ctrl & ~all) == 0 && !((op.ctrl >> op.target) & 1), "bad control mask");
-    }
-    // With split transposes, a pass keeps one of its qubits above the lane
-    // and swizzle-group bits free of register targets (the split bit): an op
-    // that would make every such qubit a register target waits for the next
-    // pass.  The lowest qubits are always in the tile, so those candidates
-    // are the tile's qubits outside the lowest max(low_bits, swz_bits).
-    const int split_keep = pp.half_lds && pp.tlog >= 7 ? pp.k - std::max(pp.low_bits, pp.swz_bits) - 1 : 64;
-    const uint64_t split_low = (uint64_t(1) << std::max(pp.low_bits, pp.swz_bits)) - 1;
+    const uint64_t all = (uint64_t(1) << pp.n) - 1, lowmask = (uint64_t(1) << pp.low_bits) - 1;
     std::vector<char> done(ops.size(), 0);
+    std::vector<int> order;
     size_t first = 0;
     while (first < ops.size()) {
         uint64_t Q = lowmask, blocked = 0, treg = 0;
-        int gen = 0;
-        std::vector<HostOp> taken;
+        int gen = 0, ip = 0;
+        order.clear();
         for (size_t i = first; i < ops.size(); i++) {
             if (done[i])
                 continue;
-            const uint64_t qs = op_qubits(ops[i]);
-            if (qs & blocked) {
-                blocked |= qs;
-                if ((blocked & all) == all)
-                    break;
-                continue;
-            }
-            const uint64_t nq = Q | qs;
-            const bool budget = ops[i].kind != OP_GEN || gen < pp.max_gen_per_pass;
-            const uint64_t nt = op_needs_register(ops[i].kind) ? (treg | (uint64_t(1) << ops[i].target)) : treg;
-            const bool split_ok = popcount64(nt & ~split_low) <= split_keep;
-            if (popcount64(nq) <= pp.k && budget && split_ok) {
-                Q = nq;
+            const SchedOp &op = so[i];
+            const uint64_t nt = op_needs_register(op.kind) ? treg | (uint64_t(1) << op.target) : treg;
+            if (!(op.bits & blocked) && popcount64(Q | op.bits) <= pp.k && (op.kind != OP_GEN || gen < lim.max_gen) &&
+                popcount64(nt & ~lim.low) <= lim.max_high_targets &&
+                !(op.group > 0 && ip > 0 && ip + op.group > lim.max_ip)) {
+                Q |= op.bits;
                 treg = nt;
-                taken.push_back(ops[i]);
+                order.push_back((int)i);
                 done[i] = 1;
-                if (ops[i].kind == OP_GEN)
-                    gen++;
+                gen += op.kind == OP_GEN;
+                ip += op_is_ip(op.kind);
             } else {
-                blocked |= qs;
+                blocked |= op.bits;
                 if ((blocked & all) == all)
                     break;
             }
@@ -757,8 +1094,159 @@ int build_plan(const std::vector<HostOp> &ops, const PlanParams &pp, Plan *out)
         // fill the tile up to k qubits with the lowest unused qubits
         for (int q = 0; q < pp.n && popcount64(Q) < pp.k; q++)
             Q |= uint64_t(1) << q;
-        DMV_TRY(make_pass(Q, taken, pp, &plan));
+        DMV_TRY(cut_pass(Q, ops, order, pp, true, out));
     }
+    return DMV_OK;
+}
+
+// Passes searched for: each takes the qubits that let it run the most ops
+// (pick_bits), whatever layer of the circuit they are in.
+static int searched_passes(const std::vector<HostOp> &ops, const std::vector<SchedOp> &so, const SchedLimits &lim,
+                           const PlanParams &pp, std::vector<PassCut> *out)
+{
+    const uint64_t all = (uint64_t(1) << pp.n) - 1, lowmask = (uint64_t(1) << pp.low_bits) - 1;
+    Frontier F;
+    F.build(so, pp.n);
+    size_t left = ops.size();
+    std::vector<int> order;
+    while (left > 0) {
+        uint64_t Q = pick_bits<false>(F, lim, false, pp.n, lowmask, all, pp.k).bits;
+        for (int q = 0; q < pp.n && popcount64(Q) < pp.k; q++)
+            Q |= uint64_t(1) << q;
+        Trial done;
+        done.bits = Q;
+        std::memcpy(done.pos, F.at, sizeof(done.pos));
+        order.clear();
+        run_trial<false>(F, lim, false, Q, done, &order);
+        if (order.empty()) {
+            set_error("internal: scheduler made no progress");
+            return DMV_ERR_STATE;
+        }
+        std::memcpy(F.at, done.pos, sizeof(F.at));
+        left -= order.size();
+        DMV_TRY(cut_pass(Q, ops, order, pp, false, out));
+    }
+    return DMV_OK;
+}
+
+// The scheduler's view of the ops and what a pass may hold.
+static std::vector<SchedOp> sched_ops(const std::vector<HostOp> &ops, const PlanParams &pp, SchedLimits *lim)
+{
+    std::vector<SchedOp> so(ops.size());
+    int run[64] = {}, head[64] = {};  // each qubit's open run of IP ops, counted at its first op
+    for (size_t i = ops.size(); i-- > 0;) {
+        so[i] = SchedOp{op_qubits(ops[i]), ops[i].ctrl, ops[i].target, ops[i].kind, op_weight(ops[i]), 0};
+        if (op_is_ip(ops[i].kind)) {
+            const int q = ops[i].target;
+            if (run[q] > 0)
+                so[(size_t)head[q]].group = 0;
+            head[q] = (int)i;
+            so[i].group = ++run[q];
+        } else {
+            for (uint64_t m = so[i].bits; m; m &= m - 1)
+                run[__builtin_ctzll(m)] = 0;
+        }
+    }
+    // With split transposes, a pass keeps one of its qubits above the lane
+    // and swizzle-group bits free of register targets (the split bit): an op
+    // that would make every such qubit a register target waits for the next
+    // pass.  The lowest qubits are always in the tile, so those candidates
+    // are the tile's qubits outside the lowest max(low_bits, swz_bits).
+    const int kept = std::max(pp.low_bits, pp.swz_bits);
+    lim->max_gen = pp.max_gen_per_pass;
+    lim->max_ip = pp.max_ip_per_pass;
+    lim->max_high_targets = pp.half_lds && pp.tlog >= 7 ? pp.k - kept - 1 : 64;
+    lim->low = (uint64_t(1) << kept) - 1;
+    return so;
+}
+
+bool same_structure(const std::vector<HostOp> &a, const std::vector<HostOp> &b)
+{
+    if (a.size() != b.size())
+        return false;
+    for (size_t i = 0; i < a.size(); i++)
+        if (a[i].kind != b[i].kind || a[i].target != b[i].target || a[i].ctrl != b[i].ctrl || a[i].slot != b[i].slot)
+            return false;
+    return true;
+}
+
+// What a device op takes from its op's values.
+static void set_values(const HostOp &h, DevOp *op)
+{
+    std::memcpy(op->m, h.m, sizeof(op->m));
+    if (h.kind == OP_GEN)
+        op->aux = h.su2 ? 1u : 0u;
+    if (h.kind == OP_DIAG)
+        op->plain = diag_is_sign_flip(op->m) ? 1u : 0u;
+}
+
+void refresh_ops(const std::vector<HostOp> &given, const std::vector<int> &op_src, std::vector<DevOp> *dev)
+{
+    std::vector<HostOp> ops = given;
+    special_unitary(&ops);
+    for (size_t i = 0; i < dev->size(); i++)
+        set_values(ops[(size_t)op_src[i]], &(*dev)[i]);
+}
+
+int in_order_budget(const std::vector<HostOp> &ops, const PlanParams &pp, int *budget)
+{
+    SchedLimits lim;
+    const std::vector<SchedOp> so = sched_ops(ops, pp, &lim);
+    size_t cost[2];
+    const int budgets[2] = {8, 12};
+    for (int i = 0; i < 2; i++) {
+        lim.max_gen = budgets[i];
+        std::vector<PassCut> cuts;
+        DMV_TRY(first_fit_passes(ops, so, lim, pp, &cuts));
+        cost[i] = 4 * cuts.size();
+        for (const PassCut &C : cuts)
+            cost[i] += 6 * C.phs.size();
+    }
+    *budget = budgets[cost[1] < cost[0]];
+    return DMV_OK;
+}
+
+int build_plan(const std::vector<HostOp> &given, const PlanParams &pp, Plan *out)
+{
+    std::vector<HostOp> ops = given;
+    special_unitary(&ops);
+    DMV_CHECK_ARG(pp.k == pp.rlog + pp.tlog, "tile qubits %d != %d + %d", pp.k, pp.rlog, pp.tlog);
+    DMV_CHECK_ARG(pp.n >= pp.k && pp.k <= kMaxTileQubits && pp.rlog >= 1 &&
+                      (1 << pp.rlog) <= kMaxRegs && pp.tlog <= kMaxThreadBits &&
+                      pp.low_bits <= pp.tlog && pp.low_bits + pp.rlog <= pp.k,
+                  "invalid tile shape n=%d k=%d rlog=%d tlog=%d", pp.n, pp.k, pp.rlog, pp.tlog);
+    Plan plan;
+    const uint64_t all = (pp.n >= 64) ? ~uint64_t(0) : ((uint64_t(1) << pp.n) - 1);
+    for (const HostOp &op : ops) {
+        DMV_CHECK_ARG(op.target >= 0 && op.target < pp.n, "target %d out of range", op.target);
+        DMV_CHECK_ARG((op.ctrl & ~all) == 0 && !((op.ctrl >> op.target) & 1), "bad control mask");
+    }
+    SchedLimits lim;
+    const std::vector<SchedOp> so = sched_ops(ops, pp, &lim);
+    // A budget of eight GENs a pass (the caller's, or tried here) is filled in
+    // op order: measured on the 30-qubit layered circuit, both ways take 19
+    // passes, but searched ones 48 phases for 38 (114 against 109 ms).
+    // Without a budget the search is tried too and the cheaper plan kept: 6
+    // passes of that circuit (77 ms), 9 for 25 at 20 qubits and 10 layers (328
+    // against 532 us).  A CNOT ring, whose next layer waits for the whole ring,
+    // takes as many passes either way.
+    constexpr int kInOrder = 8;
+    std::vector<PassCut> cuts;
+    if (pp.gen_auto || pp.max_gen_per_pass <= kInOrder) {
+        if (pp.gen_auto)
+            lim.max_gen = kInOrder;
+        DMV_TRY(first_fit_passes(ops, so, lim, pp, &cuts));
+    }
+    if (pp.gen_auto || pp.max_gen_per_pass > kInOrder) {
+        if (pp.gen_auto)
+            lim.max_gen = 1 << 30;
+        std::vector<PassCut> more;
+        DMV_TRY(searched_passes(ops, so, lim, pp, &more));
+        if (cuts.empty() || plan_cost(more) < plan_cost(cuts))
+            cuts.swap(more);
+    }
+    for (const PassCut &C : cuts)
+        DMV_TRY(make_pass(C, pp, &plan));
     // number the IP ops of every pass: pass p's gradient partials are rows
     // ip_begin[p] .. ip_begin[p+1] of the per-pass partial buffer
     plan.ip_begin.assign(plan.passes.size() + 1, 0);
@@ -768,13 +1256,12 @@ int build_plan(const std::vector<HostOp> &ops, const PlanParams &pp, Plan *out)
         for (uint32_t ph = plan.passes[p].phase_begin; ph < plan.passes[p].phase_end; ph++)
             for (uint32_t o = plan.phases[ph].op_begin; o < plan.phases[ph].op_end; o++)
                 if (op_is_ip(plan.ops[o].kind)) {
-                    plan.ops[o].ip_pos = (uint32_t)plan.ip_slots.size() - plan.ip_begin[p];
+                    plan.ops[o].aux = (uint32_t)plan.ip_slots.size() - plan.ip_begin[p];
                     plan.ip_slots.push_back(plan.ops[o].slot);
                 }
     }
     plan.ip_begin[plan.passes.size()] = (uint32_t)plan.ip_slots.size();
     DMV_TRY(validate_plan(plan, pp));
-    plan.max_gen = pp.max_gen_per_pass;
     *out = std::move(plan);
     return DMV_OK;
 }
@@ -912,6 +1399,11 @@ int validate_plan(const Plan &plan, const PlanParams &pp)
                 // kernels apply them to every pair of every lane
                 if (op.kind == OP_GEN && (op.ctrl != 0 || op.ctrl_thr != 0 || op.en != regs)) {
                     set_error("internal: controlled GEN op");
+                    return DMV_ERR_STATE;
+                }
+                if (op.kind == OP_GEN && op.aux &&
+                    (op.m[6] != op.m[0] || op.m[7] != -op.m[1] || op.m[2] != -op.m[4] || op.m[3] != op.m[5])) {
+                    set_error("internal: special-unitary flag on a general matrix");
                     return DMV_ERR_STATE;
                 }
                 if (op_is_ip(op.kind)) {

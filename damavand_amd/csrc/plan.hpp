@@ -24,6 +24,7 @@ struct HostOp {
     uint64_t ctrl;
     double m[8];
     int slot;  // parameter index of an IP op, else -1
+    bool su2 = false;  // a GEN whose matrix is special unitary to the last bit (special_unitary)
 };
 
 // Process-wide tunables (defined by the runtime; environment DMV_<NAME> or dmv_tune_set).
@@ -46,6 +47,11 @@ std::vector<HostOp> adjoint_ops(const std::vector<Gate> &gates);
 // qubits; IP ops and controlled ops end a run.
 std::vector<HostOp> merge_ops(const std::vector<HostOp> &ops);
 
+// Writes every GEN's matrix as (special unitary) x (phase) and moves the phases
+// into one GEN, which stays general (their product acts on the whole state, so
+// any place in the order will do).
+void special_unitary(std::vector<HostOp> *ops);
+
 struct PlanParams {
     int n;          // qubits of the state
     int k;          // tile qubits (= rlog + tlog)
@@ -56,16 +62,17 @@ struct PlanParams {
     int max_gen_per_pass;  // compute budget of a pass, in general 2x2 ops
     int nontemporal = 0;   // forward passes: streaming (nontemporal) loads and stores
     int half_lds = 0;      // forward passes: split transposes where a pass allows (half-LDS kernels exist)
-    int gen_auto = 0;      // forward plans: build_plan picks max_gen_per_pass (8 or 12) by plan cost
+    int max_ip_per_pass = 1 << 30;  // IP ops of a pass (a run of IP ops on one qubit stays together)
+    int gen_auto = 0;      // build_plan chooses the passes by cost instead (max_gen_per_pass is not used)
     StateLayout layout = kPlainLayout;  // element map of the states the plan runs on
 };
 
 struct Plan {
-    int max_gen = 0;             // the GEN budget per pass the plan was built with
     std::vector<DevPass> passes;
     std::vector<DevPhase> phases;
     std::vector<DevOp> ops;      // tile-local ops, grouped by phase
     std::vector<int> op_pass;    // pass of each op
+    std::vector<int> op_src;     // which of build_plan's ops each op is
     int n_slots = 0;             // 1 + largest IP slot
     // IP ops per pass: pass p holds ip_begin[p+1] - ip_begin[p] of them, whose
     // slots (parameter indices) are ip_slots[ip_begin[p] ..] in ip_pos order
@@ -77,10 +84,18 @@ struct Plan {
     std::vector<int> logical_pass;
 };
 
-// Greedy scheduler: packs ops into passes of <= k qubits (always including the
-// `low_bits` lowest qubits) so that every op commutes past the ops it skips,
-// then splits each pass into register phases.
+// The scheduler: cuts the ops into passes of <= k qubits (always including the
+// `low_bits` lowest qubits), every op moved past others on disjoint qubits
+// only, then each pass into register phases.
 int build_plan(const std::vector<HostOp> &ops, const PlanParams &pp, Plan *out);
+// The budget of GENs a pass (8 or 12) that suits the ops best when passes are
+// filled in op order.
+int in_order_budget(const std::vector<HostOp> &ops, const PlanParams &pp, int *budget);
+// Whether plans of the two op lists differ in matrices only.
+bool same_structure(const std::vector<HostOp> &a, const std::vector<HostOp> &b);
+// The device ops `dev` of a plan built from ops of the same structure, with
+// the matrices of `ops`.
+void refresh_ops(const std::vector<HostOp> &ops, const std::vector<int> &op_src, std::vector<DevOp> *dev);
 // Checks every invariant the tile kernels rely on (index ranges, layouts,
 // register bits).  Called before a plan is uploaded.
 int validate_plan(const Plan &plan, const PlanParams &pp);

@@ -365,8 +365,8 @@ PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const
     pp.tlog = tlog;
     pp.rlog = k - tlog;
     pp.max_gen_per_pass = gen;
-    // forward plans choose 8 or 12 per circuit unless a budget was given
-    pp.gen_auto = !adjoint && !gen_set ? 1 : 0;
+    // plans choose their passes by cost unless a budget was given
+    pp.gen_auto = gen_set ? 0 : 1;
     pp.nontemporal = nt != 0 ? 1 : 0;
     // forward passes split their transposes where the shape has half-LDS kernels
     pp.half_lds = !adjoint && tune_value("half_lds", 1) != 0 && tile_half_exists(dtype, pp.rlog, pp.tlog) ? 1 : 0;
@@ -417,6 +417,13 @@ int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoin
     if (same_shape && dp.version == version && dp.epoch == tune_epoch())
         return DMV_OK;
     std::vector<HostOp> merged = merge_ops(ops);
+    if (!small && same_shape && dp.epoch == tune_epoch() && same_structure(dp.source, merged)) {
+        // the same gates at other angles: passes and phases stay, the ops get new matrices
+        refresh_ops(merged, dp.plan.op_src, &dp.plan.ops);
+        DMV_TRY(upload(dp.d_ops, dp.cap_ops, dp.plan.ops));
+        dp.version = version;
+        return DMV_OK;
+    }
     dp.small = small;
     dp.dtype = dtype;
     dp.pp = pp;
@@ -431,6 +438,7 @@ int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoin
         Plan plan;
         DMV_TRY(build_plan(merged, pp, &plan));
         dp.plan = std::move(plan);
+        dp.source = std::move(merged);
         DMV_TRY(upload(dp.d_passes, dp.cap_passes, dp.plan.passes));
         DMV_TRY(upload(dp.d_phases, dp.cap_phases, dp.plan.phases));
         DMV_TRY(upload(dp.d_ops, dp.cap_ops, dp.plan.ops));

@@ -68,6 +68,7 @@ struct DevicePlan {
     bool small = false;           // whole-state kernel instead of tile passes
     PlanParams pp{};
     Plan plan;
+    std::vector<HostOp> source;   // the ops that the plan was built from
     std::vector<DevOp> small_ops;
     DevPass *d_passes = nullptr;
     DevPhase *d_phases = nullptr;

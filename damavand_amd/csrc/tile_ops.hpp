@@ -298,15 +298,41 @@ template <class V, int NR> __device__ __forceinline__ void copy_regs(V (&out)[NR
         out[r] = in[r];
 }
 
+// A special-unitary GEN, m = [[al, -be*], [be, al*]].  f: the first member holds
+// target bit 1, so rows and columns change places, which for such a matrix
+// only flips the signs of Im(al) and Re(be).
+template <class R> struct Su2 {
+    R ar, ai, br, bi;
+};
+
+template <class R> __device__ __forceinline__ Su2<R> load_su2(const double *m)
+{
+    return Su2<R>{(R)m[0], (R)m[1], (R)m[4], (R)m[5]};
+}
+
+template <class R> __device__ __forceinline__ Su2<R> flip_su2(const Su2<R> &A, bool f)
+{
+    return Su2<R>{A.ar, f ? -A.ai : A.ai, f ? -A.br : A.br, A.bi};
+}
+
+template <class V, class R>
+__device__ __forceinline__ void apply_su2_to(V &oa, V &ob, const V &a, const V &b, const Su2<R> &M)
+{
+    oa.x = M.ar * a.x - M.ai * a.y - M.br * b.x - M.bi * b.y;
+    oa.y = M.ar * a.y + M.ai * a.x - M.br * b.y + M.bi * b.x;
+    ob.x = M.br * a.x - M.bi * a.y + M.ar * b.x + M.ai * b.y;
+    ob.y = M.br * a.y + M.bi * a.x + M.ar * b.y - M.ai * b.x;
+}
+
 template <int M, class V, class R, int NR>
-__device__ __forceinline__ void oop_gen_plain_m(V (&out)[NR], const V (&in)[NR], const Mat<R> &A)
+__device__ __forceinline__ void oop_su2_m(V (&out)[NR], const V (&in)[NR], const Su2<R> &A, uint32_t fl)
 {
     constexpr int HB = highest_bit(M);
 #pragma unroll
     for (int p = 0; p < NR; p++) {
         if (p & HB)
             continue;
-        apply2_to(out[p], out[p ^ M], in[p], in[p ^ M], A);
+        apply_su2_to(out[p], out[p ^ M], in[p], in[p ^ M], flip_su2(A, (fl >> p) & 1u));
     }
 }
 
@@ -384,23 +410,24 @@ __device__ __forceinline__ void oop_op(V (&out)[NR], const V (&in)[NR], const De
 {
     const uint32_t en = op->en, fl = op->fl;
     const bool hold = thread_controls_hold(op, tid);
-    const Mat<R> A = load_mat<R>(op->m);
     // masks at or above NR have empty cases; the clamp lets the compiler drop them
     const uint32_t m = op->rmask < (uint32_t)NR ? op->rmask : 1u;
     if (op->kind == OP_DIAG) {
         oop_diag<V, R>(out, in, op, tid, hold);
-    } else if (op->plain) {
+    } else if (op->kind == OP_GEN && op->aux) {
+        const Su2<R> S = load_su2<R>(op->m);
         switch (m) {
-#define DMV_OOP_PLAIN_CASE(M)                                                                      \
+#define DMV_OOP_SU2_CASE(M)                                                                        \
     case M:                                                                                        \
         if constexpr (M < NR)                                                                      \
-            oop_gen_plain_m<M>(out, in, A);                                                        \
+            oop_su2_m<M>(out, in, S, fl);                                                          \
         break;
-            DMV_MASK_CASES_FROM2(DMV_OOP_PLAIN_CASE)
-#undef DMV_OOP_PLAIN_CASE
-        default: oop_gen_plain_m<1>(out, in, A); break;
+            DMV_MASK_CASES_FROM2(DMV_OOP_SU2_CASE)
+#undef DMV_OOP_SU2_CASE
+        default: oop_su2_m<1>(out, in, S, fl); break;
         }
     } else if (op->kind == OP_GEN) {
+        const Mat<R> A = load_mat<R>(op->m);
         switch (m) {
 #define DMV_OOP_GEN_CASE(M)                                                                        \
     case M:                                                                                        \
