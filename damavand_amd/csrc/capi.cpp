@@ -709,10 +709,9 @@ int dmv_circuit_adjoint_diag(dmv_circuit *c, dmv_state *psi, dmv_state *lam, int
 int dmv_circuit_plan_stats(dmv_circuit *c, int dtype, int *passes, int *phases, int *ops, double *hbm_bytes)
 {
     CHECK_CIRCUIT(c);
-    const int small_cap = dtype == DMV_C64 ? kSmallMaxQubitsC64 : kSmallMaxQubitsC128;
     const double state_bytes = (double)(uint64_t(1) << c->n) * amp_bytes(dtype);
     std::vector<HostOp> merged = merge_ops(forward_ops(c->gates));
-    if (c->n <= small_cap) {
+    if (c->n <= kSmallMaxQubits) {
         if (passes) *passes = 1;
         if (phases) *phases = 1;
         if (ops) *ops = (int)merged.size();

@@ -13,7 +13,7 @@ __global__ void __launch_bounds__(kSmallThreads)
 k_small(typename Cplx<R>::T *__restrict__ state, uint32_t n, const DevOp *__restrict__ ops, uint32_t n_ops)
 {
     using V = typename Cplx<R>::T;
-    constexpr int CAP = 65536 / sizeof(V);
+    constexpr int CAP = 1 << kSmallMaxQubits;
     __shared__ V s[CAP];
     const uint32_t n_amp = 1u << n;
     for (uint32_t i = threadIdx.x; i < n_amp; i += blockDim.x)
@@ -34,7 +34,7 @@ k_small_adjoint(typename Cplx<R>::T *__restrict__ psi, typename Cplx<R>::T *__re
                 const DevOp *__restrict__ ops, uint32_t n_ops, double *__restrict__ partials)
 {
     using V = typename Cplx<R>::T;
-    constexpr int CAP = 32768 / sizeof(V);
+    constexpr int CAP = 1 << kSmallMaxQubits;
     __shared__ V sp[CAP];
     __shared__ V sl[CAP];
     __shared__ double red[kSmallThreads / 64];
@@ -64,7 +64,7 @@ k_small_adjoint(typename Cplx<R>::T *__restrict__ psi, typename Cplx<R>::T *__re
 
 int launch_small(int dtype, void *state, int n, const DevOp *ops, uint32_t n_ops)
 {
-    const int cap = dtype == DMV_C64 ? kSmallMaxQubitsC64 : kSmallMaxQubitsC128;
+    const int cap = kSmallMaxQubits;
     DMV_CHECK_ARG(n >= 1 && n <= cap, "whole-state kernel holds at most %d qubits", cap);
     if (dtype == DMV_C64)
         hipLaunchKernelGGL(k_small<float>, dim3(1), dim3(kSmallThreads), 0, stream(), (c64 *)state, (uint32_t)n, ops,
@@ -77,7 +77,7 @@ int launch_small(int dtype, void *state, int n, const DevOp *ops, uint32_t n_ops
 
 int launch_small_adjoint(int dtype, void *psi, void *lam, int n, const DevOp *ops, uint32_t n_ops, double *partials)
 {
-    const int cap = (dtype == DMV_C64 ? kSmallMaxQubitsC64 : kSmallMaxQubitsC128) - 1;
+    const int cap = kSmallMaxQubits;
     DMV_CHECK_ARG(n >= 1 && n <= cap, "whole-state adjoint kernel holds at most %d qubits", cap);
     if (dtype == DMV_C64)
         hipLaunchKernelGGL(k_small_adjoint<float>, dim3(1), dim3(kSmallThreads), 0, stream(), (c64 *)psi, (c64 *)lam,

@@ -67,6 +67,7 @@ int launch_tile_adjoint(int dtype, int rlog, int tlog, bool nt, void *psi, void 
         if (tlog == 8 && rlog == 3)
             return nt ? run_tile_adj<float, 3, 8, true>(psi, lam, n, L, passes, phases, ops, pass_idx, partials)
                       : run_tile_adj<float, 3, 8>(psi, lam, n, L, passes, phases, ops, pass_idx, partials);
+        if (tlog == 8 && rlog == 2) return run_tile_adj<float, 2, 8>(psi, lam, n, L, passes, phases, ops, pass_idx, partials);
         if (tlog == 6 && rlog == 3) return run_tile_adj<float, 3, 6>(psi, lam, n, L, passes, phases, ops, pass_idx, partials);
         if (tlog == 6 && rlog == 4) return run_tile_adj<float, 4, 6>(psi, lam, n, L, passes, phases, ops, pass_idx, partials);
     }

@@ -14,6 +14,8 @@ int launch_tile_c64(int rlog, int tlog, bool nt, bool half, void *state, int n, 
     }
     if (tlog == 8 && rlog == 4) return run_tile<float, double, 4, 8, false>(nt, state, n, L, passes, phases, ops, pass_idx);
     if (tlog == 8 && rlog == 3) return run_tile<float, double, 3, 8, false>(nt, state, n, L, passes, phases, ops, pass_idx);
+    if (tlog == 9 && rlog == 3) return run_tile<float, double, 3, 9, false>(nt, state, n, L, passes, phases, ops, pass_idx);
+    if (tlog == 8 && rlog == 2) return run_tile<float, double, 2, 8, false>(nt, state, n, L, passes, phases, ops, pass_idx);
     if (tlog == 6 && rlog == 4) return run_tile<float, double, 4, 6, false>(nt, state, n, L, passes, phases, ops, pass_idx);
     if (tlog == 6 && rlog == 3) return run_tile<float, double, 3, 6, false>(nt, state, n, L, passes, phases, ops, pass_idx);
     return kNotHandled;

@@ -325,6 +325,7 @@ PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const
     int nt = adjoint ? (2 * state_bytes >= (uint64_t(512) << 20) ? 1 : 0) : (state_bytes >= (uint64_t(2) << 30) ? 1 : 0);
     bool chosen = false;  // the shape was measured for this size (table or circuit)
     bool gen_set = false;  // the GEN budget was given (table, tunable, circuit)
+    bool given = false;    // the shape was given by a tunable
     TuneChoice t;
     if (tune_lookup(tune_key(n, dtype, adjoint ? "adjoint" : "forward"), &t) && t.set()) {
         k = t.k;
@@ -340,6 +341,7 @@ PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const
         k = k_set > 0 ? (int)k_set : k;
         tlog = t_set > 0 ? (int)t_set : 8;
         chosen = false;
+        given = true;
     }
     if (tune_value("max_gen_per_pass", -1) > 0) {
         gen = (int)tune_value("max_gen_per_pass", gen);
@@ -354,10 +356,18 @@ PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const
         nt = pin->nt >= 0 ? pin->nt : nt;
         chosen = true;
     }
-    // small states: fewer threads and smaller tiles keep more workgroups busy
-    if (!chosen && n < k + 6) {
-        tlog = 6;
-        k = adjoint ? 9 : (dtype == DMV_C64 ? 10 : 9);
+    // Small states run 8 amplitudes per thread on every thread that their tiles
+    // have: with one tile a CU or fewer a pass is a chain of latencies, which
+    // more waves overlap, and the 16-amplitude kernels' code (140 KiB) does not
+    // stay in the instruction cache.  16 qubits, 8 layers: 160 us on 11-qubit
+    // tiles against 204 on 12-qubit ones and 209 on one-wave 9-qubit ones; 20
+    // qubits: 377 us on 512 threads against 414 (11-qubit tiles) and 474 (12, 16
+    // amplitudes per thread), which win from 23 qubits on (27: 21.6 ms against
+    // 22.4).  Up to 12 qubits (reverse sweeps 11) the whole state is one tile, so
+    // a plan is one pass (12 qubits: 96 us against 104 in passes of 11).
+    if (!chosen && (!given || n < k + 6) && n <= (adjoint ? 24 : 20)) {
+        k = adjoint || (n > 12 && n < 20) ? std::min(n, 11) : std::min(n, 12);
+        tlog = k <= 9 ? 6 : (k == 12 ? 9 : 8);
     }
     if (k > n)
         k = n;
@@ -406,8 +416,7 @@ template <class T> static int upload(T *&dptr, size_t &cap, const std::vector<T>
 int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoint, const std::vector<HostOp> &ops,
                  StateLayout layout, const TuneChoice *pin)
 {
-    const int small_cap = (dtype == DMV_C64 ? kSmallMaxQubitsC64 : kSmallMaxQubitsC128) - (adjoint ? 1 : 0);
-    const bool small = n <= small_cap;
+    const bool small = n <= kSmallMaxQubits;
     PlanParams pp = small ? PlanParams{} : tile_params(n, dtype, adjoint, layout, pin);
     const bool same_shape = dp.valid && dp.dtype == dtype && dp.small == small &&
                             (small || (dp.pp.k == pp.k && dp.pp.tlog == pp.tlog && dp.pp.max_gen_per_pass == pp.max_gen_per_pass &&

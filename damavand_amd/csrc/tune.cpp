@@ -236,8 +236,7 @@ int autotune_forward(dmv_circuit *c, dmv_state *s, int *chosen)
 {
     DMV_CHECK_ARG(c->n == s->n, "circuit has %d qubits but the state has %d", c->n, s->n);
     DMV_TRY(ensure_device());
-    const int small_cap = s->dtype == DMV_C64 ? kSmallMaxQubitsC64 : kSmallMaxQubitsC128;
-    if (s->n <= small_cap) {  // one whole-state launch: nothing to choose
+    if (s->n <= kSmallMaxQubits) {  // one whole-state launch: nothing to choose
         if (chosen)
             *chosen = s->n;
         return DMV_OK;
@@ -297,8 +296,7 @@ int autotune_adjoint(dmv_circuit *c, int dtype, int *chosen)
 {
     DMV_CHECK_ARG(dtype == DMV_C128 || dtype == DMV_C64, "dtype must be DMV_C128 or DMV_C64");
     DMV_TRY(ensure_device());
-    const int small_cap = (dtype == DMV_C64 ? kSmallMaxQubitsC64 : kSmallMaxQubitsC128) - 1;
-    if (c->n <= small_cap) {
+    if (c->n <= kSmallMaxQubits) {
         if (chosen)
             *chosen = c->n;
         return DMV_OK;
