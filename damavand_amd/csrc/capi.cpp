@@ -55,7 +55,7 @@ using namespace dmv;
 
 // Uploads a Z/ZZ observable into a device buffer laid out as
 // a[n] (double) | b[n_pairs] (double) | pi[n_pairs] (int) | pj[n_pairs] (int).
-static int upload_terms(double **buf, uint64_t *cap, int n, const double *a, int n_pairs, const int *pi,
+static int upload_terms(Pinned &pin, double **buf, uint64_t *cap, int n, const double *a, int n_pairs, const int *pi,
                         const int *pj, const double *b, const double **da, const double **db, const int **dpi,
                         const int **dpj)
 {
@@ -80,7 +80,7 @@ static int upload_terms(double **buf, uint64_t *cap, int n, const double *a, int
         ip[t] = pi[t];
         ip[n_pairs + t] = pj[t];
     }
-    DMV_TRY(copy_h2d(*buf, host.data(), need * sizeof(double)));
+    DMV_TRY(pinned_h2d(pin, *buf, host.data(), need * sizeof(double)));
     *da = *buf;
     *db = *buf + n;
     *dpi = reinterpret_cast<const int *>(*buf + n + n_pairs);
@@ -90,7 +90,7 @@ static int upload_terms(double **buf, uint64_t *cap, int n, const double *a, int
 
 // Uploads the table of a diagonal observable (2^n_wires doubles) and checks
 // its wires: distinct, in [0, n).
-static int upload_table(double **buf, uint64_t *cap, int n, int n_wires, const int *wires, const double *table,
+static int upload_table(Pinned &pin, double **buf, uint64_t *cap, int n, int n_wires, const int *wires, const double *table,
                         TableWires *W)
 {
     DMV_CHECK_ARG(n_wires >= 0 && n_wires <= kMaxTableWires, "a table observable has 0 to %d wires", kMaxTableWires);
@@ -113,7 +113,7 @@ static int upload_table(double **buf, uint64_t *cap, int n, int n_wires, const i
         DMV_TRY(alloc((void **)buf, need * sizeof(double)));
         *cap = need;
     }
-    return copy_h2d(*buf, table, need * sizeof(double));
+    return pinned_h2d(pin, *buf, table, need * sizeof(double));
 }
 
 int dmv::circuit_adjoint(dmv_circuit *c, dmv_state *psi, dmv_state *lam, const Observable &obs, double *energy,
@@ -131,22 +131,30 @@ int dmv::circuit_adjoint(dmv_circuit *c, dmv_state *psi, dmv_state *lam, const O
     // psi = U|0>
     DMV_TRY(state_reset(psi, 0, false));
     DMV_TRY(circuit_forward(c, psi, DMV_FORWARD_FUSED));
+    if ((uint64_t)np + 1 > c->cap_grad) {
+        release(c->d_grad);
+        c->d_grad = nullptr;
+        c->cap_grad = 0;
+        DMV_TRY(alloc((void **)&c->d_grad, ((uint64_t)np + 1) * sizeof(double)));
+        c->cap_grad = (uint64_t)np + 1;
+    }
+    double *d_energy = c->d_grad + np;
     // lambda = H psi, E = <psi|H|psi>
     if (obs.table) {
         TableWires W;
-        DMV_TRY(upload_table(&c->d_terms, &c->cap_terms, c->n, obs.n_wires, obs.wires, obs.table, &W));
+        DMV_TRY(upload_table(c->pin_terms, &c->d_terms, &c->cap_terms, c->n, obs.n_wires, obs.wires, obs.table, &W));
         prof_begin(DMV_KC_REDUCE);
         DMV_TRY(launch_obs_table(psi->dtype, psi->amp, lam->amp, c->n, psi->layout, c->d_terms, W, psi->ws,
-                                 psi->scalars));
+                                 d_energy));
         prof_end(DMV_KC_REDUCE, 3.0 * (double)psi->bytes);
     } else {
         const double *da, *db;
         const int *dpi, *dpj;
-        DMV_TRY(upload_terms(&c->d_terms, &c->cap_terms, c->n, obs.a, obs.n_pairs, obs.pi, obs.pj, obs.b, &da, &db,
+        DMV_TRY(upload_terms(c->pin_terms, &c->d_terms, &c->cap_terms, c->n, obs.a, obs.n_pairs, obs.pi, obs.pj, obs.b, &da, &db,
                              &dpi, &dpj));
         prof_begin(DMV_KC_REDUCE);
         DMV_TRY(launch_apply_obs(psi->dtype, psi->amp, lam->amp, c->n, psi->layout, da, obs.n_pairs, dpi, dpj, db,
-                                 psi->ws, psi->scalars));
+                                 psi->ws, d_energy));
         prof_end(DMV_KC_REDUCE, 3.0 * (double)psi->bytes);
     }
     // reverse sweep
@@ -176,12 +184,6 @@ int dmv::circuit_adjoint(dmv_circuit *c, dmv_state *psi, dmv_state *lam, const O
         DMV_TRY(alloc((void **)&c->d_partials, rows * per_ip * sizeof(double)));
         c->cap_partials = rows * per_ip;
     }
-    if ((uint64_t)np + 1 > c->cap_grad) {
-        release(c->d_grad);
-        c->d_grad = nullptr;
-        DMV_TRY(alloc((void **)&c->d_grad, ((uint64_t)np + 1) * sizeof(double)));
-        c->cap_grad = (uint64_t)np + 1;
-    }
     if (dp.small) {
         prof_begin(DMV_KC_ADJOINT);
         DMV_TRY(launch_small_adjoint(psi->dtype, psi->amp, lam->amp, c->n, dp.d_ops, (uint32_t)dp.small_ops.size(),
@@ -205,10 +207,12 @@ int dmv::circuit_adjoint(dmv_circuit *c, dmv_state *psi, dmv_state *lam, const O
             }
         }
     }
+    std::vector<double> out((size_t)np + 1);
+    DMV_TRY(pinned_d2h(c->pin_grad, out.data(), c->d_grad, out.size() * sizeof(double)));
     if (energy)
-        DMV_TRY(copy_d2h(energy, psi->scalars, sizeof(double)));
-    if (grad && np > 0)
-        DMV_TRY(copy_d2h(grad, c->d_grad, sizeof(double) * np));
+        *energy = out[(size_t)np];
+    if (grad)
+        std::copy(out.begin(), out.end() - 1, grad);
     return DMV_OK;
 }
 
@@ -464,7 +468,7 @@ int dmv_expect_zz(dmv_state *s, const double *a, int n_pairs, const int *pi, con
     DMV_TRY(ensure_device());
     const double *da, *db;
     const int *dpi, *dpj;
-    DMV_TRY(upload_terms(&s->terms, &s->cap_terms, s->n, a, n_pairs, pi, pj, b, &da, &db, &dpi, &dpj));
+    DMV_TRY(upload_terms(s->pin_terms, &s->terms, &s->cap_terms, s->n, a, n_pairs, pi, pj, b, &da, &db, &dpi, &dpj));
     prof_begin(DMV_KC_REDUCE);
     DMV_TRY(launch_expect_zz(s->dtype, s->amp, s->n, s->layout, da, n_pairs, dpi, dpj, db, s->ws, s->scalars));
     prof_end(DMV_KC_REDUCE, (double)s->bytes);
@@ -477,7 +481,7 @@ int dmv_expect_diag(dmv_state *s, int n_wires, const int *wires, const double *t
     DMV_CHECK_ARG(out != nullptr, "null output");
     DMV_TRY(ensure_device());
     TableWires W;
-    DMV_TRY(upload_table(&s->terms, &s->cap_terms, s->n, n_wires, wires, table, &W));
+    DMV_TRY(upload_table(s->pin_terms, &s->terms, &s->cap_terms, s->n, n_wires, wires, table, &W));
     prof_begin(DMV_KC_REDUCE);
     DMV_TRY(launch_obs_table(s->dtype, s->amp, nullptr, s->n, s->layout, s->terms, W, s->ws, s->scalars));
     prof_end(DMV_KC_REDUCE, (double)s->bytes);
@@ -556,6 +560,8 @@ int dmv_circuit_destroy(dmv_circuit *c)
         release(c->d_partials);
         release(c->d_terms);
         release(c->d_grad);
+        pinned_free(c->pin_terms);
+        pinned_free(c->pin_grad);
     }
     delete c;
     return DMV_OK;

@@ -161,7 +161,8 @@ struct alignas(16) DevPass {
     // kept by the swizzle since w >= its group width).  0: no split.
     uint32_t split;
     uint32_t lds_half;  // 1: the pass fits kernels with half a tile of LDS
-    uint32_t pad[2];
+    uint32_t ip_begin;  // IP ops of the plan's passes before it
+    uint32_t pad;
 };
 
 // A diagonal the kernels apply as sign flips: exactly diag(1, -1).

@@ -4,6 +4,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
+#include <unordered_map>
 
 namespace dmv {
 
@@ -147,10 +149,18 @@ static std::vector<HostOp> hoist_ips(const std::vector<HostOp> &ops, int n)
         double U[8];
         int group = -1;
     };
+    struct Group {
+        int first = -1, last = -1;  // its IP ops, a list in `ips`
+        bool general = false;       // one of them has an X or Y part
+    };
     std::vector<Run> run(n);
-    std::vector<std::vector<HostOp>> groups;
-    std::vector<int> where;  // per output entry: group index, or -1 for an op
-    std::vector<HostOp> body;
+    std::vector<Group> groups;
+    std::vector<HostOp> ips;
+    std::vector<int> next;   // of each entry of ips
+    std::vector<int> where;  // per output entry: -1 - group, or the index of an op
+    ips.reserve(ops.size() / 2);
+    next.reserve(ops.size() / 2);
+    where.reserve(ops.size() + (size_t)n);
     auto open_run = [&](int q) {
         Run &R = run[q];
         if (R.open)
@@ -160,10 +170,10 @@ static std::vector<HostOp> hoist_ips(const std::vector<HostOp> &ops, int n)
         std::memcpy(R.U, I, sizeof(I));
         R.group = (int)groups.size();
         groups.emplace_back();
-        where.push_back(R.group);
-        body.emplace_back();
+        where.push_back(-1 - R.group);
     };
-    for (const HostOp &op : ops) {
+    for (size_t i = 0; i < ops.size(); i++) {
+        const HostOp &op = ops[i];
         const int q = op.target;
         if (op_is_ip(op.kind)) {
             open_run(q);
@@ -180,7 +190,12 @@ static std::vector<HostOp> hoist_ips(const std::vector<HostOp> &ops, int n)
             ip.m[0] = A[4];  // A10 = ax + i ay
             ip.m[1] = A[5];
             ip.m[2] = A[0];  // A00 = az
-            groups[R.group].push_back(ip);
+            Group &G = groups[(size_t)R.group];
+            G.general = G.general || ip.m[0] != 0.0 || ip.m[1] != 0.0;
+            (G.last >= 0 ? next[(size_t)G.last] : G.first) = (int)ips.size();
+            G.last = (int)ips.size();
+            ips.push_back(ip);
+            next.push_back(-1);
             continue;
         }
         if (op.ctrl == 0) {
@@ -191,28 +206,23 @@ static std::vector<HostOp> hoist_ips(const std::vector<HostOp> &ops, int n)
             std::memcpy(R.U, nu, sizeof(nu));
         } else {
             run[q].open = false;
-            for (int c = 0; c < n; c++)
-                if ((op.ctrl >> c) & 1)
-                    run[c].open = false;
+            for (uint64_t m = op.ctrl; m; m &= m - 1)
+                run[__builtin_ctzll(m)].open = false;
         }
-        where.push_back(-1);
-        body.push_back(op);
+        where.push_back((int)i);
     }
     std::vector<HostOp> out;
     out.reserve(ops.size());
-    for (size_t i = 0; i < where.size(); i++) {
-        if (where[i] < 0) {
-            out.push_back(body[i]);
+    for (int w : where) {
+        if (w >= 0) {
+            out.push_back(ops[(size_t)w]);
             continue;
         }
-        std::vector<HostOp> &G = groups[where[i]];
         // one kind per group, so that the kernel computes its sums once
-        bool general = false;
-        for (const HostOp &ip : G)
-            general = general || ip.m[0] != 0.0 || ip.m[1] != 0.0;
-        for (HostOp &ip : G) {
-            ip.kind = general ? OP_IPG : OP_IPZ;
-            out.push_back(ip);
+        const Group &G = groups[(size_t)(-1 - w)];
+        for (int i = G.first; i >= 0; i = next[(size_t)i]) {
+            ips[(size_t)i].kind = G.general ? OP_IPG : OP_IPZ;
+            out.push_back(ips[(size_t)i]);
         }
     }
     return out;
@@ -304,9 +314,8 @@ std::vector<HostOp> merge_ops(const std::vector<HostOp> &ops)
         } else {
             out.push_back(op);
             pending[op.target] = -1;
-            for (int q = 0; q < 64; q++)
-                if ((op.ctrl >> q) & 1)
-                    pending[q] = -1;
+            for (uint64_t m = op.ctrl; m; m &= m - 1)
+                pending[__builtin_ctzll(m)] = -1;
         }
     }
     return out;
@@ -1188,6 +1197,72 @@ void refresh_ops(const std::vector<HostOp> &given, const std::vector<int> &op_sr
         set_values(ops[(size_t)op_src[i]], &(*dev)[i]);
 }
 
+namespace {
+struct KeptPlan {
+    PlanParams pp;
+    int renaming, mem_order;  // the tunables that make_pass reads
+    std::vector<HostOp> source;
+    std::shared_ptr<const Plan> plan;
+};
+
+struct PlanCache {
+    std::mutex mu;
+    std::unordered_multimap<uint64_t, KeptPlan> kept;
+    size_t ops = 0;
+};
+
+PlanCache &plan_cache()
+{
+    static PlanCache *c = new PlanCache();  // never destroyed: outlives static destructors
+    return *c;
+}
+
+bool same_params(const PlanParams &a, const PlanParams &b)
+{
+    return a.n == b.n && a.k == b.k && a.rlog == b.rlog && a.tlog == b.tlog && a.low_bits == b.low_bits &&
+           a.swz_bits == b.swz_bits && a.max_gen_per_pass == b.max_gen_per_pass && a.half_lds == b.half_lds &&
+           a.max_ip_per_pass == b.max_ip_per_pass && a.gen_auto == b.gen_auto && same_layout(a.layout, b.layout);
+}
+}  // namespace
+
+int shared_plan(const std::vector<HostOp> &ops, const PlanParams &pp, std::shared_ptr<const Plan> *out)
+{
+    const int renaming = tune_value("register_renaming", 1) != 0, mem_order = tune_value("memory_layouts", 0) != 0;
+    uint64_t key = (uint64_t)pp.n + 64 * ((uint64_t)pp.k + 16 * ((uint64_t)pp.tlog + 16 * (uint64_t)pp.swz_bits));
+    for (const HostOp &op : ops)
+        key = (key ^ (op.kind + 16 * (uint64_t)op.target + 1024 * (op.ctrl + 1))) * 0x9E3779B97F4A7C15ull;
+    PlanCache &C = plan_cache();
+    {
+        std::lock_guard<std::mutex> lk(C.mu);
+        const auto range = C.kept.equal_range(key);
+        for (auto it = range.first; it != range.second; ++it) {
+            const KeptPlan &P = it->second;
+            if (P.renaming == renaming && P.mem_order == mem_order && same_params(P.pp, pp) &&
+                same_structure(P.source, ops)) {
+                *out = P.plan;
+                return DMV_OK;
+            }
+        }
+    }
+    auto made = std::make_shared<Plan>();
+    DMV_TRY(build_plan(ops, pp, made.get()));
+    made->logical = {};
+    made->logical_pass = {};
+    made->op_pass = {};
+    *out = made;
+    std::lock_guard<std::mutex> lk(C.mu);
+    const size_t size = ops.size() + made->ops.size();
+    if (size > kKeptOps)
+        return DMV_OK;
+    if (C.ops + size > kKeptOps) {
+        C.kept.clear();
+        C.ops = 0;
+    }
+    C.kept.emplace(key, KeptPlan{pp, renaming, mem_order, ops, made});
+    C.ops += size;
+    return DMV_OK;
+}
+
 int in_order_budget(const std::vector<HostOp> &ops, const PlanParams &pp, int *budget)
 {
     SchedLimits lim;
@@ -1252,7 +1327,7 @@ int build_plan(const std::vector<HostOp> &given, const PlanParams &pp, Plan *out
     plan.ip_begin.assign(plan.passes.size() + 1, 0);
     plan.ip_slots.clear();
     for (size_t p = 0; p < plan.passes.size(); p++) {
-        plan.ip_begin[p] = (uint32_t)plan.ip_slots.size();
+        plan.ip_begin[p] = plan.passes[p].ip_begin = (uint32_t)plan.ip_slots.size();
         for (uint32_t ph = plan.passes[p].phase_begin; ph < plan.passes[p].phase_end; ph++)
             for (uint32_t o = plan.phases[ph].op_begin; o < plan.phases[ph].op_end; o++)
                 if (op_is_ip(plan.ops[o].kind)) {

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <cstdint>
+#include <memory>
 #include <vector>
 
 #include "common.hpp"
@@ -91,6 +92,13 @@ int build_plan(const std::vector<HostOp> &ops, const PlanParams &pp, Plan *out);
 // The budget of GENs a pass (8 or 12) that suits the ops best when passes are
 // filled in op order.
 int in_order_budget(const std::vector<HostOp> &ops, const PlanParams &pp, int *budget);
+// A plan for these ops, kept between calls: found by its parameters and the ops
+// without their matrices (compared in full), so that a program plans a circuit
+// structure once.  Thread-safe; bounded by kKeptOps device ops in all, and dropped
+// together when the next plan would not fit.  Its device ops have the matrices of
+// the call that built it (refresh_ops); `logical` and `op_pass` are left out.
+constexpr size_t kKeptOps = size_t(1) << 18;
+int shared_plan(const std::vector<HostOp> &ops, const PlanParams &pp, std::shared_ptr<const Plan> *out);
 // Whether plans of the two op lists differ in matrices only.
 bool same_structure(const std::vector<HostOp> &a, const std::vector<HostOp> &b);
 // The device ops `dev` of a plan built from ops of the same structure, with

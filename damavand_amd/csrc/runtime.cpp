@@ -188,6 +188,126 @@ int copy_d2h(void *dst, const void *src, uint64_t bytes)
     return DMV_OK;
 }
 
+// Pinned buffers that objects gave back, for the next ones: allocating one takes
+// 100-300 us, which a new circuit's first pass paid for (10 qubits, complex64:
+// 582 us, 240 us with a copy that the host waits for).  At most kPinnedKept bytes.
+constexpr uint64_t kPinnedKept = uint64_t(32) << 20;
+constexpr int kPinnedClasses = 12;  // 4 KiB << class
+
+struct PinnedPool {
+    std::mutex mu;
+    std::vector<void *> kept[kPinnedClasses];
+    uint64_t bytes = 0;
+};
+
+static PinnedPool &pinned_pool()
+{
+    static PinnedPool *pool = new PinnedPool;  // outlives every object's destructor
+    return *pool;
+}
+
+static int pinned_class(uint64_t bytes)
+{
+    int c = 0;
+    while ((uint64_t(4096) << c) < bytes)
+        c++;
+    return c;
+}
+
+static int pinned_take(Pinned &b, uint64_t bytes)
+{
+    const int c = pinned_class(bytes);
+    {
+        PinnedPool &P = pinned_pool();
+        std::lock_guard<std::mutex> lk(P.mu);
+        if (c < kPinnedClasses && !P.kept[c].empty()) {
+            b.p = P.kept[c].back();
+            P.kept[c].pop_back();
+            b.cap = uint64_t(4096) << c;
+            P.bytes -= b.cap;
+            return DMV_OK;
+        }
+    }
+    HIPCALL(hipHostMalloc(&b.p, uint64_t(4096) << c, hipHostMallocDefault));
+    b.cap = uint64_t(4096) << c;
+    return DMV_OK;
+}
+
+// No copy uses b any more.
+static void pinned_give(Pinned &b)
+{
+    if (!b.p)
+        return;
+    const int c = pinned_class(b.cap);
+    {
+        PinnedPool &P = pinned_pool();
+        std::lock_guard<std::mutex> lk(P.mu);
+        if (c < kPinnedClasses && P.bytes + b.cap <= kPinnedKept) {
+            P.kept[c].push_back(b.p);
+            P.bytes += b.cap;
+            b.p = nullptr;
+        }
+    }
+    if (b.p)
+        (void)hipHostFree(b.p);
+    b.p = nullptr;
+    b.cap = 0;
+}
+
+// Room for `bytes` in b, once its last copy out is done.
+static int pinned_ready(Pinned &b, uint64_t bytes)
+{
+    if (!b.done)
+        HIPCALL(hipEventCreateWithFlags(&b.done, hipEventDisableTiming));
+    if (b.busy)
+        HIPCALL(hipEventSynchronize(b.done));
+    b.busy = false;
+    if (bytes > b.cap) {
+        pinned_give(b);
+        DMV_TRY(pinned_take(b, bytes));
+    }
+    return DMV_OK;
+}
+
+constexpr uint64_t kPinnedMax = uint64_t(4) << 20;  // larger copies wait instead
+
+int pinned_h2d(Pinned &b, void *dst, const void *src, uint64_t bytes)
+{
+    if (bytes == 0)
+        return DMV_OK;
+    if (bytes > kPinnedMax)
+        return copy_h2d(dst, src, bytes);
+    DMV_TRY(pinned_ready(b, bytes));
+    std::memcpy(b.p, src, bytes);
+    HIPCALL(hipMemcpyAsync(dst, b.p, bytes, hipMemcpyHostToDevice, stream()));
+    HIPCALL(hipEventRecord(b.done, stream()));
+    b.busy = true;
+    return DMV_OK;
+}
+
+int pinned_d2h(Pinned &b, void *dst, const void *src, uint64_t bytes)
+{
+    if (bytes == 0)
+        return DMV_OK;
+    if (bytes > kPinnedMax)
+        return copy_d2h(dst, src, bytes);
+    DMV_TRY(pinned_ready(b, bytes));
+    HIPCALL(hipMemcpyAsync(b.p, src, bytes, hipMemcpyDeviceToHost, stream()));
+    HIPCALL(hipStreamSynchronize(stream()));
+    std::memcpy(dst, b.p, bytes);
+    return DMV_OK;
+}
+
+void pinned_free(Pinned &b)
+{
+    if (b.busy)
+        (void)hipEventSynchronize(b.done);
+    pinned_give(b);
+    if (b.done)
+        (void)hipEventDestroy(b.done);
+    b = Pinned();
+}
+
 // --------------------------------------------------------------- profiling --
 // get_event and collect run with prof_mu held.
 static hipEvent_t get_event()
@@ -393,6 +513,7 @@ void free_plan(DevicePlan &dp)
     release(dp.d_phases);
     release(dp.d_ops);
     release(dp.d_ip_slots);
+    pinned_free(dp.pin_ops);
     dp.d_passes = nullptr;
     dp.d_phases = nullptr;
     dp.d_ops = nullptr;
@@ -401,16 +522,30 @@ void free_plan(DevicePlan &dp)
     dp.valid = false;
 }
 
-template <class T> static int upload(T *&dptr, size_t &cap, const std::vector<T> &v)
+template <class T> static int room(T *&dptr, size_t &cap, size_t count)
 {
-    if (v.size() > cap) {
+    if (count > cap) {
         release(dptr);
         dptr = nullptr;
-        const size_t want = v.size() + v.size() / 2 + 4;
+        cap = 0;
+        const size_t want = count + count / 2 + 4;
         DMV_TRY(alloc((void **)&dptr, want * sizeof(T)));
         cap = want;
     }
+    return DMV_OK;
+}
+
+template <class T> static int upload(T *&dptr, size_t &cap, const std::vector<T> &v)
+{
+    DMV_TRY(room(dptr, cap, v.size()));
     return copy_h2d(dptr, v.data(), v.size() * sizeof(T));
+}
+
+// A plan's ops, which change with every set of angles: not waited for.
+static int upload_ops(DevicePlan &dp, const std::vector<DevOp> &ops)
+{
+    DMV_TRY(room(dp.d_ops, dp.cap_ops, ops.size()));
+    return pinned_h2d(dp.pin_ops, dp.d_ops, ops.data(), ops.size() * sizeof(DevOp));
 }
 
 int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoint, const std::vector<HostOp> &ops,
@@ -429,7 +564,7 @@ int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoin
     if (!small && same_shape && dp.epoch == tune_epoch() && same_structure(dp.source, merged)) {
         // the same gates at other angles: passes and phases stay, the ops get new matrices
         refresh_ops(merged, dp.plan.op_src, &dp.plan.ops);
-        DMV_TRY(upload(dp.d_ops, dp.cap_ops, dp.plan.ops));
+        DMV_TRY(upload_ops(dp, dp.plan.ops));
         dp.version = version;
         return DMV_OK;
     }
@@ -442,15 +577,16 @@ int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoin
         for (const DevOp &o : dp.small_ops)
             if (o.slot + 1 > dp.plan.n_slots)
                 dp.plan.n_slots = o.slot + 1;
-        DMV_TRY(upload(dp.d_ops, dp.cap_ops, dp.small_ops));
+        DMV_TRY(upload_ops(dp, dp.small_ops));
     } else {
-        Plan plan;
-        DMV_TRY(build_plan(merged, pp, &plan));
-        dp.plan = std::move(plan);
+        std::shared_ptr<const Plan> plan;
+        DMV_TRY(shared_plan(merged, pp, &plan));
+        dp.plan = *plan;
+        refresh_ops(merged, dp.plan.op_src, &dp.plan.ops);
         dp.source = std::move(merged);
         DMV_TRY(upload(dp.d_passes, dp.cap_passes, dp.plan.passes));
         DMV_TRY(upload(dp.d_phases, dp.cap_phases, dp.plan.phases));
-        DMV_TRY(upload(dp.d_ops, dp.cap_ops, dp.plan.ops));
+        DMV_TRY(upload_ops(dp, dp.plan.ops));
         if (!dp.plan.ip_slots.empty())
             DMV_TRY(upload(dp.d_ip_slots, dp.cap_ip, dp.plan.ip_slots));
     }
@@ -518,6 +654,7 @@ void state_destroy(dmv_state *s)
     release(s->scalars);
     release(s->stage);
     release(s->terms);
+    pinned_free(s->pin_terms);
     if (s->bounce) {
         (void)hipStreamSynchronize(stream());
         (void)hipHostFree(s->bounce);

@@ -34,6 +34,15 @@ struct SpreadBuffer {
     hipMemGenericAllocationHandle_t h[kSpreadPieces] = {};
 };
 
+// A pinned host buffer for copies that the host does not wait for (on first
+// use).  `done` marks the last copy out of it.
+struct Pinned {
+    void *p = nullptr;
+    uint64_t cap = 0;
+    hipEvent_t done = nullptr;
+    bool busy = false;
+};
+
 }  // namespace dmv
 
 struct dmv_state {
@@ -52,6 +61,7 @@ struct dmv_state {
     uint64_t stage_cap = 0;       // amplitudes per staged chunk
     double *terms = nullptr;      // Z/ZZ observable terms of dmv_expect_zz (on first use)
     uint64_t cap_terms = 0;
+    dmv::Pinned pin_terms;
     void *bounce = nullptr;       // pinned host buffer (two halves) of device-to-host copies (on first use)
     hipEvent_t bounce_ev[2] = {nullptr, nullptr};
 };
@@ -75,6 +85,7 @@ struct DevicePlan {
     DevOp *d_ops = nullptr;
     int *d_ip_slots = nullptr;    // plan.ip_slots (reverse-sweep plans)
     size_t cap_passes = 0, cap_phases = 0, cap_ops = 0, cap_ip = 0;
+    Pinned pin_ops;
     // hipGraph of the forward passes on one state buffer
     hipGraphExec_t graph = nullptr;
     const void *graph_state = nullptr;
@@ -93,8 +104,9 @@ struct dmv_circuit {
     uint64_t cap_partials = 0;
     double *d_terms = nullptr;      // observable terms
     uint64_t cap_terms = 0;
-    double *d_grad = nullptr;
+    double *d_grad = nullptr;       // gradient, then the energy
     uint64_t cap_grad = 0;
+    dmv::Pinned pin_terms, pin_grad;
 };
 
 namespace dmv {
@@ -110,6 +122,11 @@ int spread_alloc(uint64_t bytes, SpreadBuffer *out);
 void spread_free(SpreadBuffer *b);
 int copy_h2d(void *dst, const void *src, uint64_t bytes);
 int copy_d2h(void *dst, const void *src, uint64_t bytes);
+// Host to device through b without waiting; src may change after the call.
+int pinned_h2d(Pinned &b, void *dst, const void *src, uint64_t bytes);
+// Device to host through b, waiting for it.
+int pinned_d2h(Pinned &b, void *dst, const void *src, uint64_t bytes);
+void pinned_free(Pinned &b);
 int64_t tune_value(const char *name, int64_t dflt);
 uint64_t tune_epoch();
 
