@@ -44,7 +44,7 @@ def expectation(circuit: Circuit, theta: torch.Tensor, a=None, pairs=(), b=None)
 class BatchedAdjointExpectation(torch.autograd.Function):
     """Energies of every circuit of a packed batch at angles ``theta`` (all
     circuits' RX/RY/RZ angles, in PackedBatch.parameters() order), with the
-    gradients from the same persistent launch."""
+    gradients from the same call."""
 
     @staticmethod
     def forward(ctx, theta, batch: PackedBatch, dtype):

@@ -1,4 +1,4 @@
-"""Batched forward + adjoint of many small circuits in one persistent launch."""
+"""Batched forward + adjoint of many small circuits together."""
 from __future__ import annotations
 
 import ctypes
@@ -101,7 +101,7 @@ def pack_circuits(circuits: Sequence) -> PackedBatch:
 
 
 def batch_forward_adjoint_packed(batch: PackedBatch, dtype="complex128"):
-    """One persistent launch over a packed batch: returns (energies, flat
+    """Runs a packed batch: returns (energies, flat
     gradient array in the order of ``batch.param_offset``)."""
     energy = np.empty(batch.count)
     grad = np.empty(max(1, batch.total_params))
@@ -125,7 +125,7 @@ def batch_autotune(batch: PackedBatch, dtype="complex128") -> int:
 
 def batch_forward_adjoint(circuits: Sequence, dtype="complex128"):
     """Runs every circuit from |0>, evaluates its chain observable and its
-    adjoint gradient, all in one persistent kernel launch.
+    adjoint gradient, with a kernel launch per pass of all the circuits.
 
     ``circuits`` is a sequence of ``(n, gates, a, b)``: ``gates`` a list of
     ``(kind, control, target, params)``, ``a`` the n Z coefficients and ``b``

@@ -1,4 +1,4 @@
-// Batched forward + adjoint of many small circuits in one persistent launch.
+// Batched forward + adjoint of many small circuits in common launches.
 #include <algorithm>
 #include <atomic>
 #include <chrono>
@@ -7,6 +7,8 @@
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <unordered_map>
@@ -18,16 +20,14 @@
 
 namespace dmv {
 
-// The batched kernel's tile shape (tile qubits k, log2 threads) and
-// workgroups per CU: from the caller's choice `pin`, else the tunables
-// batch_tile_qubits / batch_threads_log2 / batch_wgs_per_cu, else the tuning
-// table for (qubits of the largest circuit, dtype), else k = 11 on 256
-// threads, two workgroups per CU.
+// The batched kernels' tile shape (tile qubits k, log2 threads): from the
+// caller's choice `pin`, else the tunables batch_tile_qubits /
+// batch_threads_log2, else the tuning table for (qubits of the largest circuit,
+// dtype), else k = 11 on 256 threads.  The workgroups per CU of earlier tuning
+// files and of the tunable batch_wgs_per_cu are checked and have no effect: the
+// grid is the circuits' tiles.
 static void batch_shape(int nmax, int dtype, const TuneChoice *pin, int *k, int *tlog, int *wgs)
 {
-    // three workgroups per CU (the kernel keeps to 168 VGPRs for it);
-    // measured on the 4096-circuit 12-18 qubit batch: complex128 219 -> 183-193
-    // ms and complex64 200 -> 159 ms against two
     *k = 11;
     *tlog = 8;
     *wgs = 3;
@@ -46,6 +46,117 @@ static void batch_shape(int nmax, int dtype, const TuneChoice *pin, int *k, int 
         *wgs = pin->wgs > 0 ? pin->wgs : *wgs;
     }
 }
+
+// One device buffer a call, cut into parts of 256 bytes' alignment, and a host
+// buffer for what goes into the first parts.  Both are kept for the next call up
+// to kKeptBytes each (the host buffer is pinned then); calls from other threads
+// meanwhile allocate their own.
+class Arena {
+public:
+    static constexpr uint64_t kKeptBytes = uint64_t(64) << 20;
+    ~Arena()
+    {
+        if (copying_)  // an error came between the copy and the call's last wait
+            (void)hipStreamSynchronize(stream());
+        {
+            std::lock_guard<std::mutex> lk(mu());
+            Bufs &K = kept();
+            if (b_.cap <= kKeptBytes && !K.dev)
+                std::swap(K.dev, b_.dev), std::swap(K.cap, b_.cap);
+            if (!K.host)
+                std::swap(K.host, b_.host), std::swap(K.host_cap, b_.host_cap);
+        }
+        release(b_.dev);
+        if (b_.host)
+            (void)hipHostFree(b_.host);
+    }
+    static bool give_back()
+    {
+        void *dev = nullptr;
+        {
+            std::lock_guard<std::mutex> lk(mu());
+            std::swap(dev, kept().dev);
+            kept().cap = 0;
+        }
+        release(dev);
+        return dev != nullptr;
+    }
+    uint64_t part(uint64_t bytes)
+    {
+        const uint64_t at = size_;
+        size_ += (std::max<uint64_t>(bytes, 1) + 255) & ~uint64_t(255);
+        return at;
+    }
+    // The buffers, the host's of `filled` bytes.
+    int get(uint64_t filled)
+    {
+        {
+            std::lock_guard<std::mutex> lk(mu());
+            std::swap(b_, kept());
+        }
+        if (b_.cap < size_) {
+            release(b_.dev);
+            b_.dev = nullptr;
+            b_.cap = 0;
+            DMV_TRY(alloc(&b_.dev, size_));
+            b_.cap = size_;
+        }
+        filled_ = filled;
+        if (filled > kKeptBytes) {
+            own_.reset(new char[filled]);
+        } else if (b_.host_cap < filled) {
+            if (b_.host)
+                (void)hipHostFree(b_.host);
+            b_.host = nullptr;
+            b_.host_cap = 0;
+            const uint64_t want = std::min(kKeptBytes, filled + filled / 4);
+            if (hipHostMalloc(&b_.host, want, hipHostMallocDefault) == hipSuccess) {
+                b_.host_cap = want;
+            } else {
+                (void)hipGetLastError();
+                b_.host = nullptr;
+                own_.reset(new char[filled]);
+            }
+        }
+        return DMV_OK;
+    }
+    char *host() const { return own_ ? own_.get() : (char *)b_.host; }
+    int send()
+    {
+        if (own_)
+            return copy_h2d(b_.dev, own_.get(), filled_);
+        if (hipMemcpyAsync(b_.dev, b_.host, filled_, hipMemcpyHostToDevice, stream()) != hipSuccess) {
+            set_error("batch upload failed");
+            return DMV_ERR_HIP;
+        }
+        copying_ = true;
+        return DMV_OK;
+    }
+    void sent() { copying_ = false; }  // the stream has been waited for since
+    template <class T> T *at(uint64_t offset) const { return (T *)((char *)b_.dev + offset); }
+
+private:
+    struct Bufs {
+        void *dev = nullptr, *host = nullptr;
+        uint64_t cap = 0, host_cap = 0;
+    };
+    static Bufs &kept()
+    {
+        static Bufs b;
+        return b;
+    }
+    static std::mutex &mu()
+    {
+        static std::mutex *m = new std::mutex();
+        return *m;
+    }
+    Bufs b_;
+    std::unique_ptr<char[]> own_;
+    uint64_t size_ = 0, filled_ = 0;
+    bool copying_ = false;
+};
+
+bool give_back_batch() { return Arena::give_back(); }
 
 int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_offset, const int *gate_kind,
                           const int *gate_control, const int *gate_target, const double *gate_param,
@@ -75,7 +186,6 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
     DMV_CHECK_ARG(batch_kernel_exists(dtype, rlog, tlog), "no batched kernel for %d tile qubits on %d threads", K,
                   1 << tlog);
     DMV_CHECK_ARG(per_cu >= 1 && per_cu <= 16, "batch_wgs_per_cu must be in [1, 16], got %d", per_cu);
-    const int small_max = K - 1;
 
     // Circuits with the same gates on the same qubits share one plan: their
     // ops differ in matrices only.  Lowering (matrices), planning and filling
@@ -84,12 +194,12 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
         int rc = DMV_OK;
         std::string err;
         int np = 0;
-        double cost = 0.0;
-        bool small = false;
+        uint64_t key = 0;              // of its structure
         int like = -1;                 // the first circuit of the same structure (perhaps itself)
         std::vector<HostOp> f, a;      // merged ops
-        Plan pf, pa;                   // tile path, where like is the circuit itself
+        std::shared_ptr<const Plan> pf, pa;  // where like is the circuit itself
         uint32_t fwd = 0, adj = 0;     // ... its first passes among all
+        uint32_t slots = 0;            // ... and its slots in the slot table
     };
     std::vector<Built> built(count);
     PlanParams pp0;
@@ -101,7 +211,6 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
     const int64_t gen = tune_value("max_gen_per_pass", -1);
     pp0.max_gen_per_pass = gen > 0 ? (int)gen : 8;
     pp0.gen_auto = gen > 0 ? 0 : 1;
-    pp0.max_ip_per_pass = (int)kBatchMaxIp;
     auto lower = [&](int i, Built &B) -> int {
         const int ni = n[i];
         DMV_CHECK_ARG(ni >= 2 && ni <= 24, "batch circuit %d: qubits must be in [2, 24], got %d", i, ni);
@@ -130,19 +239,29 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
                 B.np++;
         B.f = merge_ops(forward_ops(gates));
         B.a = merge_ops(adjoint_ops(gates));
-        B.cost = (double)(B.f.size() + B.a.size()) * std::ldexp(1.0, ni);
-        B.small = ni <= small_max;
+        if (B.f.empty()) {
+            // the first forward pass also writes |0>: a circuit without gates
+            // gets an identity
+            HostOp id{OP_DIAG, 0, 0, {1, 0, 0, 0, 0, 0, 1, 0}, -1, false};
+            B.f.push_back(id);
+        }
+        B.key = (uint64_t)ni;
+        for (const std::vector<HostOp> *v : {&B.f, &B.a})
+            for (const HostOp &op : *v)
+                B.key = (B.key ^ (op.kind + 16 * (uint64_t)op.target + 1024 * (op.ctrl + 1))) * 0x9E3779B97F4A7C15ull;
         return DMV_OK;
     };
     auto plan_one = [&](int i, Built &B) -> int {
         PlanParams pp = pp0;
-        pp.n = n[i];
-        DMV_TRY(build_plan(B.f, pp, &B.pf));
-        DMV_TRY(build_plan(B.a, pp, &B.pa));
-        for (size_t p = 0; p + 1 < B.pa.ip_begin.size(); p++)
-            DMV_CHECK_ARG(B.pa.ip_begin[p + 1] - B.pa.ip_begin[p] <= kBatchMaxIp,
-                          "batch circuit %d: %u parameters in one reverse pass (at most %u)", i,
-                          B.pa.ip_begin[p + 1] - B.pa.ip_begin[p], kBatchMaxIp);
+        pp.n = std::max(n[i], K);  // a circuit smaller than a tile leaves qubits idle
+        pp.max_ip_per_pass = n[i] >= K ? (int)kBatchMaxIp : pp.max_ip_per_pass;
+        DMV_TRY(shared_plan(B.f, pp, &B.pf));
+        DMV_TRY(shared_plan(B.a, pp, &B.pa));
+        const std::vector<uint32_t> &ip = B.pa->ip_begin;
+        for (size_t p = 0; p + 1 < ip.size() && n[i] >= K; p++)
+            DMV_CHECK_ARG(ip[p + 1] - ip[p] <= kBatchMaxIp,
+                          "batch circuit %d: %u parameters in one reverse pass (at most %u)", i, ip[p + 1] - ip[p],
+                          kBatchMaxIp);
         return DMV_OK;
     };
     // fn(i) for i < total, on up to 16 threads taking `grain` at a time or more
@@ -171,29 +290,21 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
             set_error("%s", built[i].err.c_str());
             return built[i].rc;
         }
-    std::vector<int> firsts;  // circuits of a new structure, tile path
+    std::vector<int> firsts;  // circuits of a new structure
     {
-        std::unordered_multimap<uint64_t, int> seen;
-        for (int i = 0; i < count; i++) {
+        std::unordered_map<uint64_t, int> seen;
+        for (int i = 0; i < count; i++)
+            built[i].like = seen.emplace(built[i].key, i).first->second;
+        on_threads(count, 16, [&](int i) {  // a circuit whose key another structure has goes on its own
             Built &B = built[i];
-            if (B.small)
-                continue;
-            uint64_t h = (uint64_t)n[i];
-            for (const std::vector<HostOp> *v : {&B.f, &B.a})
-                for (const HostOp &op : *v)
-                    h = (h ^ (op.kind + 16 * (uint64_t)op.target + 1024 * (op.ctrl + 1))) * 0x9E3779B97F4A7C15ull;
-            const auto range = seen.equal_range(h);
-            for (auto it = range.first; it != range.second && B.like < 0; ++it) {
-                const Built &O = built[it->second];
-                if (n[it->second] == n[i] && same_structure(O.f, B.f) && same_structure(O.a, B.a))
-                    B.like = it->second;
-            }
-            if (B.like < 0) {
+            const Built &O = built[B.like];
+            if (B.like != i &&
+                !(n[B.like] == n[i] && same_structure(O.f, B.f) && same_structure(O.a, B.a)))
                 B.like = i;
-                seen.emplace(h, i);
+        });
+        for (int i = 0; i < count; i++)
+            if (built[i].like == i)
                 firsts.push_back(i);
-            }
-        }
     }
     on_threads((int)firsts.size(), 2, [&](int j) {
         Built &B = built[firsts[(size_t)j]];
@@ -205,41 +316,24 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
     std::vector<BatchCircuit> circ(count);
     std::vector<DevPass> passes;
     std::vector<DevPhase> phases;
-    std::vector<double> cost(count);
-    int nmax = 1;
+    std::vector<int> slots;
     int64_t total_params = 0;
-    uint64_t n_ops = 0, n_sops = 0;
+    uint64_t n_ops = 0;
     for (int i = 0; i < count; i++) {
         Built &B = built[i];
         if (B.rc != DMV_OK) {
             set_error("%s", B.err.c_str());
             return B.rc;
         }
-        const int ni = n[i];
-        nmax = std::max(nmax, ni);
         if (param_offset[i] != total_params) {
             set_error("param_offset[%d] is %d; it must be the number of parameters of the circuits before it (%lld)", i,
                       param_offset[i], (long long)total_params);
             return DMV_ERR_ARG;
         }
         total_params += B.np;
-        BatchCircuit &C = circ[i];
-        C.n = (uint32_t)ni;
-        C.coef = (uint32_t)coef_offset[i];
-        C.grad = (uint32_t)param_offset[i];
-        cost[i] = B.cost;
-        C.small = B.small ? 1u : 0u;
-        if (B.small) {
-            C.fwd_begin = (uint32_t)n_sops;
-            C.fwd_end = C.adj_begin = C.fwd_begin + (uint32_t)B.f.size();
-            C.adj_end = C.adj_begin + (uint32_t)B.a.size();
-            C.fwd_ops = C.adj_ops = 0;
-            n_sops = C.adj_end;
-            continue;
-        }
         if (B.like == i) {
             for (int which = 0; which < 2; which++) {
-                const Plan &plan = which == 0 ? B.pf : B.pa;
+                const Plan &plan = which == 0 ? *B.pf : *B.pa;
                 (which == 0 ? B.fwd : B.adj) = (uint32_t)passes.size();
                 const uint32_t phbase = (uint32_t)phases.size();
                 for (DevPass P : plan.passes) {
@@ -249,99 +343,142 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
                 }
                 phases.insert(phases.end(), plan.phases.begin(), plan.phases.end());
             }
+            B.slots = (uint32_t)slots.size();
+            slots.insert(slots.end(), B.pa->ip_slots.begin(), B.pa->ip_slots.end());
         }
         const Built &T = built[B.like];
+        BatchCircuit &C = circ[i];
+        C.n = (uint32_t)n[i];
+        C.index = (uint32_t)i;
+        C.coef = (uint32_t)coef_offset[i];
+        C.grad = (uint32_t)param_offset[i];
         C.fwd_begin = T.fwd;
-        C.fwd_end = T.fwd + (uint32_t)T.pf.passes.size();
         C.adj_begin = T.adj;
-        C.adj_end = T.adj + (uint32_t)T.pa.passes.size();
+        C.n_ip = (uint32_t)T.pa->ip_slots.size();
+        C.slots = T.slots;
+        C.amps = uint64_t(1) << std::max(n[i], K);
+        C.tiles = (uint32_t)(C.amps >> K);
         C.fwd_ops = n_ops;
-        C.adj_ops = n_ops + T.pf.ops.size();
-        n_ops += T.pf.ops.size() + T.pa.ops.size();
+        C.adj_ops = n_ops + T.pf->ops.size();
+        n_ops += T.pf->ops.size() + T.pa->ops.size();
     }
-    std::vector<DevOp> ops((size_t)n_ops), sops((size_t)n_sops);
-    on_threads(count, 16, [&](int i) {
-        const Built &B = built[i];
-        const BatchCircuit &C = circ[i];
-        std::vector<DevOp> dev;
-        if (B.small) {
-            dev = global_dev_ops(B.f);
-            std::copy(dev.begin(), dev.end(), sops.begin() + C.fwd_begin);
-            dev = global_dev_ops(B.a);
-            std::copy(dev.begin(), dev.end(), sops.begin() + C.adj_begin);
-            return;
+    // Circuits run in groups whose states and partials fit kPoolBytes (one
+    // circuit at least); with the default tiles the 4096-circuit 12-18 qubit
+    // batch in complex128 takes 9.8 + 1.3 GB and is one group.
+    constexpr uint64_t kPoolBytes = uint64_t(16) << 30;
+    const uint32_t waves = (1u << tlog) / 64;
+    struct Group {
+        uint32_t first, count;
+        uint64_t tile_at;            // first entry in by_fwd / by_adj
+        std::vector<uint32_t> fwd_tiles, adj_tiles;
+        uint32_t tiles;
+    };
+    std::vector<Group> groups;
+    std::vector<BatchTile> by_fwd, by_adj;
+    uint64_t pool_amps = 0, pool_parts = 0, pool_tiles = 0;
+    for (int i = 0; i < count;) {
+        Group G{(uint32_t)i, 0, by_fwd.size(), {}, {}, 0};
+        uint64_t amps = 0, parts = 0, tiles = 0;
+        for (; i < count; i++) {
+            BatchCircuit &C = circ[i];
+            const uint64_t a2 = amps + 2 * C.amps, p2 = parts + (uint64_t)C.n_ip * C.tiles * waves;
+            if (G.count > 0 && a2 * amp_bytes(dtype) + p2 * 8 > kPoolBytes)
+                break;
+            C.state = amps;
+            C.parts = parts;
+            C.tile0 = (uint32_t)tiles;
+            amps = a2;
+            parts = p2;
+            tiles += C.tiles;
+            G.count++;
         }
-        const Built &T = built[B.like];
-        dev = T.pf.ops;
-        refresh_ops(B.f, T.pf.op_src, &dev);
-        std::copy(dev.begin(), dev.end(), ops.begin() + (int64_t)C.fwd_ops);
-        dev = T.pa.ops;
-        refresh_ops(B.a, T.pa.op_src, &dev);
-        std::copy(dev.begin(), dev.end(), ops.begin() + (int64_t)C.adj_ops);
-    });
-    built.clear();
-    built.shrink_to_fit();
-    std::vector<uint32_t> order(count);
-    for (int i = 0; i < count; i++)
-        order[i] = (uint32_t)i;
-    std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return cost[x] > cost[y]; });
+        DMV_CHECK_ARG(tiles <= 0x7FFFFFFFull, "batch too large");
+        G.tiles = (uint32_t)tiles;
+        pool_amps = std::max(pool_amps, amps);
+        pool_parts = std::max(pool_parts, parts);
+        pool_tiles = std::max(pool_tiles, tiles);
+        for (int which = 0; which < 2; which++) {
+            auto levels = [&](uint32_t c) {
+                const Built &T = built[built[c].like];
+                return (which == 0 ? *T.pf : *T.pa).passes.size();
+            };
+            std::vector<uint32_t> order(G.count);
+            for (uint32_t j = 0; j < G.count; j++)
+                order[j] = G.first + j;
+            std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return levels(x) > levels(y); });
+            std::vector<BatchTile> &list = which == 0 ? by_fwd : by_adj;
+            std::vector<uint32_t> &per_level = which == 0 ? G.fwd_tiles : G.adj_tiles;
+            per_level.assign(levels(order[0]), 0);
+            for (uint32_t c : order) {
+                for (uint32_t t = 0; t < circ[c].tiles; t++)
+                    list.push_back({c, t});
+                for (size_t p = 0; p < levels(c); p++)
+                    per_level[p] += circ[c].tiles;
+            }
+        }
+        groups.push_back(std::move(G));
+    }
 
     // host work and argument checks are done: only now touch the device
     DMV_TRY(ensure_device());
-    uint32_t grid = (uint32_t)std::min<int64_t>(count, (int64_t)device_cus() * per_cu);
-    const uint64_t slot_amps = uint64_t(1) << std::max(nmax, K);
-    const uint64_t scratch_bytes = (uint64_t)grid * 2 * slot_amps * amp_bytes(dtype);
-
     int64_t coef_len = 0;
     for (int i = 0; i < count; i++)
         coef_len = std::max<int64_t>(coef_len, (int64_t)coef_offset[i] + 2 * n[i] - 1);
 
-    // device buffers
-    struct Buf {
-        void *p = nullptr;
-        ~Buf() { release(p); }
-    } b_circ, b_order, b_counter, b_passes, b_phases, b_ops, b_sops, b_coef, b_scratch, b_energy, b_grad;
-    DMV_TRY(alloc(&b_circ.p, circ.size() * sizeof(BatchCircuit)));
-    DMV_TRY(alloc(&b_order.p, order.size() * sizeof(uint32_t)));
-    DMV_TRY(alloc(&b_counter.p, 64));
-    DMV_TRY(alloc(&b_passes.p, std::max<size_t>(1, passes.size()) * sizeof(DevPass)));
-    DMV_TRY(alloc(&b_phases.p, std::max<size_t>(1, phases.size()) * sizeof(DevPhase)));
-    DMV_TRY(alloc(&b_ops.p, std::max<size_t>(1, ops.size()) * sizeof(DevOp)));
-    DMV_TRY(alloc(&b_sops.p, std::max<size_t>(1, sops.size()) * sizeof(DevOp)));
-    DMV_TRY(alloc(&b_coef.p, (uint64_t)std::max<int64_t>(1, coef_len) * sizeof(double)));
-    DMV_TRY(alloc(&b_scratch.p, scratch_bytes));
-    DMV_TRY(alloc(&b_energy.p, (uint64_t)count * sizeof(double)));
-    DMV_TRY(alloc(&b_grad.p, (uint64_t)std::max<int64_t>(1, total_params) * sizeof(double)));
-    DMV_TRY(copy_h2d(b_circ.p, circ.data(), circ.size() * sizeof(BatchCircuit)));
-    DMV_TRY(copy_h2d(b_order.p, order.data(), order.size() * sizeof(uint32_t)));
-    DMV_TRY(copy_h2d(b_passes.p, passes.data(), passes.size() * sizeof(DevPass)));
-    DMV_TRY(copy_h2d(b_phases.p, phases.data(), phases.size() * sizeof(DevPhase)));
-    DMV_TRY(copy_h2d(b_ops.p, ops.data(), ops.size() * sizeof(DevOp)));
-    DMV_TRY(copy_h2d(b_sops.p, sops.data(), sops.size() * sizeof(DevOp)));
-    DMV_TRY(copy_h2d(b_coef.p, coef, (uint64_t)coef_len * sizeof(double)));
+    // One device buffer: what the host fills in first, so that it goes over in
+    // one copy, then the results, partials and states.
+    Arena A;
+    const uint64_t o_circ = A.part(circ.size() * sizeof(BatchCircuit));
+    const uint64_t o_fwd = A.part(by_fwd.size() * sizeof(BatchTile));
+    const uint64_t o_adj = A.part(by_adj.size() * sizeof(BatchTile));
+    const uint64_t o_passes = A.part(passes.size() * sizeof(DevPass));
+    const uint64_t o_phases = A.part(phases.size() * sizeof(DevPhase));
+    const uint64_t o_ops = A.part(n_ops * sizeof(DevOp));
+    const uint64_t o_slots = A.part(slots.size() * sizeof(int));
+    const uint64_t o_coef = A.part((uint64_t)coef_len * sizeof(double));
+    const uint64_t o_energy = A.part((uint64_t)count * sizeof(double) + (uint64_t)total_params * sizeof(double));
+    const uint64_t o_grad = o_energy + (uint64_t)count * sizeof(double);
+    const uint64_t o_eparts = A.part(pool_tiles * sizeof(double));
+    const uint64_t o_parts = A.part(pool_parts * sizeof(double));
+    const uint64_t o_pool = A.part(pool_amps * (uint64_t)amp_bytes(dtype));
+    DMV_TRY(A.get(o_energy));
+    char *filled = A.host();
+    std::memcpy(filled + o_circ, circ.data(), circ.size() * sizeof(BatchCircuit));
+    std::memcpy(filled + o_fwd, by_fwd.data(), by_fwd.size() * sizeof(BatchTile));
+    std::memcpy(filled + o_adj, by_adj.data(), by_adj.size() * sizeof(BatchTile));
+    std::memcpy(filled + o_passes, passes.data(), passes.size() * sizeof(DevPass));
+    std::memcpy(filled + o_phases, phases.data(), phases.size() * sizeof(DevPhase));
+    std::memcpy(filled + o_slots, slots.data(), slots.size() * sizeof(int));
+    std::memcpy(filled + o_coef, coef, (size_t)coef_len * sizeof(double));
+    DevOp *ops = (DevOp *)(filled + o_ops);
+    on_threads(count, 16, [&](int i) {
+        const Built &B = built[i], &T = built[B.like];
+        std::vector<DevOp> dev = T.pf->ops;
+        refresh_ops(B.f, T.pf->op_src, &dev);
+        std::copy(dev.begin(), dev.end(), ops + circ[i].fwd_ops);
+        dev = T.pa->ops;
+        refresh_ops(B.a, T.pa->op_src, &dev);
+        std::copy(dev.begin(), dev.end(), ops + circ[i].adj_ops);
+    });
+    DMV_TRY(A.send());
 
     BatchLaunch L;
-    L.circ = (const BatchCircuit *)b_circ.p;
-    L.order = (const uint32_t *)b_order.p;
-    L.count = (uint32_t)count;
-    L.counter = (uint32_t *)b_counter.p;
-    L.passes = (const DevPass *)b_passes.p;
-    L.phases = (const DevPhase *)b_phases.p;
-    L.ops = (const DevOp *)b_ops.p;
-    L.sops = (const DevOp *)b_sops.p;
-    L.coef = (const double *)b_coef.p;
-    L.scratch = b_scratch.p;
-    L.slot_amps = slot_amps;
-    L.energy = (double *)b_energy.p;
-    L.grad = (double *)b_grad.p;
-    L.grid = grid;
+    L.circ = A.at<BatchCircuit>(o_circ);
+    L.passes = A.at<DevPass>(o_passes);
+    L.phases = A.at<DevPhase>(o_phases);
+    L.ops = A.at<DevOp>(o_ops);
+    L.slots = A.at<int>(o_slots);
+    L.coef = A.at<double>(o_coef);
+    L.pool = A.at<void>(o_pool);
+    L.parts = A.at<double>(o_parts);
+    L.energy_parts = A.at<double>(o_eparts);
+    L.energy = A.at<double>(o_energy);
+    L.grad = A.at<double>(o_grad);
     L.rlog = rlog;
     L.tlog = tlog;
-    // streaming loads and stores once the scratch states take twice the
-    // last-level cache (512 MiB): measured on the 4096-circuit 12-18 qubit
-    // batch (6 GiB of scratch), complex128 169 -> 159 ms and complex64
-    // 120-123 -> 111-118 ms
-    L.nt = tune_value("nontemporal", scratch_bytes >= (uint64_t(512) << 20) ? 1 : 0) != 0;
+    // streaming loads and stores once the states take twice the last-level
+    // cache (512 MiB)
+    L.nt = tune_value("nontemporal", pool_amps * amp_bytes(dtype) >= (uint64_t(512) << 20) ? 1 : 0) != 0;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (kernel_ms && (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)) {
         if (e0)
@@ -352,7 +489,20 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
     if (kernel_ms)
         (void)hipEventRecord(e0, stream());
     prof_begin(DMV_KC_BATCH);
-    int rc = launch_batch(dtype, L);
+    int rc = DMV_OK;
+    for (const Group &G : groups) {
+        L.first = G.first;
+        L.count = G.count;
+        L.by_fwd = A.at<BatchTile>(o_fwd) + G.tile_at;
+        L.by_adj = A.at<BatchTile>(o_adj) + G.tile_at;
+        L.all_tiles = G.tiles;
+        L.fwd_levels = (uint32_t)G.fwd_tiles.size();
+        L.adj_levels = (uint32_t)G.adj_tiles.size();
+        L.fwd_tiles = G.fwd_tiles.data();
+        L.adj_tiles = G.adj_tiles.data();
+        if (rc == DMV_OK)
+            rc = launch_batch(dtype, L);
+    }
     if (kernel_ms) {
         (void)hipEventRecord(e1, stream());
         float ms = 0.f;
@@ -365,17 +515,16 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
     DMV_TRY(rc);
     double bytes = 0.0;
     for (int i = 0; i < count; i++) {
-        const double sb = std::ldexp((double)amp_bytes(dtype), n[i]);
-        const BatchCircuit &C = circ[i];
-        if (C.small)
-            bytes += 4.0 * sb;  // reads and writes of psi and lambda stay in LDS
-        else
-            bytes += 2.0 * sb * (C.fwd_end - C.fwd_begin) + 4.0 * sb * (C.adj_end - C.adj_begin) + 3.0 * sb;
+        const double sb = (double)circ[i].amps * amp_bytes(dtype);
+        const Built &T = built[built[i].like];
+        bytes += 2.0 * sb * T.pf->passes.size() + 4.0 * sb * T.pa->passes.size() + 3.0 * sb;
     }
     prof_end(DMV_KC_BATCH, bytes);
-    DMV_TRY(copy_d2h(energy, b_energy.p, (uint64_t)count * sizeof(double)));
-    if (total_params > 0)
-        DMV_TRY(copy_d2h(grad, b_grad.p, (uint64_t)total_params * sizeof(double)));
+    std::vector<double> out((size_t)count + (size_t)total_params);
+    DMV_TRY(copy_d2h(out.data(), A.at<void>(o_energy), out.size() * sizeof(double)));
+    A.sent();
+    std::copy(out.begin(), out.begin() + count, energy);
+    std::copy(out.begin() + count, out.end(), grad);
     return DMV_OK;
 }
 

@@ -27,37 +27,45 @@ int launch_small(int dtype, void *state, int n, const DevOp *ops, uint32_t n_ops
 // partials[slot].
 int launch_small_adjoint(int dtype, void *psi, void *lam, int n, const DevOp *ops, uint32_t n_ops,
                          double *partials);
-// Batched persistent launch: one circuit per queue entry.  Circuits with
-// n < k run with psi and lambda in LDS (ops in `sops`, global positions);
-// larger ones run tile passes over per-workgroup scratch states.
-// IP ops (gradient outputs) per reverse pass that the batched kernel keeps
-// per-wave sums for in LDS; the host rejects plans with more.
+// Batched circuits (k_batch.hip): launches over the tiles of all circuits.
+// IP ops (gradient outputs) of one reverse pass of a circuit of more qubits than
+// a tile; the host rejects plans with more.
 constexpr uint32_t kBatchMaxIp = 128;
 struct BatchCircuit {
-    uint32_t n, small;
-    uint32_t fwd_begin, fwd_end;  // pass range (tile path) or op range (small path)
-    uint32_t adj_begin, adj_end;
-    uint32_t coef;                // a_q at coef[coef + q], b_q at coef[coef + n + q]
-    uint32_t grad;                // gradient of parameter k at grad[grad + k]
-    uint64_t fwd_ops, adj_ops;    // tile path: the circuit's ops; phases count from there
+    uint32_t n;
+    uint32_t fwd_begin, adj_begin;  // first passes
+    uint32_t coef;                  // a_q at coef[coef + q], b_q at coef[coef + n + q]
+    uint32_t grad;                  // gradient of parameter k at grad[grad + k]
+    uint32_t index;                 // its place in the caller's arrays
+    uint32_t n_ip, slots;           // IP ops; their parameters are slots[slots ..] of the slot table
+    uint32_t tiles, tile0;          // tiles, and the first among the energy parts
+    uint64_t amps;                  // amplitudes of a state (at least a tile)
+    uint64_t state;                 // psi in the pool; lambda follows
+    uint64_t parts;                 // gradient partials [IP op][tile][wave]
+    uint64_t fwd_ops, adj_ops;      // its ops; phases count from there
 };
+struct BatchTile {
+    uint32_t circuit, tile;
+};
+// One group of circuits.  The tiles of the circuits with the most passes come
+// first, so that the first fwd_tiles[p] (adj_tiles[p]) are those of pass p.
 struct BatchLaunch {
     const BatchCircuit *circ;
-    const uint32_t *order;
-    uint32_t count;
-    uint32_t *counter;
+    uint32_t first, count;          // the group's circuits
+    const BatchTile *by_fwd, *by_adj;
+    uint32_t all_tiles, fwd_levels, adj_levels;
+    const uint32_t *fwd_tiles, *adj_tiles;  // host
     const DevPass *passes;
     const DevPhase *phases;
     const DevOp *ops;
-    const DevOp *sops;
+    const int *slots;
     const double *coef;
-    void *scratch;        // grid * 2 * slot_amps amplitudes
-    uint64_t slot_amps;
+    void *pool;
+    double *parts, *energy_parts;
     double *energy;
     double *grad;
-    uint32_t grid;
     int rlog, tlog;       // tile shape: 2^rlog amplitudes per thread, 2^tlog threads
-    bool nt;              // streaming loads and stores of the scratch states (default shape only)
+    bool nt;              // streaming loads and stores of the states (default shape only)
 };
 // Whether the batched kernel is built for this tile shape.
 bool batch_kernel_exists(int dtype, int rlog, int tlog);

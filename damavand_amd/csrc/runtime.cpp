@@ -153,6 +153,10 @@ int alloc(void **p, uint64_t bytes)
     if (bytes == 0)
         return DMV_OK;
     hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess && give_back_batch()) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
     if (e != hipSuccess) {
         (void)hipGetLastError();
         *p = nullptr;

@@ -115,6 +115,8 @@ int ensure_device();              // initialises the context, selects the device
 int synchronize();
 int alloc(void **p, uint64_t bytes);
 void release(void *p);
+// Frees the device buffer that batches keep between calls (false: there is none).
+bool give_back_batch();
 // Large state buffers whose physical pieces lie kSpreadStride apart (see
 // spread_alloc.cpp); DMV_ERR_MEMORY when the device cannot do it, with no
 // error left set, so that the caller falls back to alloc.

@@ -1,5 +1,5 @@
 // Device building blocks of the fused tile executor, shared by the big-state
-// pass kernels, the whole-state kernels and the batched persistent kernel.
+// pass kernels, the whole-state kernels and the batched kernels.
 //
 // The host resolves every op against the phase's register/thread layout and
 // against the register renaming in force (see make_pass in plan.cpp):

@@ -7,7 +7,7 @@
 //  * forward: tile qubits, threads per workgroup, GEN budget per pass and
 //    streaming stores of the fused passes;
 //  * adjoint: tile qubits, threads and GEN budget of the reverse sweep;
-//  * batch: tile shape and workgroups per CU of the persistent kernel.
+//  * batch: tile shape.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -360,24 +360,22 @@ int autotune_batch(int count, int dtype, const int *n, const int *gate_offset, c
     std::vector<double> energy(count), grad(std::max<int64_t>(1, n_params));
     TuneChoice best;
     double best_ms = 1e300;
-    for (auto [k, tlog] : std::vector<std::pair<int, int>>{{11, 8}, {10, 8}, {10, 7}, {12, 9}})
-        for (int wgs : {1, 2, 3, 4}) {
-            TuneChoice cand;
-            cand.k = k;
-            cand.tlog = tlog;
-            cand.wgs = wgs;
-            double ms = 0.0, t = 0.0;
-            for (int r = 0; r < 2; r++) {  // the second run is timed
-                DMV_TRY(batch_forward_adjoint(count, dtype, n, gate_offset, gate_kind, gate_control, gate_target,
-                                              gate_param, coef_offset, coef, param_offset, energy.data(),
-                                              grad.data(), &cand, &t));
-                ms = t;
-            }
-            if (ms < best_ms) {
-                best_ms = ms;
-                best = cand;
-            }
+    for (auto [k, tlog] : std::vector<std::pair<int, int>>{{11, 8}, {10, 8}, {10, 7}, {12, 9}}) {
+        TuneChoice cand;
+        cand.k = k;
+        cand.tlog = tlog;
+        double ms = 0.0, t = 0.0;
+        for (int r = 0; r < 2; r++) {  // the second run is timed
+            DMV_TRY(batch_forward_adjoint(count, dtype, n, gate_offset, gate_kind, gate_control, gate_target,
+                                          gate_param, coef_offset, coef, param_offset, energy.data(),
+                                          grad.data(), &cand, &t));
+            ms = t;
         }
+        if (ms < best_ms) {
+            best_ms = ms;
+            best = cand;
+        }
+    }
     best.ms = best_ms;
     tune_store(tune_key(nmax, dtype, "batch"), best);
     if (chosen)

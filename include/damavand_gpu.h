@@ -297,7 +297,7 @@ int dmv_circuit_plan_ops(dmv_circuit *c, int dtype, int tile_qubits, int *kind, 
 int dmv_circuit_plan_json(dmv_circuit *c, int dtype, int adjoint, int tile_qubits, int threads_log2,
                           int max_gen_per_pass, char *buffer, uint64_t capacity, uint64_t *length);
 
-/* ---- batched forward + adjoint: many small circuits in one persistent launch ---- */
+/* ---- batched forward + adjoint: many small circuits, a launch per pass of all of them ---- */
 /* Circuit i has n[i] qubits and the gates gate_kind/control/target/param in
  * [gate_offset[i], gate_offset[i+1]); its observable is the Z/ZZ chain
  * H = sum_q a_q Z_q + sum_{q<n-1} b_q Z_q Z_{q+1} with a_q at
@@ -309,8 +309,7 @@ int dmv_circuit_plan_json(dmv_circuit *c, int dtype, int adjoint, int tile_qubit
  * (param_offset[0] = 0), so grad holds sum_i (parameters of circuit i)
  * values; anything else returns DMV_ERR_ARG before the device is touched.
  * Circuits have 2 to 24 qubits, and a circuit's reverse sweep may hold at
- * most 128 parametrised gates in one fused pass (the kernel keeps their
- * per-wave sums in LDS); a batch with more returns DMV_ERR_ARG. */
+ * most 128 parametrised gates in one fused pass; a batch with more returns DMV_ERR_ARG. */
 int dmv_batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_offset,
                               const int *gate_kind, const int *gate_control,
                               const int *gate_target, const double *gate_param,
@@ -326,7 +325,7 @@ enum {
     DMV_KC_REDUCE = 3,   /* norm / <Z> / <H> / probabilities */
     DMV_KC_SAMPLE = 4,   /* sampler */
     DMV_KC_ADJOINT = 5,  /* adjoint tile pass */
-    DMV_KC_BATCH = 6,    /* batched persistent kernel */
+    DMV_KC_BATCH = 6,    /* batched kernels */
     DMV_KC_COPY = 7,     /* device copy (bandwidth reference) */
     DMV_KC_COUNT = 8
 };
@@ -342,14 +341,17 @@ int dmv_synchronize(void);
 
 /* ---- tuning ---- */
 /* Sets a tunable, e.g. "tile_qubits" / "adjoint_tile_qubits" (9..13),
- * "tile_threads_log2" (6..9), "max_gen_per_pass" (default: 8 or 12, chosen per
- * circuit for forward plans by their pass and phase counts; 8 for reverse
- * sweeps), "nontemporal" (0/1: streaming loads and stores; default 1 for
+ * "tile_threads_log2" (6..9), "max_gen_per_pass" (up to 8: gates in order, at
+ * most so many matrices a pass; more: passes are searched for within it;
+ * default: searched for without it, or in order where that is cheaper;
+ * complex64 forwards: in order, 8 or 12),
+ * "nontemporal" (0/1: streaming loads and stores; default 1 for
  * forward passes over states of 2 GiB and more, for reverse sweeps whose
  * two states together take 512 MiB and more, and for batches whose scratch
  * states take 512 MiB and more),
  * "gate_pairs_per_thread" (1, 2, 4), "batch_tile_qubits",
- * "batch_threads_log2", "batch_wgs_per_cu", "graph" (0/1: replay forward
+ * "batch_threads_log2", "batch_wgs_per_cu" (1..16, without
+ * effect: a batch's launches fill the chip), "graph" (0/1: replay forward
  * passes from a captured hipGraph), "half_lds" (0/1, default 1: forward
  * passes of the default tile shapes split their LDS transposes in two
  * rounds through half a tile of LDS, so three workgroups share a CU).
