@@ -454,10 +454,10 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
     on_threads(count, 16, [&](int i) {
         const Built &B = built[i], &T = built[B.like];
         std::vector<DevOp> dev = T.pf->ops;
-        refresh_ops(B.f, T.pf->op_src, &dev);
+        refresh_ops(B.f, false, T.pf->op_src, &dev);
         std::copy(dev.begin(), dev.end(), ops + circ[i].fwd_ops);
         dev = T.pa->ops;
-        refresh_ops(B.a, T.pa->op_src, &dev);
+        refresh_ops(B.a, false, T.pa->op_src, &dev);
         std::copy(dev.begin(), dev.end(), ops + circ[i].adj_ops);
     });
     DMV_TRY(A.send());

@@ -41,7 +41,8 @@ constexpr int kMaxQubits = 33;      // 2^33 complex128 = 128 GiB, one MI355X
 constexpr int kMaxRegs = 32;        // amplitudes per thread in a tile kernel
 constexpr int kMaxThreadBits = 9;   // up to 512 threads per tile workgroup
 constexpr int kMaxTileQubits = 13;  // 2^13 * 8 B (c64) or 2^12 * 16 B (c128) = 64 KiB of LDS
-constexpr int kSmallMaxQubits = 8;  // whole-state kernels: an amplitude per thread, in LDS
+constexpr int kSmallMaxQubits = 8;       // whole-state kernels: an amplitude per thread, in LDS
+constexpr int kSmallMaxQubitsFp32 = 13;  // ... of FP32 forward plans (64 KiB of LDS)
 
 inline int amp_bytes(int dtype) { return dtype == DMV_C64 ? 8 : 16; }
 // Low qubits a tile always keeps in lanes so that 8 consecutive lanes read one
@@ -267,7 +268,7 @@ inline DMV_HD uint64_t elem(uint64_t i, StateLayout L)
     return e;
 }
 
-static_assert(kSmallMaxQubits <= 17,
+static_assert(kSmallMaxQubits <= 17 && kSmallMaxQubitsFp32 <= 18,
               "whole-state kernels index states of the plain layout");
 static_assert(kMaxQubits - 17 <= 16, "span index wider than the swizzle");
 

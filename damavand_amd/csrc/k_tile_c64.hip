@@ -1,4 +1,5 @@
-// Fused tile passes, complex64 states computed in FP64 (see tile_body).
+// Fused tile passes, complex64 states computed in FP64 (see tile_body): the
+// forward of a gradient.
 #include "k_tile_impl.hpp"
 
 namespace dmv {
@@ -6,8 +7,6 @@ namespace dmv {
 int launch_tile_c64(int rlog, int tlog, bool nt, bool half, void *state, int n, StateLayout L, const DevPass *passes,
                     const DevPhase *phases, const DevOp *ops, uint32_t pass_idx)
 {
-    if (rlog == 5)
-        return launch_tile_c64_wide(rlog, tlog, nt, half, state, n, L, passes, phases, ops, pass_idx);
     if (half) {
         if (tlog == 8 && rlog == 4) return run_tile<float, double, 4, 8, true>(nt, state, n, L, passes, phases, ops, pass_idx);
         return kNotHandled;

@@ -388,16 +388,6 @@ void special_unitary(std::vector<HostOp> *ops)
 
 static uint64_t op_qubits(const HostOp &op) { return (uint64_t(1) << op.target) | op.ctrl; }
 
-// Local index of a global bit mask: bit j of the result is qubit qpos[j].
-static uint64_t to_local(uint64_t global, const uint32_t *qpos, int k)
-{
-    uint64_t l = 0;
-    for (int j = 0; j < k; j++)
-        if ((global >> qpos[j]) & 1)
-            l |= uint64_t(1) << j;
-    return l;
-}
-
 static uint64_t deposit(uint64_t x, const uint32_t *pos, int nbits)
 {
     uint64_t r = 0;
@@ -1189,10 +1179,11 @@ static void set_values(const HostOp &h, DevOp *op)
         op->plain = diag_is_sign_flip(op->m) ? 1u : 0u;
 }
 
-void refresh_ops(const std::vector<HostOp> &given, const std::vector<int> &op_src, std::vector<DevOp> *dev)
+void refresh_ops(const std::vector<HostOp> &given, bool fp32, const std::vector<int> &op_src, std::vector<DevOp> *dev)
 {
     std::vector<HostOp> ops = given;
-    special_unitary(&ops);
+    if (!fp32)
+        special_unitary(&ops);
     for (size_t i = 0; i < dev->size(); i++)
         set_values(ops[(size_t)op_src[i]], &(*dev)[i]);
 }
@@ -1221,7 +1212,7 @@ bool same_params(const PlanParams &a, const PlanParams &b)
 {
     return a.n == b.n && a.k == b.k && a.rlog == b.rlog && a.tlog == b.tlog && a.low_bits == b.low_bits &&
            a.swz_bits == b.swz_bits && a.max_gen_per_pass == b.max_gen_per_pass && a.half_lds == b.half_lds &&
-           a.max_ip_per_pass == b.max_ip_per_pass && a.gen_auto == b.gen_auto && same_layout(a.layout, b.layout);
+           a.max_ip_per_pass == b.max_ip_per_pass && a.gen_auto == b.gen_auto && a.fp32 == b.fp32 && same_layout(a.layout, b.layout);
 }
 }  // namespace
 
@@ -1284,7 +1275,8 @@ int in_order_budget(const std::vector<HostOp> &ops, const PlanParams &pp, int *b
 int build_plan(const std::vector<HostOp> &given, const PlanParams &pp, Plan *out)
 {
     std::vector<HostOp> ops = given;
-    special_unitary(&ops);
+    if (!pp.fp32)
+        special_unitary(&ops);
     DMV_CHECK_ARG(pp.k == pp.rlog + pp.tlog, "tile qubits %d != %d + %d", pp.k, pp.rlog, pp.tlog);
     DMV_CHECK_ARG(pp.n >= pp.k && pp.k <= kMaxTileQubits && pp.rlog >= 1 &&
                       (1 << pp.rlog) <= kMaxRegs && pp.tlog <= kMaxThreadBits &&
@@ -1307,12 +1299,16 @@ int build_plan(const std::vector<HostOp> &given, const PlanParams &pp, Plan *out
     // takes as many passes either way.
     constexpr int kInOrder = 8;
     std::vector<PassCut> cuts;
-    if (pp.gen_auto || pp.max_gen_per_pass <= kInOrder) {
+    if (pp.fp32) {
+        if (pp.gen_auto)
+            DMV_TRY(in_order_budget(ops, pp, &lim.max_gen));
+        DMV_TRY(first_fit_passes(ops, so, lim, pp, &cuts));
+    } else if (pp.gen_auto || pp.max_gen_per_pass <= kInOrder) {
         if (pp.gen_auto)
             lim.max_gen = kInOrder;
         DMV_TRY(first_fit_passes(ops, so, lim, pp, &cuts));
     }
-    if (pp.gen_auto || pp.max_gen_per_pass > kInOrder) {
+    if (!pp.fp32 && (pp.gen_auto || pp.max_gen_per_pass > kInOrder)) {
         if (pp.gen_auto)
             lim.max_gen = 1 << 30;
         std::vector<PassCut> more;

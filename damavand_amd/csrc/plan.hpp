@@ -64,6 +64,10 @@ struct PlanParams {
     int nontemporal = 0;   // forward passes: streaming (nontemporal) loads and stores
     int half_lds = 0;      // forward passes: split transposes where a pass allows (half-LDS kernels exist)
     int max_ip_per_pass = 1 << 30;  // IP ops of a pass (a run of IP ops on one qubit stays together)
+    // complex64 forward plans (Circuit forward): FP32 arithmetic, general
+    // matrices and ops in order.  What a program samples from a complex64 state is
+    // decided by its last bits, so these states keep theirs.
+    int fp32 = 0;
     int gen_auto = 0;      // build_plan chooses the passes by cost instead (max_gen_per_pass is not used)
     StateLayout layout = kPlainLayout;  // element map of the states the plan runs on
 };
@@ -102,8 +106,8 @@ int shared_plan(const std::vector<HostOp> &ops, const PlanParams &pp, std::share
 // Whether plans of the two op lists differ in matrices only.
 bool same_structure(const std::vector<HostOp> &a, const std::vector<HostOp> &b);
 // The device ops `dev` of a plan built from ops of the same structure, with
-// the matrices of `ops`.
-void refresh_ops(const std::vector<HostOp> &ops, const std::vector<int> &op_src, std::vector<DevOp> *dev);
+// the matrices of `ops` (fp32: the plan's).
+void refresh_ops(const std::vector<HostOp> &ops, bool fp32, const std::vector<int> &op_src, std::vector<DevOp> *dev);
 // Checks every invariant the tile kernels rely on (index ranges, layouts,
 // register bits).  Called before a plan is uploaded.
 int validate_plan(const Plan &plan, const PlanParams &pp);

@@ -424,9 +424,10 @@ bool gate_nontemporal(uint32_t target, int dtype)
 }
 
 // ------------------------------------------------------------------- plans --
-PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const TuneChoice *pin)
+PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const TuneChoice *pin, bool inner)
 {
     PlanParams pp;
+    pp.fp32 = dtype == DMV_C64 && !adjoint && !inner ? 1 : 0;
     pp.n = n;
     pp.layout = layout;
     pp.low_bits = coalesce_bits(dtype);
@@ -435,9 +436,9 @@ PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const
     if (runs > pp.low_bits && runs <= 6)
         pp.low_bits = (int)runs;
     pp.swz_bits = dtype == DMV_C64 ? 4 : 3;
-    // defaults: 256 threads; k = 12 forward, 11 for reverse sweeps, which hold
-    // psi and lambda in registers together
-    int k = adjoint ? 11 : 12;
+    // defaults: 256 threads; k = 12 forward (FP32: 13), 11 for reverse sweeps,
+    // which hold psi and lambda in registers together
+    int k = adjoint ? 11 : (pp.fp32 ? 13 : 12);
     // streaming (nontemporal) loads and stores: forward passes from 2 GiB
     // states up (measured 1.5-3.5% faster per pass at 27, 30 and 33 qubits,
     // complex128, and slower at 24 qubits, where much of the state stays in
@@ -489,7 +490,12 @@ PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const
     // amplitudes per thread), which win from 23 qubits on (27: 21.6 ms against
     // 22.4).  Up to 12 qubits (reverse sweeps 11) the whole state is one tile, so
     // a plan is one pass (12 qubits: 96 us against 104 in passes of 11).
-    if (!chosen && (!given || n < k + 6) && n <= (adjoint ? 24 : 20)) {
+    if (!chosen && pp.fp32) {
+        if (n < k + 6) {
+            tlog = 6;
+            k = 10;
+        }
+    } else if (!chosen && (!given || n < k + 6) && n <= (adjoint ? 24 : 20)) {
         k = adjoint || (n > 12 && n < 20) ? std::min(n, 11) : std::min(n, 12);
         tlog = k <= 9 ? 6 : (k == 12 ? 9 : 8);
     }
@@ -503,7 +509,7 @@ PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const
     pp.gen_auto = gen_set ? 0 : 1;
     pp.nontemporal = nt != 0 ? 1 : 0;
     // forward passes split their transposes where the shape has half-LDS kernels
-    pp.half_lds = !adjoint && tune_value("half_lds", 1) != 0 && tile_half_exists(dtype, pp.rlog, pp.tlog) ? 1 : 0;
+    pp.half_lds = !adjoint && tune_value("half_lds", 1) != 0 && tile_half_exists(pp.fp32 != 0, pp.rlog, pp.tlog) ? 1 : 0;
     return pp;
 }
 
@@ -553,10 +559,10 @@ static int upload_ops(DevicePlan &dp, const std::vector<DevOp> &ops)
 }
 
 int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoint, const std::vector<HostOp> &ops,
-                 StateLayout layout, const TuneChoice *pin)
+                 StateLayout layout, const TuneChoice *pin, bool inner)
 {
-    const bool small = n <= kSmallMaxQubits;
-    PlanParams pp = small ? PlanParams{} : tile_params(n, dtype, adjoint, layout, pin);
+    const bool small = n <= small_qubits(dtype, adjoint || inner);
+    PlanParams pp = small ? PlanParams{} : tile_params(n, dtype, adjoint, layout, pin, inner);
     const bool same_shape = dp.valid && dp.dtype == dtype && dp.small == small &&
                             (small || (dp.pp.k == pp.k && dp.pp.tlog == pp.tlog && dp.pp.max_gen_per_pass == pp.max_gen_per_pass &&
                                        dp.pp.gen_auto == pp.gen_auto &&
@@ -567,7 +573,7 @@ int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoin
     std::vector<HostOp> merged = merge_ops(ops);
     if (!small && same_shape && dp.epoch == tune_epoch() && same_structure(dp.source, merged)) {
         // the same gates at other angles: passes and phases stay, the ops get new matrices
-        refresh_ops(merged, dp.plan.op_src, &dp.plan.ops);
+        refresh_ops(merged, pp.fp32 != 0, dp.plan.op_src, &dp.plan.ops);
         DMV_TRY(upload_ops(dp, dp.plan.ops));
         dp.version = version;
         return DMV_OK;
@@ -586,7 +592,7 @@ int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoin
         std::shared_ptr<const Plan> plan;
         DMV_TRY(shared_plan(merged, pp, &plan));
         dp.plan = *plan;
-        refresh_ops(merged, dp.plan.op_src, &dp.plan.ops);
+        refresh_ops(merged, pp.fp32 != 0, dp.plan.op_src, &dp.plan.ops);
         dp.source = std::move(merged);
         DMV_TRY(upload(dp.d_passes, dp.cap_passes, dp.plan.passes));
         DMV_TRY(upload(dp.d_phases, dp.cap_phases, dp.plan.phases));
@@ -796,7 +802,7 @@ static int forward_passes(DevicePlan &dp, dmv_state *s)
     const bool nt = dp.pp.nontemporal != 0;
     for (uint32_t p = 0; p < dp.plan.passes.size(); p++) {
         prof_begin(DMV_KC_TILE);
-        DMV_TRY(launch_tile(s->dtype, dp.pp.rlog, dp.pp.tlog, nt, dp.plan.passes[p].lds_half != 0, s->amp, s->n,
+        DMV_TRY(launch_tile(s->dtype, dp.pp.fp32 != 0, dp.pp.rlog, dp.pp.tlog, nt, dp.plan.passes[p].lds_half != 0, s->amp, s->n,
                             s->layout, dp.d_passes, dp.d_phases, dp.d_ops, p));
         prof_end(DMV_KC_TILE, 2.0 * (double)s->bytes);
     }
@@ -885,6 +891,14 @@ int circuit_forward(dmv_circuit *c, dmv_state *s, int mode)
 }
 
 int run_forward_plan(DevicePlan &dp, dmv_state *s) { return forward_passes(dp, s); }
+
+int circuit_inner_forward(dmv_circuit *c, dmv_state *s)
+{
+    if (s->dtype != DMV_C64)
+        return circuit_forward(c, s, DMV_FORWARD_FUSED);
+    DMV_TRY(prepare_plan(c->inner, c->version, c->n, s->dtype, false, forward_ops(c->gates), s->layout, nullptr, true));
+    return forward_passes(c->inner, s);
+}
 
 // -------------------------------------------------------- profiling access --
 int profile_enable(int on)

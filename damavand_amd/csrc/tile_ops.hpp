@@ -336,6 +336,18 @@ __device__ __forceinline__ void oop_su2_m(V (&out)[NR], const V (&in)[NR], const
     }
 }
 
+template <int M, class V, class R, int NR>
+__device__ __forceinline__ void oop_gen_plain_m(V (&out)[NR], const V (&in)[NR], const Mat<R> &A)
+{
+    constexpr int HB = highest_bit(M);
+#pragma unroll
+    for (int p = 0; p < NR; p++) {
+        if (p & HB)
+            continue;
+        apply2_to(out[p], out[p ^ M], in[p], in[p ^ M], A);
+    }
+}
+
 // A GEN whose pair members are swapped where fl says so (GENs carry no
 // controls, so every pair of every lane takes it).
 template <int M, class V, class R, int NR>
@@ -414,12 +426,24 @@ __device__ __forceinline__ void oop_op(V (&out)[NR], const V (&in)[NR], const De
     const uint32_t m = op->rmask < (uint32_t)NR ? op->rmask : 1u;
     if (op->kind == OP_DIAG) {
         oop_diag<V, R>(out, in, op, tid, hold);
-    } else if (op->kind == OP_GEN && op->aux) {
+    } else if (sizeof(R) == 4 && op->plain) {
+        const Mat<R> A = load_mat<R>(op->m);
+        switch (m) {
+#define DMV_OOP_PLAIN_CASE(M)                                                                      \
+    case M:                                                                                        \
+        if constexpr (M < NR && sizeof(R) == 4)                                                    \
+            oop_gen_plain_m<M>(out, in, A);                                                        \
+        break;
+            DMV_MASK_CASES_FROM2(DMV_OOP_PLAIN_CASE)
+#undef DMV_OOP_PLAIN_CASE
+        default: oop_gen_plain_m<1>(out, in, A); break;
+        }
+    } else if (sizeof(R) == 8 && op->kind == OP_GEN && op->aux) {
         const Su2<R> S = load_su2<R>(op->m);
         switch (m) {
 #define DMV_OOP_SU2_CASE(M)                                                                        \
     case M:                                                                                        \
-        if constexpr (M < NR)                                                                      \
+        if constexpr (M < NR && sizeof(R) == 8)                                                    \
             oop_su2_m<M>(out, in, S, fl);                                                          \
         break;
             DMV_MASK_CASES_FROM2(DMV_OOP_SU2_CASE)
@@ -553,11 +577,14 @@ __device__ __forceinline__ void process_tile(typename Cplx<R>::T (&v)[1 << RLOG]
 }
 
 // One tile of a forward pass: load, run the phases, store.  S: the state's
-// real type, R: the type it is computed in.  complex64 states are computed in
-// FP64: without packed FP32 instructions an FP32 operation takes a vector
-// instruction as an FP64 one does, so this costs registers and LDS only (16
+// real type, R: the type it is computed in.  complex64 gradients and batches are
+// computed in FP64: without packed FP32 instructions an FP32 operation takes a
+// vector instruction as an FP64 one does, so this costs registers and LDS only (16
 // amplitudes per thread instead of 32), a pass then rounds each amplitude once,
-// at its store, and the matrices are not rounded at all.
+// at its store, and the matrices are not rounded at all (energy of 21 qubits,
+// 4 layers: error 2e-7 -> 4e-8).  A complex64 forward whose state the caller gets
+// is computed in FP32, gates in order: which basis state a sample falls on
+// hangs on the last bits, and those stay what they are.
 template <class S, class R, int RLOG, int TLOG, bool NT, bool HALF = false>
 __device__ __forceinline__ void tile_body(typename Cplx<S>::T *__restrict__ state, const DevPass *P,
                                           const DevPhase *__restrict__ phases, const DevOp *__restrict__ ops,

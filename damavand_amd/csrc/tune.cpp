@@ -236,7 +236,7 @@ int autotune_forward(dmv_circuit *c, dmv_state *s, int *chosen)
 {
     DMV_CHECK_ARG(c->n == s->n, "circuit has %d qubits but the state has %d", c->n, s->n);
     DMV_TRY(ensure_device());
-    if (s->n <= kSmallMaxQubits) {  // one whole-state launch: nothing to choose
+    if (s->n <= small_qubits(s->dtype, false)) {  // one whole-state launch: nothing to choose
         if (chosen)
             *chosen = s->n;
         return DMV_OK;
