@@ -7,9 +7,14 @@
 namespace dmv {
 
 // HALF: half a tile of LDS (split transposes), so that three workgroups of
-// the 64 KiB tiles share a CU instead of two.
+// the 64 KiB tiles share a CU instead of two.  The FP32 kernel of 32 amplitudes
+// a thread took 187 registers, two waves a SIMD; with scalar matrices (op_bits) and
+// thread bits made anew (tid_again) it takes 163 and runs three.  complex64, 27
+// qubits, 10 ansatz layers: 18.6 -> 16.0 ms; 28 qubits, 4 layers of H, RX, RY, RZ and
+// CNOT: 15.1 -> 12.9 ms.  (Held to 168 registers without tid_again it spilled 14, and
+// the ansatz took 21.0 ms.)
 template <class S, class R, int RLOG, int TLOG, bool NT, bool HALF>
-__global__ void __launch_bounds__(1 << TLOG)
+__global__ void __launch_bounds__(1 << TLOG, sizeof(R) == 4 && RLOG == 5 && HALF ? 3 : 1)
 k_tile(typename Cplx<S>::T *__restrict__ state, const DevPass *__restrict__ passes,
        const DevPhase *__restrict__ phases, const DevOp *__restrict__ ops, uint32_t pass_idx, uint32_t xcd_log2,
        StateLayout L)

@@ -551,9 +551,20 @@ template <class T> static int upload(T *&dptr, size_t &cap, const std::vector<T>
     return copy_h2d(dptr, v.data(), v.size() * sizeof(T));
 }
 
-// A plan's ops, which change with every set of angles: not waited for.
-static int upload_ops(DevicePlan &dp, const std::vector<DevOp> &ops)
+// A plan's ops, which change with every set of angles: not waited for.  fp32:
+// the matrices as op_mat<float> reads them.
+static int upload_ops(DevicePlan &dp, const std::vector<DevOp> &given, bool fp32)
 {
+    std::vector<DevOp> rounded;
+    if (fp32) {
+        rounded = given;
+        for (DevOp &op : rounded)
+            for (int i = 0; i < 4; i++) {
+                const float pair[2] = {(float)op.m[2 * i], (float)op.m[2 * i + 1]};
+                std::memcpy(&op.m[i], pair, sizeof(pair));
+            }
+    }
+    const std::vector<DevOp> &ops = fp32 ? rounded : given;
     DMV_TRY(room(dp.d_ops, dp.cap_ops, ops.size()));
     return pinned_h2d(dp.pin_ops, dp.d_ops, ops.data(), ops.size() * sizeof(DevOp));
 }
@@ -574,7 +585,7 @@ int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoin
     if (!small && same_shape && dp.epoch == tune_epoch() && same_structure(dp.source, merged)) {
         // the same gates at other angles: passes and phases stay, the ops get new matrices
         refresh_ops(merged, pp.fp32 != 0, dp.plan.op_src, &dp.plan.ops);
-        DMV_TRY(upload_ops(dp, dp.plan.ops));
+        DMV_TRY(upload_ops(dp, dp.plan.ops, pp.fp32 != 0));
         dp.version = version;
         return DMV_OK;
     }
@@ -587,7 +598,7 @@ int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoin
         for (const DevOp &o : dp.small_ops)
             if (o.slot + 1 > dp.plan.n_slots)
                 dp.plan.n_slots = o.slot + 1;
-        DMV_TRY(upload_ops(dp, dp.small_ops));
+        DMV_TRY(upload_ops(dp, dp.small_ops, false));
     } else {
         std::shared_ptr<const Plan> plan;
         DMV_TRY(shared_plan(merged, pp, &plan));
@@ -596,7 +607,7 @@ int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoin
         dp.source = std::move(merged);
         DMV_TRY(upload(dp.d_passes, dp.cap_passes, dp.plan.passes));
         DMV_TRY(upload(dp.d_phases, dp.cap_phases, dp.plan.phases));
-        DMV_TRY(upload_ops(dp, dp.plan.ops));
+        DMV_TRY(upload_ops(dp, dp.plan.ops, pp.fp32 != 0));
         if (!dp.plan.ip_slots.empty())
             DMV_TRY(upload(dp.d_ip_slots, dp.cap_ip, dp.plan.ip_slots));
     }

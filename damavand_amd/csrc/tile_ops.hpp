@@ -17,6 +17,16 @@
 
 namespace dmv {
 
+// tid for one use.  The compiler keeps the bits of tid that offsets are made
+// of, 14 registers, from one transpose to the next; the FP32 kernels have none to
+// spare (see k_tile) and make them again.
+template <class R> __device__ __forceinline__ uint32_t tid_again(uint32_t tid)
+{
+    if constexpr (sizeof(R) == 4)
+        asm volatile("" : "+v"(tid));
+    return tid;
+}
+
 template <int TLOG> __device__ __forceinline__ uint32_t thread_local_offset(const DevLayout *L, uint32_t tid)
 {
     uint32_t o = 0;
@@ -291,6 +301,12 @@ __device__ __forceinline__ void apply2_to(V &oa, V &ob, const V &a, const V &b, 
     ob.y = M.m10r * a.y + M.m10i * a.x + M.m11r * b.y + M.m11i * b.x;
 }
 
+__device__ __forceinline__ void unpack(uint64_t pair, float &re, float &im)
+{
+    re = __int_as_float((int)(uint32_t)pair);
+    im = __int_as_float((int)(uint32_t)(pair >> 32));
+}
+
 template <class V, int NR> __device__ __forceinline__ void copy_regs(V (&out)[NR], const V (&in)[NR])
 {
 #pragma unroll
@@ -348,23 +364,71 @@ __device__ __forceinline__ void oop_gen_plain_m(V (&out)[NR], const V (&in)[NR],
     }
 }
 
+// Rows and columns of A change places where bit p of fl is set.
+template <int P> __device__ __forceinline__ Mat<double> flip_mat(const Mat<double> &A, uint32_t fl)
+{
+    const bool f = (fl >> P) & 1u;
+    Mat<double> B;
+    B.m00r = f ? A.m11r : A.m00r; B.m00i = f ? A.m11i : A.m00i;
+    B.m01r = f ? A.m10r : A.m01r; B.m01i = f ? A.m10i : A.m01i;
+    B.m10r = f ? A.m01r : A.m10r; B.m10i = f ? A.m01i : A.m10i;
+    B.m11r = f ? A.m00r : A.m11r; B.m11i = f ? A.m00i : A.m11i;
+    return B;
+}
+
+// FP32: as masks on whole (re, im) pairs, seven scalar instructions; choices
+// between floats are not kept scalar and became eight v_cndmask beside the pair's
+// sixteen FMAs.
+struct MatBits {
+    uint64_t m00, m01, m10, m11;
+};
+
+__device__ __forceinline__ MatBits mat_bits(const double *m)
+{
+    return MatBits{(uint64_t)__double_as_longlong(m[0]), (uint64_t)__double_as_longlong(m[1]),
+                   (uint64_t)__double_as_longlong(m[2]), (uint64_t)__double_as_longlong(m[3])};
+}
+
+template <int P> __device__ __forceinline__ Mat<float> flip_mat(const MatBits &A, uint32_t fl)
+{
+    const uint64_t mask = (uint64_t)(int64_t)((int32_t)(fl << (31 - P)) >> 31);
+    const uint64_t d = (A.m00 ^ A.m11) & mask, o = (A.m01 ^ A.m10) & mask;
+    Mat<float> B;
+    unpack(A.m00 ^ d, B.m00r, B.m00i);
+    unpack(A.m01 ^ o, B.m01r, B.m01i);
+    unpack(A.m10 ^ o, B.m10r, B.m10i);
+    unpack(A.m11 ^ d, B.m11r, B.m11i);
+    return B;
+}
+
+// An op's matrix.  The ops of FP32 plans come with rounded entries, as four
+// (re, im) pairs of floats in m[0..3]: no scalar instruction converts, so entries
+// rounded here would be in vector registers.
+template <class R> __device__ __forceinline__ auto op_bits(const double *m)
+{
+    if constexpr (sizeof(R) == 4)
+        return mat_bits(m);
+    else
+        return load_mat<R>(m);
+}
+
+template <class R> __device__ __forceinline__ Mat<R> op_mat(const double *m)
+{
+    if constexpr (sizeof(R) == 4)
+        return flip_mat<0>(mat_bits(m), 0);
+    else
+        return load_mat<R>(m);
+}
+
 // A GEN whose pair members are swapped where fl says so (GENs carry no
 // controls, so every pair of every lane takes it).
-template <int M, class V, class R, int NR>
-__device__ __forceinline__ void oop_gen_m(V (&out)[NR], const V (&in)[NR], const Mat<R> &A, uint32_t fl)
+template <int M, class V, class A, int NR, int P = 0>
+__device__ __forceinline__ void oop_gen_m(V (&out)[NR], const V (&in)[NR], const A &m, uint32_t fl)
 {
-    constexpr int HB = highest_bit(M);
-#pragma unroll
-    for (int p = 0; p < NR; p++) {
-        if (p & HB)
-            continue;
-        const bool f = (fl >> p) & 1u;
-        Mat<R> B;
-        B.m00r = f ? A.m11r : A.m00r; B.m00i = f ? A.m11i : A.m00i;
-        B.m01r = f ? A.m10r : A.m01r; B.m01i = f ? A.m10i : A.m01i;
-        B.m10r = f ? A.m01r : A.m10r; B.m10i = f ? A.m01i : A.m10i;
-        B.m11r = f ? A.m00r : A.m11r; B.m11i = f ? A.m00i : A.m11i;
-        apply2_to(out[p], out[p ^ M], in[p], in[p ^ M], B);
+    if constexpr (P < NR) {
+        if constexpr (!(P & highest_bit(M)))
+            apply2_to(out[P], out[P ^ M], in[P], in[P ^ M], flip_mat<P>(m, fl));
+        oop_gen_m<M, V, A, NR, P + 1>(out, in, m, fl);
     }
 }
 
@@ -392,7 +456,8 @@ __device__ __forceinline__ void oop_diag(V (&out)[NR], const V (&in)[NR], const 
             out[r] = flip_sign(in[r], flip_mask<NR>(op, r, lane));
         return;
     }
-    const R d0r = (R)op->m[0], d0i = (R)op->m[1], d1r = (R)op->m[6], d1i = (R)op->m[7];
+    const Mat<R> A = op_mat<R>(op->m);
+    const R d0r = A.m00r, d0i = A.m00i, d1r = A.m11r, d1i = A.m11i;
     const uint32_t en = op->en;
     const uint32_t all = NR >= 32 ? 0xFFFFFFFFu : ((1u << NR) - 1);
     if (op->tbit == kNoReg) {
@@ -427,7 +492,7 @@ __device__ __forceinline__ void oop_op(V (&out)[NR], const V (&in)[NR], const De
     if (op->kind == OP_DIAG) {
         oop_diag<V, R>(out, in, op, tid, hold);
     } else if (sizeof(R) == 4 && op->plain) {
-        const Mat<R> A = load_mat<R>(op->m);
+        const Mat<R> A = op_mat<R>(op->m);
         switch (m) {
 #define DMV_OOP_PLAIN_CASE(M)                                                                      \
     case M:                                                                                        \
@@ -451,7 +516,7 @@ __device__ __forceinline__ void oop_op(V (&out)[NR], const V (&in)[NR], const De
         default: oop_su2_m<1>(out, in, S, fl); break;
         }
     } else if (op->kind == OP_GEN) {
-        const Mat<R> A = load_mat<R>(op->m);
+        const auto A = op_bits<R>(op->m);
         switch (m) {
 #define DMV_OOP_GEN_CASE(M)                                                                        \
     case M:                                                                                        \
@@ -561,18 +626,18 @@ __device__ __forceinline__ void process_tile(typename Cplx<R>::T (&v)[1 << RLOG]
         const DevPhase *D = phases + ph;
         if (D->transpose_in) {
             if constexpr (HALF)
-                transpose_half<V, ST, NR, TLOG>(v, lds, cur, D->src_lswz, &D->lay, D->dst_lswz, P->split, tid);
+                transpose_half<V, ST, NR, TLOG>(v, lds, cur, D->src_lswz, &D->lay, D->dst_lswz, P->split, tid_again<R>(tid));
             else
-                transpose<V, ST, NR, TLOG>(v, lds, cur, D->src_lswz, &D->lay, D->dst_lswz, tid);
+                transpose<V, ST, NR, TLOG>(v, lds, cur, D->src_lswz, &D->lay, D->dst_lswz, tid_again<R>(tid));
         }
         cur = &D->lay;
         run_ops<V, R, RLOG>(v, ops, D->op_begin, D->op_end, tid);
     }
     if (P->transpose_st) {
         if constexpr (HALF)
-            transpose_half<V, ST, NR, TLOG>(v, lds, cur, P->st_src_lswz, &P->lay_st, P->st_dst_lswz, P->split, tid);
+            transpose_half<V, ST, NR, TLOG>(v, lds, cur, P->st_src_lswz, &P->lay_st, P->st_dst_lswz, P->split, tid_again<R>(tid));
         else
-            transpose<V, ST, NR, TLOG>(v, lds, cur, P->st_src_lswz, &P->lay_st, P->st_dst_lswz, tid);
+            transpose<V, ST, NR, TLOG>(v, lds, cur, P->st_src_lswz, &P->lay_st, P->st_dst_lswz, tid_again<R>(tid));
     }
 }
 
@@ -595,9 +660,9 @@ __device__ __forceinline__ void tile_body(typename Cplx<S>::T *__restrict__ stat
     const uint32_t tid = threadIdx.x;
     const uint64_t g = tile_base<K>(P, tile);
     V v[NR];
-    load_tile<NT>(v, state, g | thread_global_offset<TLOG>(P->gthr_ld, tid), P->greg_ld, L);
+    load_tile<NT>(v, state, g | thread_global_offset<TLOG>(P->gthr_ld, tid_again<R>(tid)), P->greg_ld, L);
     process_tile<S, R, RLOG, TLOG, HALF>(v, P, phases, ops, lds);
-    store_tile<NT>(v, state, g | thread_global_offset<TLOG>(P->gthr_st, tid), P->greg_st, L);
+    store_tile<NT>(v, state, g | thread_global_offset<TLOG>(P->gthr_st, tid_again<R>(tid)), P->greg_st, L);
 }
 
 // --------------------------------------------------------------- adjoint --

@@ -1,0 +1,77 @@
+"""The plans the library makes by itself (searched passes, special-unitary gates
+with their global phase, shapes by size, complex64 forwards in gate order),
+emulated on the CPU against the oracle."""
+import math
+
+import numpy as np
+import pytest
+
+import oracle
+from damavand_amd import _native as N
+from damavand_amd import workloads as wl
+from tests.libhelpers import NativeCircuit
+from tests.test_tile_emulation import random_gates, zero_state
+from tests.tile_emulator import TileEmulator, plan_json
+
+
+@pytest.mark.parametrize("dtype,elem", [(N.C128, 16), (N.C64, 8)])
+@pytest.mark.parametrize("n,count,seed", [(9, 60, 1), (10, 200, 2), (12, 250, 3), (13, 250, 4), (16, 300, 5), (18, 150, 6),
+                                          (19, 120, 7), (20, 120, 8)])
+def test_default_forward_plan(n, count, seed, dtype, elem):
+    """Amplitudes, not only probabilities: the phases taken out of the gates come back."""
+    if dtype == N.C64 and n <= 13:
+        pytest.skip("a whole-state kernel's size")
+    gates = random_gates(np.random.default_rng(seed), n, count)
+    nc = NativeCircuit(n, gates)
+    plan = plan_json(nc.h, dtype=dtype)
+    got = TileEmulator(plan, elem=elem).forward(zero_state(n))
+    np.testing.assert_allclose(got, oracle.run_gates(n, gates).amp, atol=1e-12)
+
+
+@pytest.mark.parametrize("kind,params", [(wl.GATE_H, ()), (wl.GATE_Y, ()), (wl.GATE_U3, (0.3, 2.1, 5.0)),
+                                         (wl.GATE_U3, (math.pi, 0.0, 0.0)), (wl.GATE_T, ()), (wl.GATE_RX, (0.0,))])
+def test_global_phase_of_one_gate(kind, params):
+    """One gate of determinant other than 1 on each qubit, so that the phase has to be kept by another gate's op, or by its own."""
+    n = 13
+    for last in (0, n - 1):
+        gates = [(kind, -1, q, params) for q in range(n)] + [(wl.GATE_RY, -1, last, (0.4,))]
+        nc = NativeCircuit(n, gates)
+        got = TileEmulator(plan_json(nc.h)).forward(zero_state(n))
+        np.testing.assert_allclose(got, oracle.run_gates(n, gates).amp, atol=1e-13)
+
+
+def test_complex64_forward_keeps_gate_order():
+    """The general matrices, in the order of the gates: what a program samples depends on a state's last bits."""
+    n = 17
+    gates = random_gates(np.random.default_rng(11), n, 200)
+    nc = NativeCircuit(n, gates)
+    auto = plan_json(nc.h, dtype=N.C64)
+    m = np.array([op["m"] for P in auto["passes"] for ph in P["phases"] for op in ph["ops"] if op["kind"] == 0])
+    m = m[:, ::2] + 1j * m[:, 1::2]
+    assert (np.abs(m[:, 0] * m[:, 3] - m[:, 1] * m[:, 2] - 1.0) > 0.1).sum() > len(m) // 4  # determinants are kept
+    given = [plan_json(nc.h, dtype=N.C64, tile_qubits=auto["k"], tlog=auto["tlog"], max_gen=g) for g in (8, 12)]
+    assert auto["passes"] in [g["passes"] for g in given]
+
+
+@pytest.mark.parametrize("n,layers", [(9, 1), (11, 1), (12, 1), (13, 1), (15, 1)])
+def test_default_reverse_plan(n, layers):
+    """The reverse sweep by itself: psi back to |0>, gradients against parameter shift."""
+    gates, a, b = wl.ansatz_circuit(n, layers, 900 + n)
+    gates = [(wl.GATE_H, -1, 0, ()), (wl.GATE_U3, -1, n - 1, (0.2, 0.7, 1.9))] + gates + [(wl.GATE_T, -1, n // 2, ())]
+    pairs = wl.chain_pairs(n)
+    nc = NativeCircuit(n, gates)
+    st = oracle.run_gates(n, gates)
+    idx = np.arange(1 << n)
+    h = sum(c * (1.0 - 2.0 * ((idx >> q) & 1)) for q, c in enumerate(a))
+    h = h + sum(c * (1.0 - 2.0 * (((idx >> i) ^ (idx >> j)) & 1)) for (i, j), c in zip(pairs, b))
+    psi0, _, grads = TileEmulator(plan_json(nc.h, adjoint=True)).reverse(st.amp, h * st.amp)
+    # up to a global phase, which no gradient sees
+    assert abs(abs(psi0[0]) - 1.0) <= 1e-12 and np.abs(psi0[1:]).max() <= 1e-12
+    ref = []
+    for gi in [i for i, g in enumerate(gates) if g[0] in wl.PARAMETRIC]:
+        vals = []
+        for s in (0.5 * math.pi, -0.5 * math.pi):
+            kk, c, t, p = gates[gi]
+            vals.append(oracle.run_gates(n, gates[:gi] + [(kk, c, t, (p[0] + s,))] + gates[gi + 1:]).expect_zz(a, pairs, b))
+        ref.append(0.5 * (vals[0] - vals[1]))
+    np.testing.assert_allclose(grads, ref, atol=1e-10)
