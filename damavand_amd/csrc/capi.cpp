@@ -130,7 +130,7 @@ int dmv::circuit_adjoint(dmv_circuit *c, dmv_state *psi, dmv_state *lam, const O
     dmv_circuit_num_parameters(c, &np);
     // psi = U|0>
     DMV_TRY(state_reset(psi, 0, false));
-    DMV_TRY(circuit_inner_forward(c, psi));
+    DMV_TRY(circuit_forward(c, psi, DMV_FORWARD_FUSED));
     if ((uint64_t)np + 1 > c->cap_grad) {
         release(c->d_grad);
         c->d_grad = nullptr;
@@ -554,10 +554,9 @@ int dmv_circuit_destroy(dmv_circuit *c)
 {
     if (!c)
         return DMV_OK;
-    if (c->fwd.valid || c->adj.valid || c->inner.valid || c->d_partials || c->d_terms || c->d_grad) {
+    if (c->fwd.valid || c->adj.valid || c->d_partials || c->d_terms || c->d_grad) {
         free_plan(c->fwd);
         free_plan(c->adj);
-        free_plan(c->inner);
         release(c->d_partials);
         release(c->d_terms);
         release(c->d_grad);
@@ -809,7 +808,7 @@ int dmv_circuit_plan_json(dmv_circuit *c, int dtype, int adjoint, int tile_qubit
         pp.k = tile_qubits;
         pp.tlog = threads_log2 > 0 ? threads_log2 : (tile_qubits >= 10 ? 8 : 6);
         pp.rlog = pp.k - pp.tlog;
-        pp.half_lds = !adjoint && tune_value("half_lds", 1) != 0 && tile_half_exists(pp.fp32 != 0, pp.rlog, pp.tlog) ? 1 : 0;
+        pp.half_lds = !adjoint && tune_value("half_lds", 1) != 0 && tile_half_exists(dtype, pp.rlog, pp.tlog) ? 1 : 0;
     }
     if (max_gen_per_pass > 0) {
         pp.max_gen_per_pass = max_gen_per_pass;

@@ -12,16 +12,16 @@
 
 namespace dmv {
 
-bool tile_half_exists(bool fp32, int rlog, int tlog)
+bool tile_half_exists(int dtype, int rlog, int tlog)
 {
-    return tlog == 8 && rlog == (fp32 ? 5 : 4);
+    return tlog == 8 && rlog == (dtype == DMV_C64 ? 5 : 4);
 }
 
-int launch_tile(int dtype, bool fp32, int rlog, int tlog, bool nt, bool half, void *state, int n, StateLayout L,
+int launch_tile(int dtype, int rlog, int tlog, bool nt, bool half, void *state, int n, StateLayout L,
                 const DevPass *passes, const DevPhase *phases, const DevOp *ops, uint32_t pass_idx)
 {
     DMV_CHECK_ARG(n >= rlog + tlog && n - (rlog + tlog) <= 31, "tile shape does not fit %d qubits", n);
-    DMV_CHECK_ARG(!half || tile_half_exists(fp32, rlog, tlog), "no half-LDS tile kernel for rlog %d tlog %d", rlog,
+    DMV_CHECK_ARG(!half || tile_half_exists(dtype, rlog, tlog), "no half-LDS tile kernel for rlog %d tlog %d", rlog,
                   tlog);
     int rc = kNotHandled;
     if (dtype == DMV_C128) {
@@ -29,8 +29,7 @@ int launch_tile(int dtype, bool fp32, int rlog, int tlog, bool nt, bool half, vo
         if (rc == kNotHandled && !half)
             rc = launch_tile_c128_other(rlog, tlog, nt, state, n, L, passes, phases, ops, pass_idx);
     } else {
-        rc = fp32 ? launch_tile_c64_fp32(rlog, tlog, nt, half, state, n, L, passes, phases, ops, pass_idx)
-                  : launch_tile_c64(rlog, tlog, nt, half, state, n, L, passes, phases, ops, pass_idx);
+        rc = launch_tile_c64(rlog, tlog, nt, half, state, n, L, passes, phases, ops, pass_idx);
     }
     if (rc != kNotHandled)
         return rc;

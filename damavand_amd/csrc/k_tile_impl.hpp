@@ -62,7 +62,4 @@ int launch_tile_c128_wave32(int rlog, int tlog, bool nt, void *state, int n, Sta
 int launch_tile_c64(int rlog, int tlog, bool nt, bool half, void *state, int n, StateLayout L, const DevPass *passes,
                     const DevPhase *phases, const DevOp *ops, uint32_t pass_idx);
 
-int launch_tile_c64_fp32(int rlog, int tlog, bool nt, bool half, void *state, int n, StateLayout L,
-                         const DevPass *passes, const DevPhase *phases, const DevOp *ops, uint32_t pass_idx);
-
 }  // namespace dmv

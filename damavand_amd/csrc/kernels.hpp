@@ -11,11 +11,10 @@ namespace dmv {
 // One fused pass of a tile plan over a state of n qubits in layout L (every
 // state launcher below takes the state's layout L).  half: the kernel with
 // half a tile of LDS, for passes whose transposes are all split.
-// fp32: a complex64 state computed in FP32 (PlanParams::fp32).
-int launch_tile(int dtype, bool fp32, int rlog, int tlog, bool nontemporal, bool half, void *state, int n, StateLayout L,
+int launch_tile(int dtype, int rlog, int tlog, bool nontemporal, bool half, void *state, int n, StateLayout L,
                 const DevPass *passes, const DevPhase *phases, const DevOp *ops, uint32_t pass_idx);
 // Whether a half-LDS tile kernel exists for the shape.
-bool tile_half_exists(bool fp32, int rlog, int tlog);
+bool tile_half_exists(int dtype, int rlog, int tlog);
 // Reverse-sweep tile pass over psi and lambda; the IP ops of the pass write
 // one partial per (IP op, tile, wave) into
 // partials[(ip_pos * tiles + tile) * waves + wave].

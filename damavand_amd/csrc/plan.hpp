@@ -64,9 +64,9 @@ struct PlanParams {
     int nontemporal = 0;   // forward passes: streaming (nontemporal) loads and stores
     int half_lds = 0;      // forward passes: split transposes where a pass allows (half-LDS kernels exist)
     int max_ip_per_pass = 1 << 30;  // IP ops of a pass (a run of IP ops on one qubit stays together)
-    // complex64 forward plans (Circuit forward): FP32 arithmetic, general
-    // matrices and ops in order.  What a program samples from a complex64 state is
-    // decided by its last bits, so these states keep theirs.
+    // complex64 forward plans: FP32 arithmetic, general matrices and ops in order.
+    // What a program samples from a complex64 state, and an energy whose terms
+    // cancel, are decided by its last bits, so these states keep theirs.
     int fp32 = 0;
     int gen_auto = 0;      // build_plan chooses the passes by cost instead (max_gen_per_pass is not used)
     StateLayout layout = kPlainLayout;  // element map of the states the plan runs on

@@ -424,10 +424,10 @@ bool gate_nontemporal(uint32_t target, int dtype)
 }
 
 // ------------------------------------------------------------------- plans --
-PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const TuneChoice *pin, bool inner)
+PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const TuneChoice *pin)
 {
     PlanParams pp;
-    pp.fp32 = dtype == DMV_C64 && !adjoint && !inner ? 1 : 0;
+    pp.fp32 = dtype == DMV_C64 && !adjoint ? 1 : 0;
     pp.n = n;
     pp.layout = layout;
     pp.low_bits = coalesce_bits(dtype);
@@ -509,7 +509,7 @@ PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const
     pp.gen_auto = gen_set ? 0 : 1;
     pp.nontemporal = nt != 0 ? 1 : 0;
     // forward passes split their transposes where the shape has half-LDS kernels
-    pp.half_lds = !adjoint && tune_value("half_lds", 1) != 0 && tile_half_exists(pp.fp32 != 0, pp.rlog, pp.tlog) ? 1 : 0;
+    pp.half_lds = !adjoint && tune_value("half_lds", 1) != 0 && tile_half_exists(dtype, pp.rlog, pp.tlog) ? 1 : 0;
     return pp;
 }
 
@@ -570,10 +570,10 @@ static int upload_ops(DevicePlan &dp, const std::vector<DevOp> &given, bool fp32
 }
 
 int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoint, const std::vector<HostOp> &ops,
-                 StateLayout layout, const TuneChoice *pin, bool inner)
+                 StateLayout layout, const TuneChoice *pin)
 {
-    const bool small = n <= small_qubits(dtype, adjoint || inner);
-    PlanParams pp = small ? PlanParams{} : tile_params(n, dtype, adjoint, layout, pin, inner);
+    const bool small = n <= small_qubits(dtype, adjoint);
+    PlanParams pp = small ? PlanParams{} : tile_params(n, dtype, adjoint, layout, pin);
     const bool same_shape = dp.valid && dp.dtype == dtype && dp.small == small &&
                             (small || (dp.pp.k == pp.k && dp.pp.tlog == pp.tlog && dp.pp.max_gen_per_pass == pp.max_gen_per_pass &&
                                        dp.pp.gen_auto == pp.gen_auto &&
@@ -813,7 +813,7 @@ static int forward_passes(DevicePlan &dp, dmv_state *s)
     const bool nt = dp.pp.nontemporal != 0;
     for (uint32_t p = 0; p < dp.plan.passes.size(); p++) {
         prof_begin(DMV_KC_TILE);
-        DMV_TRY(launch_tile(s->dtype, dp.pp.fp32 != 0, dp.pp.rlog, dp.pp.tlog, nt, dp.plan.passes[p].lds_half != 0, s->amp, s->n,
+        DMV_TRY(launch_tile(s->dtype, dp.pp.rlog, dp.pp.tlog, nt, dp.plan.passes[p].lds_half != 0, s->amp, s->n,
                             s->layout, dp.d_passes, dp.d_phases, dp.d_ops, p));
         prof_end(DMV_KC_TILE, 2.0 * (double)s->bytes);
     }
@@ -902,14 +902,6 @@ int circuit_forward(dmv_circuit *c, dmv_state *s, int mode)
 }
 
 int run_forward_plan(DevicePlan &dp, dmv_state *s) { return forward_passes(dp, s); }
-
-int circuit_inner_forward(dmv_circuit *c, dmv_state *s)
-{
-    if (s->dtype != DMV_C64)
-        return circuit_forward(c, s, DMV_FORWARD_FUSED);
-    DMV_TRY(prepare_plan(c->inner, c->version, c->n, s->dtype, false, forward_ops(c->gates), s->layout, nullptr, true));
-    return forward_passes(c->inner, s);
-}
 
 // -------------------------------------------------------- profiling access --
 int profile_enable(int on)

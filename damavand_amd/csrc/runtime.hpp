@@ -99,7 +99,6 @@ struct dmv_circuit {
     std::vector<dmv::Gate> gates;
     uint64_t version = 0;
     dmv::DevicePlan fwd, adj;
-    dmv::DevicePlan inner;          // complex64: the forward of a gradient
     dmv::TuneChoice tune_fwd, tune_adj;  // set by the autotuner for this gate list
     double *d_partials = nullptr;   // adjoint partials of one pass: per (IP op, tile, wave)
     uint64_t cap_partials = 0;
@@ -139,20 +138,16 @@ StateLayout default_layout(int n, int dtype);
 // over states of the given layout.  Each field comes from the first of: the
 // circuit's own choice `pin` (may be null), the tunables set by
 // dmv_tune_set or DMV_<NAME>, the tuning table, the defaults.
-// `inner`: the forward of a gradient, whose state the caller does not get (see
-// PlanParams::fp32).
-PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const TuneChoice *pin = nullptr,
-                       bool inner = false);
+PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const TuneChoice *pin = nullptr);
 // States of up to this many qubits take the whole-state kernels.
-inline int small_qubits(int dtype, bool inner)
+inline int small_qubits(int dtype, bool adjoint)
 {
-    return dtype == DMV_C64 && !inner ? kSmallMaxQubitsFp32 : kSmallMaxQubits;
+    return dtype == DMV_C64 && !adjoint ? kSmallMaxQubitsFp32 : kSmallMaxQubits;
 }
 // Builds (if stale) and uploads the plan for `ops` into `dp`, for states of
 // the given layout.
 int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoint,
-                 const std::vector<HostOp> &ops, StateLayout layout, const TuneChoice *pin = nullptr,
-                 bool inner = false);
+                 const std::vector<HostOp> &ops, StateLayout layout, const TuneChoice *pin = nullptr);
 // Runs the passes of a prepared forward plan on s.
 int run_forward_plan(DevicePlan &dp, dmv_state *s);
 
@@ -172,8 +167,6 @@ int state_set(dmv_state *s, const double *re, const double *im);
 int state_probs(dmv_state *s, double *host);
 
 int circuit_forward(dmv_circuit *c, dmv_state *s, int mode);
-// The forward of a gradient, on its own scratch state.
-int circuit_inner_forward(dmv_circuit *c, dmv_state *s);
 // The observable of an adjoint gradient: the Z/ZZ form
 // H = sum_q a_q Z_q + sum_t b_t Z_pi[t] Z_pj[t] when table is null, else the
 // diagonal H|x> = table[sum_j bit_{wires[j]}(x) 2^j] |x>.

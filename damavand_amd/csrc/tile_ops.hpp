@@ -642,14 +642,13 @@ __device__ __forceinline__ void process_tile(typename Cplx<R>::T (&v)[1 << RLOG]
 }
 
 // One tile of a forward pass: load, run the phases, store.  S: the state's
-// real type, R: the type it is computed in.  complex64 gradients and batches are
-// computed in FP64: without packed FP32 instructions an FP32 operation takes a
-// vector instruction as an FP64 one does, so this costs registers and LDS only (16
-// amplitudes per thread instead of 32), a pass then rounds each amplitude once,
-// at its store, and the matrices are not rounded at all (energy of 21 qubits,
-// 4 layers: error 2e-7 -> 4e-8).  A complex64 forward whose state the caller gets
-// is computed in FP32, gates in order: which basis state a sample falls on
-// hangs on the last bits, and those stay what they are.
+// real type, R: the type it is computed in.  Reverse sweeps and batches of complex64
+// states are computed in FP64: without packed FP32 instructions an FP32 operation
+// takes a vector instruction as an FP64 one does, so this costs registers and
+// LDS only, a pass then rounds each amplitude once, at its store, and the
+// matrices are not rounded at all.  complex64 forwards are computed in FP32, gates
+// in order: which basis state a sample falls on, and what is left of an energy
+// whose terms cancel, hang on the last bits, and those stay what they are.
 template <class S, class R, int RLOG, int TLOG, bool NT, bool HALF = false>
 __device__ __forceinline__ void tile_body(typename Cplx<S>::T *__restrict__ state, const DevPass *P,
                                           const DevPhase *__restrict__ phases, const DevOp *__restrict__ ops,
