@@ -20,7 +20,7 @@ k_tile(typename Cplx<S>::T *__restrict__ state, const DevPass *__restrict__ pass
        StateLayout L)
 {
     using V = typename Cplx<R>::T;
-    __shared__ V lds[1 << (RLOG + TLOG - (HALF ? 1 : 0))];
+    __shared__ V lds[1 << (RLOG + TLOG - (HALF || by_parts<R, RLOG, TLOG>() ? 1 : 0))];
     // Workgroups are dealt to the XCDs round-robin.  With xcd_log2 = x > 0
     // (grid a multiple of 2^x), XCD j takes the j-th contiguous 2^-x share of
     // the tiles, so the tiles one XCD runs at a time are neighbours in memory.

@@ -109,6 +109,42 @@ __device__ __forceinline__ void transpose_half(V (&v)[NR], V *lds, const DevLayo
     }
 }
 
+// The same through half a tile of LDS in any pass: the real parts first, then the
+// imaginary ones, at the same indices.
+template <class P, class V, class ST, int NR, int TLOG>
+__device__ __forceinline__ void transpose_parts(V (&v)[NR], V *lds, const DevLayout *A, const uint32_t *src,
+                                                const DevLayout *B, const uint32_t *dst, uint32_t tid)
+{
+    constexpr int G = sizeof(ST) == 16 ? 3 : 4;
+    constexpr uint32_t UP = sizeof(P) > sizeof(ST) ? sizeof(P) / sizeof(ST) : 1;
+    constexpr uint32_t DOWN = sizeof(ST) > sizeof(P) ? sizeof(ST) / sizeof(P) : 1;
+    char *base = reinterpret_cast<char *>(lds);
+    const uint32_t la = swz_index<G>(thread_local_offset<TLOG>(A, tid)) * (uint32_t)sizeof(ST);
+    const uint32_t lb = swz_index<G>(thread_local_offset<TLOG>(B, tid)) * (uint32_t)sizeof(ST);
+#pragma unroll
+    for (int r = 0; r < NR; r++)
+        *reinterpret_cast<P *>(base + (la ^ src[r]) * UP / DOWN) = v[r].x;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < NR; r++)
+        v[r].x = *reinterpret_cast<const P *>(base + (lb ^ dst[r]) * UP / DOWN);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < NR; r++)
+        *reinterpret_cast<P *>(base + (la ^ src[r]) * UP / DOWN) = v[r].y;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < NR; r++)
+        v[r].y = *reinterpret_cast<const P *>(base + (lb ^ dst[r]) * UP / DOWN);
+    __syncthreads();
+}
+
+// Kernels whose registers allow three workgroups a CU (154) where a full tile of
+// LDS, 64 KiB, allows two.  Twice the LDS instructions and barriers, half of the
+// bytes each; complex128: 30 qubits, layered, 4 of 6 passes by parts 75.7 -> 71.9
+// ms, 24 qubits, random, 2.00 -> 1.85 ms, 28 qubits 20.2 -> 19.6 ms.
+template <class R, int RLOG, int TLOG> constexpr bool by_parts() { return sizeof(R) == 8 && RLOG == 4 && TLOG == 8; }
+
 constexpr int highest_bit(int m) { return m >= 16 ? 16 : m >= 8 ? 8 : m >= 4 ? 4 : m >= 2 ? 2 : 1; }
 
 // In-place pair ops of the reverse sweep.  A GEN (plain or not: one code
@@ -627,6 +663,8 @@ __device__ __forceinline__ void process_tile(typename Cplx<R>::T (&v)[1 << RLOG]
         if (D->transpose_in) {
             if constexpr (HALF)
                 transpose_half<V, ST, NR, TLOG>(v, lds, cur, D->src_lswz, &D->lay, D->dst_lswz, P->split, tid_again<R>(tid));
+            else if constexpr (by_parts<R, RLOG, TLOG>())
+                transpose_parts<R, V, ST, NR, TLOG>(v, lds, cur, D->src_lswz, &D->lay, D->dst_lswz, tid);
             else
                 transpose<V, ST, NR, TLOG>(v, lds, cur, D->src_lswz, &D->lay, D->dst_lswz, tid_again<R>(tid));
         }
@@ -636,6 +674,8 @@ __device__ __forceinline__ void process_tile(typename Cplx<R>::T (&v)[1 << RLOG]
     if (P->transpose_st) {
         if constexpr (HALF)
             transpose_half<V, ST, NR, TLOG>(v, lds, cur, P->st_src_lswz, &P->lay_st, P->st_dst_lswz, P->split, tid_again<R>(tid));
+        else if constexpr (by_parts<R, RLOG, TLOG>())
+            transpose_parts<R, V, ST, NR, TLOG>(v, lds, cur, P->st_src_lswz, &P->lay_st, P->st_dst_lswz, tid);
         else
             transpose<V, ST, NR, TLOG>(v, lds, cur, P->st_src_lswz, &P->lay_st, P->st_dst_lswz, tid_again<R>(tid));
     }
