@@ -1294,7 +1294,7 @@ int build_plan(const std::vector<HostOp> &given, const PlanParams &pp, Plan *out
     // op order: measured on the 30-qubit layered circuit, both ways take 19
     // passes, but searched ones 48 phases for 38 (114 against 109 ms).
     // Without a budget the search is tried too and the cheaper plan kept: 6
-    // passes of that circuit (77 ms), 9 for 25 at 20 qubits and 10 layers (328
+    // passes of that circuit (70 ms), 9 for 25 at 20 qubits and 10 layers (328
     // against 532 us).  A CNOT ring, whose next layer waits for the whole ring,
     // takes as many passes either way.
     constexpr int kInOrder = 8;
