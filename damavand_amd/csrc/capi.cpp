@@ -554,15 +554,14 @@ int dmv_circuit_destroy(dmv_circuit *c)
 {
     if (!c)
         return DMV_OK;
-    if (c->fwd.valid || c->adj.valid || c->d_partials || c->d_terms || c->d_grad) {
-        free_plan(c->fwd);
-        free_plan(c->adj);
-        release(c->d_partials);
-        release(c->d_terms);
-        release(c->d_grad);
-        pinned_free(c->pin_terms);
-        pinned_free(c->pin_grad);
-    }
+    // each of these does nothing where there is nothing on the device
+    free_plan(c->fwd);
+    free_plan(c->adj);
+    release(c->d_partials);
+    release(c->d_terms);
+    release(c->d_grad);
+    pinned_free(c->pin_terms);
+    pinned_free(c->pin_grad);
     delete c;
     return DMV_OK;
 }

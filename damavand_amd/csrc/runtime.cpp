@@ -589,6 +589,7 @@ int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoin
         dp.version = version;
         return DMV_OK;
     }
+    dp.valid = false;  // until everything is on the device: a call that fails on the way leaves no plan
     dp.small = small;
     dp.dtype = dtype;
     dp.pp = pp;

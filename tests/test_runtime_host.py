@@ -1,0 +1,84 @@
+"""The library's host code against a HIP runtime without a GPU
+(tests/hip_stand_in.cpp): what is left after a refused allocation, and how much
+memory a call asks for.  Each test runs in a process of its own, since the
+stand-in has to be loaded before the library."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = r"""
+import ctypes, sys
+S = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
+for name in ("stand_in_launches", "stand_in_bad_launches", "stand_in_peak", "stand_in_reset_peak"):
+    getattr(S, name).restype = ctypes.c_int64
+S.stand_in_capacity.argtypes = [ctypes.c_uint64]
+import numpy as np
+from damavand_amd import _native as N, workloads as wl
+from damavand_amd.circuit import Circuit
+
+def build(n, gates, dtype="complex128"):
+    c = Circuit(n, dtype=dtype)
+    for g in gates:
+        c.add_gate(*g)
+    return c
+"""
+
+
+@pytest.fixture(scope="module")
+def stand_in(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("hip") / "stand_in.so")
+    r = subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                        "-I/opt/rocm/include", os.path.join(ROOT, "tests", "hip_stand_in.cpp"), "-o", lib],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    return lib
+
+
+def run(stand_in, code, *args):
+    env = {k: v for k, v in os.environ.items() if not k.startswith("DMV_")}
+    env["PYTHONPATH"] = ROOT
+    r = subprocess.run([sys.executable, "-c", PRELUDE + code, stand_in, *args], env=env, capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+    return r.stdout
+
+
+@pytest.mark.parametrize("adjoint", [0, 1])
+def test_refused_allocation_leaves_no_plan(stand_in, adjoint):
+    """Gates are added, an allocation of the new plan is refused, and the call is made again: the passes and phases
+    that it launches are the new plan's, on the device."""
+    run(stand_in, r"""
+adjoint = int(sys.argv[2])
+refused = 0
+live = S.stand_in_reset_peak()
+for nth in range(1, 30):
+    c = build(16, wl.layered_circuit(16, 1, 1))
+    work = (lambda: c.gradient(np.ones(16))) if adjoint else c.forward
+    work()
+    for g in wl.layered_circuit(16, 6, 2):
+        c.add_gate(*g)
+    S.stand_in_fail_malloc(nth)
+    try:
+        work()
+        done = True
+    except N.OutOfDeviceMemory:
+        done = False
+    S.stand_in_fail_malloc(0)
+    before = S.stand_in_launches()
+    work()
+    again = S.stand_in_launches() - before
+    fresh = build(16, wl.layered_circuit(16, 1, 1) + wl.layered_circuit(16, 6, 2))
+    (fresh.gradient(np.ones(16)) if adjoint else fresh.forward())
+    assert S.stand_in_bad_launches() == 0, nth
+    assert c.plan_stats() == fresh.plan_stats()
+    refused += not done
+    del c, fresh, work
+    assert S.stand_in_reset_peak() == live, "device memory left behind"
+    if done:
+        break
+assert done and refused >= 2
+""", str(adjoint))
