@@ -67,6 +67,7 @@ static int upload_terms(Pinned &pin, double **buf, uint64_t *cap, int n, const d
     if (need > *cap) {
         release(*buf);
         *buf = nullptr;
+        *cap = 0;
         DMV_TRY(alloc((void **)buf, need * sizeof(double)));
         *cap = need;
     }
@@ -110,6 +111,7 @@ static int upload_table(Pinned &pin, double **buf, uint64_t *cap, int n, int n_w
     if (need > *cap) {
         release(*buf);
         *buf = nullptr;
+        *cap = 0;
         DMV_TRY(alloc((void **)buf, need * sizeof(double)));
         *cap = need;
     }
@@ -181,6 +183,7 @@ int dmv::circuit_adjoint(dmv_circuit *c, dmv_state *psi, dmv_state *lam, const O
     if (rows * per_ip > c->cap_partials) {
         release(c->d_partials);
         c->d_partials = nullptr;
+        c->cap_partials = 0;
         DMV_TRY(alloc((void **)&c->d_partials, rows * per_ip * sizeof(double)));
         c->cap_partials = rows * per_ip;
     }

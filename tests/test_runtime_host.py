@@ -82,3 +82,33 @@ for nth in range(1, 30):
         break
 assert done and refused >= 2
 """, str(adjoint))
+
+
+def test_refused_allocation_leaves_no_buffer_size(stand_in):
+    """A workspace that could not grow is gone with its size: what needs less of it afterwards allocates it again."""
+    run(stand_in, r"""
+refused = 0
+a, few, many = np.ones(16), [(0, 1)], [(q, q + 1) for q in range(15)]
+for nth in range(1, 30):
+    c = build(16, wl.layered_circuit(16, 1, 1))
+    c.gradient(a, few, np.ones(1))
+    c.expectation(a, few, np.ones(1))
+    for g in wl.layered_circuit(16, 6, 2):
+        c.add_gate(*g)
+    S.stand_in_fail_malloc(nth)
+    for work in (lambda: c.gradient(a, many, np.ones(15)), lambda: c.expectation(a, many, np.ones(15))):
+        try:
+            work()
+        except N.OutOfDeviceMemory:
+            refused += 1
+    S.stand_in_fail_malloc(0)
+    c.reset()
+    for g in wl.layered_circuit(16, 1, 1):
+        c.add_gate(*g)
+    c.gradient(a, few, np.ones(1))
+    c.expectation(a, few, np.ones(1))
+    assert S.stand_in_bad_launches() == 0, nth
+    if refused < nth:
+        break
+assert refused >= 5
+""")
