@@ -275,13 +275,24 @@ static int pinned_ready(Pinned &b, uint64_t bytes)
 
 constexpr uint64_t kPinnedMax = uint64_t(4) << 20;  // larger copies wait instead
 
+// Whether a copy goes through b: not a large one, and not where there is no
+// pinned memory to be had (its error would be taken for the next launch's).
+static bool goes_pinned(Pinned &b, uint64_t bytes)
+{
+    if (bytes > kPinnedMax)
+        return false;
+    if (pinned_ready(b, bytes) == DMV_OK)
+        return true;
+    (void)hipGetLastError();
+    return false;
+}
+
 int pinned_h2d(Pinned &b, void *dst, const void *src, uint64_t bytes)
 {
     if (bytes == 0)
         return DMV_OK;
-    if (bytes > kPinnedMax)
+    if (!goes_pinned(b, bytes))
         return copy_h2d(dst, src, bytes);
-    DMV_TRY(pinned_ready(b, bytes));
     std::memcpy(b.p, src, bytes);
     HIPCALL(hipMemcpyAsync(dst, b.p, bytes, hipMemcpyHostToDevice, stream()));
     HIPCALL(hipEventRecord(b.done, stream()));
@@ -293,9 +304,8 @@ int pinned_d2h(Pinned &b, void *dst, const void *src, uint64_t bytes)
 {
     if (bytes == 0)
         return DMV_OK;
-    if (bytes > kPinnedMax)
+    if (!goes_pinned(b, bytes))
         return copy_d2h(dst, src, bytes);
-    DMV_TRY(pinned_ready(b, bytes));
     HIPCALL(hipMemcpyAsync(b.p, src, bytes, hipMemcpyDeviceToHost, stream()));
     HIPCALL(hipStreamSynchronize(stream()));
     std::memcpy(dst, b.p, bytes);

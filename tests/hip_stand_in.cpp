@@ -18,7 +18,8 @@ std::map<uintptr_t, size_t> blocks;              // live device memory
 std::map<const void *, std::string> kernels;     // by host stub
 size_t live = 0, peak = 0, capacity = size_t(288) << 30;
 int64_t launches = 0, bad_launches = 0;
-int fail_malloc = 0, fail_host = 0;              // 1: the next one fails
+int fail_malloc = 0;                             // 1: the next one fails
+bool fail_host = false;                          // all pinned allocations fail
 hipError_t last = hipSuccess;
 struct Call {
     dim3 grid, block;
@@ -62,7 +63,7 @@ extern "C" {
 // ------------------------------------------------------ what tests look at --
 void stand_in_capacity(uint64_t bytes) { capacity = bytes; }
 void stand_in_fail_malloc(int nth) { fail_malloc = nth; }
-void stand_in_fail_host(int nth) { fail_host = nth; }
+void stand_in_fail_host(int on) { fail_host = on != 0; }
 int64_t stand_in_launches(void) { return launches; }
 int64_t stand_in_bad_launches(void) { return bad_launches; }
 uint64_t stand_in_peak(void) { return peak; }
@@ -139,7 +140,7 @@ hipError_t hipHostMalloc(void **p, size_t bytes, unsigned)
 {
     std::lock_guard<std::mutex> lk(mu);
     *p = nullptr;
-    if (fail_host > 0 && --fail_host == 0)
+    if (fail_host)
         return fail(hipErrorOutOfMemory);
     *p = ::operator new(bytes);
     return hipSuccess;

@@ -112,3 +112,18 @@ for nth in range(1, 30):
         break
 assert refused >= 5
 """)
+
+
+def test_no_pinned_memory(stand_in):
+    """Copies that go through pinned memory for speed are made without it where there is none."""
+    run(stand_in, r"""
+S.stand_in_fail_host(1)
+c = build(16, wl.layered_circuit(16, 2, 1))
+c.forward()
+c.expectation(np.ones(16), [(0, 1)], np.ones(1))
+c.state.expect_diag([1, 3], np.ones(4))
+c.gradient(np.ones(16))
+c.set_parameters(np.zeros(c.num_parameters))
+c.gradient(np.ones(16))
+assert S.stand_in_bad_launches() == 0
+""")
