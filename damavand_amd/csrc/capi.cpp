@@ -159,33 +159,48 @@ int dmv::circuit_adjoint(dmv_circuit *c, dmv_state *psi, dmv_state *lam, const O
                                  psi->ws, d_energy));
         prof_end(DMV_KC_REDUCE, 3.0 * (double)psi->bytes);
     }
-    // reverse sweep
-    DMV_TRY(prepare_plan(dp, c->version, c->n, psi->dtype, true, adjoint_ops(c->gates), psi->layout, pin));
-    if (dp.plan.n_slots != np) {
-        set_error("internal: adjoint plan has %d slots for %d parameters", dp.plan.n_slots, np);
-        return DMV_ERR_STATE;
-    }
-    // gradient partials: per (IP op, tile, wave) on the tile path, per slot
-    // on the whole-state path.  The tile path keeps the rows of as many
-    // consecutive passes as fit in kPartialBudget bytes (at least one pass)
-    // and sums them into grad with one launch whenever the next pass would
-    // not fit, so the buffer stays bounded at any state size.
+    // reverse sweep, with gradient partials per (IP op, tile, wave) on the tile
+    // path and per slot on the whole-state path.  The tile path keeps the rows
+    // of as many consecutive passes as fit in kPartialBudget bytes (at least
+    // one pass) and sums them into grad with one launch whenever the next pass
+    // would not fit.  Where the device has not even the room for one pass, the
+    // passes are planned with fewer IP ops.
     constexpr uint64_t kPartialBudget = uint64_t(256) << 20;
-    uint64_t per_ip = 1, rows = (uint64_t)(np > 0 ? np : 1);
-    if (!dp.small) {
-        per_ip = (uint64_t(1) << (c->n - dp.pp.k)) * ((uint64_t(1) << dp.pp.tlog) / 64);
+    uint64_t per_ip, rows, before = ~uint64_t(0);
+    for (;;) {
+        DMV_TRY(prepare_plan(dp, c->version, c->n, psi->dtype, true, adjoint_ops(c->gates), psi->layout, pin, c->max_ip));
+        if (dp.plan.n_slots != np) {
+            set_error("internal: adjoint plan has %d slots for %d parameters", dp.plan.n_slots, np);
+            return DMV_ERR_STATE;
+        }
         uint64_t widest = 1;
-        for (size_t p = 0; p < dp.plan.passes.size(); p++)
-            widest = std::max<uint64_t>(widest, dp.plan.ip_begin[p + 1] - dp.plan.ip_begin[p]);
-        rows = std::max(widest, std::min<uint64_t>(std::max<uint64_t>(1, dp.plan.ip_slots.size()),
-                                                   kPartialBudget / (per_ip * sizeof(double))));
-    }
-    if (rows * per_ip > c->cap_partials) {
+        per_ip = 1;
+        rows = (uint64_t)(np > 0 ? np : 1);
+        if (!dp.small) {
+            per_ip = partials_per_ip(dp.pp);
+            for (size_t p = 0; p < dp.plan.passes.size(); p++)
+                widest = std::max<uint64_t>(widest, dp.plan.ip_begin[p + 1] - dp.plan.ip_begin[p]);
+            rows = std::max(widest, std::min<uint64_t>(std::max<uint64_t>(1, dp.plan.ip_slots.size()),
+                                                       kPartialBudget / (per_ip * sizeof(double))));
+        }
+        if (rows * per_ip <= c->cap_partials)
+            break;
         release(c->d_partials);
         c->d_partials = nullptr;
         c->cap_partials = 0;
-        DMV_TRY(alloc((void **)&c->d_partials, rows * per_ip * sizeof(double)));
-        c->cap_partials = rows * per_ip;
+        int rc = alloc((void **)&c->d_partials, rows * per_ip * sizeof(double));
+        if (rc == DMV_ERR_MEMORY && rows > widest) {
+            rows = widest;
+            rc = alloc((void **)&c->d_partials, rows * per_ip * sizeof(double));
+        }
+        if (rc == DMV_OK) {
+            c->cap_partials = rows * per_ip;
+            break;
+        }
+        if (rc != DMV_ERR_MEMORY || dp.small || widest < 2 || widest >= before)
+            return rc;
+        before = widest;
+        c->max_ip = (int)(widest / 2);
     }
     if (dp.small) {
         prof_begin(DMV_KC_ADJOINT);
@@ -811,6 +826,8 @@ int dmv_circuit_plan_json(dmv_circuit *c, int dtype, int adjoint, int tile_qubit
         pp.tlog = threads_log2 > 0 ? threads_log2 : (tile_qubits >= 10 ? 8 : 6);
         pp.rlog = pp.k - pp.tlog;
         pp.half_lds = !adjoint && tune_value("half_lds", 1) != 0 && tile_half_exists(dtype, pp.rlog, pp.tlog) ? 1 : 0;
+        if (adjoint && pp.k <= pp.n)
+            pp.max_ip_per_pass = dmv::max_ip_per_pass(pp);
     }
     if (max_gen_per_pass > 0) {
         pp.max_gen_per_pass = max_gen_per_pass;

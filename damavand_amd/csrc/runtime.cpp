@@ -434,6 +434,14 @@ bool gate_nontemporal(uint32_t target, int dtype)
 }
 
 // ------------------------------------------------------------------- plans --
+int max_ip_per_pass(const PlanParams &pp)
+{
+    const uint64_t row = partials_per_ip(pp) * sizeof(double);
+    const int64_t kib = tune_value("adjoint_partial_kib", 0);
+    const uint64_t bytes = kib > 0 ? (uint64_t)kib << 10 : std::max(uint64_t(256) << 20, uint64_t(1) << pp.n);
+    return row ? (int)std::min(std::max<uint64_t>(1, bytes / row), uint64_t(1) << 30) : 1 << 30;
+}
+
 PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const TuneChoice *pin)
 {
     PlanParams pp;
@@ -520,6 +528,8 @@ PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const
     pp.nontemporal = nt != 0 ? 1 : 0;
     // forward passes split their transposes where the shape has half-LDS kernels
     pp.half_lds = !adjoint && tune_value("half_lds", 1) != 0 && tile_half_exists(dtype, pp.rlog, pp.tlog) ? 1 : 0;
+    if (adjoint)
+        pp.max_ip_per_pass = max_ip_per_pass(pp);
     return pp;
 }
 
@@ -580,13 +590,15 @@ static int upload_ops(DevicePlan &dp, const std::vector<DevOp> &given, bool fp32
 }
 
 int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoint, const std::vector<HostOp> &ops,
-                 StateLayout layout, const TuneChoice *pin)
+                 StateLayout layout, const TuneChoice *pin, int max_ip)
 {
     const bool small = n <= small_qubits(dtype, adjoint);
     PlanParams pp = small ? PlanParams{} : tile_params(n, dtype, adjoint, layout, pin);
+    if (max_ip > 0)
+        pp.max_ip_per_pass = std::min(pp.max_ip_per_pass, max_ip);
     const bool same_shape = dp.valid && dp.dtype == dtype && dp.small == small &&
                             (small || (dp.pp.k == pp.k && dp.pp.tlog == pp.tlog && dp.pp.max_gen_per_pass == pp.max_gen_per_pass &&
-                                       dp.pp.gen_auto == pp.gen_auto &&
+                                       dp.pp.gen_auto == pp.gen_auto && dp.pp.max_ip_per_pass == pp.max_ip_per_pass &&
                                        dp.pp.nontemporal == pp.nontemporal && dp.pp.half_lds == pp.half_lds &&
                                        same_layout(dp.pp.layout, pp.layout)));
     if (same_shape && dp.version == version && dp.epoch == tune_epoch())

@@ -102,6 +102,7 @@ struct dmv_circuit {
     dmv::TuneChoice tune_fwd, tune_adj;  // set by the autotuner for this gate list
     double *d_partials = nullptr;   // adjoint partials of one pass: per (IP op, tile, wave)
     uint64_t cap_partials = 0;
+    int max_ip = 0;                 // IP ops a pass that there was memory for, if fewer than planned (0: enough)
     double *d_terms = nullptr;      // observable terms
     uint64_t cap_terms = 0;
     double *d_grad = nullptr;       // gradient, then the energy
@@ -144,10 +145,20 @@ inline int small_qubits(int dtype, bool adjoint)
 {
     return dtype == DMV_C64 && !adjoint ? kSmallMaxQubitsFp32 : kSmallMaxQubits;
 }
+// How many IP ops a pass of a reverse sweep may hold.  Each takes a partial, a
+// double, per tile and wave: 16 MiB an op at 30 qubits.  A byte an amplitude (a
+// sixteenth of a complex128 state, 256 MiB at least; tunable adjoint_partial_kib)
+// is 64 ops with 11-qubit tiles.  Without a limit the searched passes of 20
+// brickwork layers at 33 qubits hold up to 315: 39 GiB beside two states of
+// 128 GiB.
+inline uint64_t partials_per_ip(const PlanParams &pp) { return (uint64_t(1) << (pp.n - pp.k)) * ((uint64_t(1) << pp.tlog) / 64); }
+int max_ip_per_pass(const PlanParams &pp);
 // Builds (if stale) and uploads the plan for `ops` into `dp`, for states of
-// the given layout.
+// the given layout.  max_ip: fewer IP ops a pass than
+// max_ip_per_pass says (0: as many).
 int prepare_plan(DevicePlan &dp, uint64_t version, int n, int dtype, bool adjoint,
-                 const std::vector<HostOp> &ops, StateLayout layout, const TuneChoice *pin = nullptr);
+                 const std::vector<HostOp> &ops, StateLayout layout, const TuneChoice *pin = nullptr,
+                 int max_ip = 0);
 // Runs the passes of a prepared forward plan on s.
 int run_forward_plan(DevicePlan &dp, dmv_state *s);
 

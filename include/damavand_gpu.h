@@ -349,6 +349,8 @@ int dmv_synchronize(void);
  * forward passes over states of 2 GiB and more, for reverse sweeps whose
  * two states together take 512 MiB and more, and for batches whose scratch
  * states take 512 MiB and more),
+ * "adjoint_partial_kib" (gradient partials of one reverse pass, which bound
+ * its parametrised gates; default a KiB per 1024 amplitudes, 256 MiB at least),
  * "gate_pairs_per_thread" (1, 2, 4), "batch_tile_qubits",
  * "batch_threads_log2", "batch_wgs_per_cu" (1..16, without
  * effect: a batch's launches fill the chip), "graph" (0/1: replay forward

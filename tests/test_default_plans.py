@@ -75,3 +75,27 @@ def test_default_reverse_plan(n, layers):
             vals.append(oracle.run_gates(n, gates[:gi] + [(kk, c, t, (p[0] + s,))] + gates[gi + 1:]).expect_zz(a, pairs, b))
         ref.append(0.5 * (vals[0] - vals[1]))
     np.testing.assert_allclose(grads, ref, atol=1e-10)
+
+
+@pytest.mark.parametrize("kib,most", [(1, 8), (2, 16), (8, 64)])
+def test_reverse_plan_within_its_partials(kib, most):
+    """Passes of a bounded number of gradient entries (128 bytes of partials each at 13 qubits), in order all the
+    same: the gradients of the unbounded plan."""
+    n = 13
+    gates, a, b = wl.ansatz_circuit(n, 4, 31)
+    gates = [(k, -1, q, (0.3 * q + j,)) for q in range(n) for j, k in enumerate((wl.GATE_RX, wl.GATE_RY, wl.GATE_RX))] + gates
+    nc = NativeCircuit(n, gates)
+    psi = oracle.run_gates(n, gates).amp
+    idx = np.arange(1 << n)
+    lam = psi * sum(c * (1.0 - 2.0 * ((idx >> q) & 1)) for q, c in enumerate(a))
+    free = plan_json(nc.h, adjoint=True)
+    N.tune_set("adjoint_partial_kib", kib)
+    try:
+        plan = plan_json(nc.h, adjoint=True)
+    finally:
+        N.tune_set("adjoint_partial_kib", -1)
+    per_pass = [[op["slot"] for ph in p["phases"] for op in ph["ops"] if op["slot"] >= 0] for p in plan["passes"]]
+    assert max(len(s) for s in per_pass) <= most
+    assert sorted(s for p in per_pass for s in p) == list(range(sum(g[0] in wl.PARAMETRIC for g in gates)))
+    want = TileEmulator(free).reverse(psi, lam)[2]
+    np.testing.assert_allclose(TileEmulator(plan).reverse(psi, lam)[2], want, atol=1e-11)

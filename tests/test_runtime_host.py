@@ -127,3 +127,48 @@ c.set_parameters(np.zeros(c.num_parameters))
 c.gradient(np.ones(16))
 assert S.stand_in_bad_launches() == 0
 """)
+
+
+BRICKWORK = r"""
+def brickwork(n, layers):
+    rng = np.random.default_rng(n)
+    gates = []
+    for layer in range(layers):
+        for kind in (wl.GATE_RX, wl.GATE_RY, wl.GATE_RZ):
+            gates += [(kind, -1, q, (t,)) for q, t in enumerate(rng.uniform(0, 6, n))]
+        gates += [(wl.GATE_CZ, q, q + 1, ()) for q in range(layer % 2, n - 1, 2)]
+    return gates
+"""
+
+
+def test_gradient_of_the_largest_states_fits(stand_in):
+    """33 qubits: two states of 128 GiB and the partials of 1980 angles on a card of 288 GiB."""
+    run(stand_in, BRICKWORK + r"""
+from tests.libhelpers import NativeCircuit
+n = 33
+c = NativeCircuit(n, brickwork(n, 20))
+psi, lam, e = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_double(0)
+N.call("dmv_state_create", n, N.C128, ctypes.byref(psi))
+N.call("dmv_state_create", n, N.C128, ctypes.byref(lam))
+a, g = np.ones(n), np.empty(3 * 20 * n)
+before = S.stand_in_reset_peak()
+N.call("dmv_circuit_adjoint", c.h, psi, lam, N.dptr(a), 0, None, None, None, ctypes.byref(e), N.dptr(g))
+assert S.stand_in_bad_launches() == 0
+assert S.stand_in_peak() - before <= (1 << n) + (1 << 20)  # the partials: a byte an amplitude
+""")
+
+
+@pytest.mark.parametrize("mib", [40, 16, 6])
+def test_gradient_plans_for_the_memory_there_is(stand_in, mib):
+    """24 qubits, where the widest pass would take 79 MiB of partials, with less than that left on the device."""
+    run(stand_in, BRICKWORK + r"""
+n, left = 24, int(sys.argv[2]) << 20
+c = build(n, brickwork(n, 20))
+c._scratch = (c.state, build(n, []).state)
+c.forward()
+S.stand_in_capacity(S.stand_in_reset_peak() + left)
+for _ in range(2):
+    c.gradient(np.ones(n))
+    c.set_parameters(np.zeros(c.num_parameters))
+assert S.stand_in_bad_launches() == 0
+""", str(mib))
