@@ -1012,8 +1012,8 @@ int dmv_circuit_tile_shape(dmv_circuit *c, int dtype, int adjoint, int *tile_qub
         *threads_log2 = pp.tlog;
     if (max_gen_per_pass) {
         *max_gen_per_pass = pp.max_gen_per_pass;
-        if (pp.gen_auto && !adjoint && c->n > pp.k) {
-            // no budget is set: the one that would suit the forward's gates in their order
+        if (pp.gen_auto && pp.max_gen_per_pass > 0 && !adjoint && c->n > pp.k) {
+            // nothing is set: the budget that would suit the forward's gates in their order
             DMV_TRY(in_order_budget(merge_ops(forward_ops(c->gates)), pp, max_gen_per_pass));
         }
     }

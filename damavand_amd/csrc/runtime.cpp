@@ -442,6 +442,33 @@ int max_ip_per_pass(const PlanParams &pp)
     return row ? (int)std::min(std::max<uint64_t>(1, bytes / row), uint64_t(1) << 30) : 1 << 30;
 }
 
+void default_shape(int n, int dtype, bool adjoint, int *k, int *tlog)
+{
+    const bool fp32 = dtype == DMV_C64 && !adjoint;
+    // 256 threads; k = 12 forward (FP32: 13), 11 for reverse sweeps, which hold
+    // psi and lambda in registers together
+    *k = adjoint ? 11 : (fp32 ? 13 : 12);
+    *tlog = 8;
+    // Small states run 8 amplitudes per thread on every thread that their tiles
+    // have: with one tile a CU or fewer a pass is a chain of latencies, which
+    // more waves overlap, and the 16-amplitude kernels' code (140 KiB) does not
+    // stay in the instruction cache.  16 qubits, 8 layers: 160 us on 11-qubit
+    // tiles against 204 on 12-qubit ones and 209 on one-wave 9-qubit ones; 20
+    // qubits: 377 us on 512 threads against 414 (11-qubit tiles) and 474 (12, 16
+    // amplitudes per thread), which win from 23 qubits on (27: 21.6 ms against
+    // 22.4).  Up to 12 qubits (reverse sweeps 11) the whole state is one tile, so
+    // a plan is one pass (12 qubits: 96 us against 104 in passes of 11).
+    if (fp32) {
+        if (n < 19) {
+            *tlog = 6;
+            *k = 10;
+        }
+    } else if (n <= (adjoint ? 24 : 20)) {
+        *k = adjoint || (n > 12 && n < 20) ? std::min(n, 11) : std::min(n, 12);
+        *tlog = *k <= 9 ? 6 : (*k == 12 ? 9 : 8);
+    }
+}
+
 PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const TuneChoice *pin)
 {
     PlanParams pp;
@@ -454,8 +481,6 @@ PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const
     if (runs > pp.low_bits && runs <= 6)
         pp.low_bits = (int)runs;
     pp.swz_bits = dtype == DMV_C64 ? 4 : 3;
-    // defaults: 256 threads; k = 12 forward (FP32: 13), 11 for reverse sweeps,
-    // which hold psi and lambda in registers together
     int k = adjoint ? 11 : (pp.fp32 ? 13 : 12);
     // streaming (nontemporal) loads and stores: forward passes from 2 GiB
     // states up (measured 1.5-3.5% faster per pass at 27, 30 and 33 qubits,
@@ -473,8 +498,8 @@ PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const
     if (tune_lookup(tune_key(n, dtype, adjoint ? "adjoint" : "forward"), &t) && t.set()) {
         k = t.k;
         tlog = t.tlog > 0 ? t.tlog : tlog;
-        gen = t.max_gen > 0 ? t.max_gen : gen;
-        gen_set = t.max_gen > 0;
+        gen = t.max_gen;
+        gen_set = gen > 0;
         nt = t.nt >= 0 ? t.nt : nt;
         chosen = true;
     }
@@ -494,29 +519,13 @@ PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const
     if (pin && pin->set()) {
         k = pin->k;
         tlog = pin->tlog > 0 ? pin->tlog : tlog;
-        gen = pin->max_gen > 0 ? pin->max_gen : gen;
-        gen_set = gen_set || pin->max_gen > 0;
+        gen = pin->max_gen;
+        gen_set = gen > 0;
         nt = pin->nt >= 0 ? pin->nt : nt;
         chosen = true;
     }
-    // Small states run 8 amplitudes per thread on every thread that their tiles
-    // have: with one tile a CU or fewer a pass is a chain of latencies, which
-    // more waves overlap, and the 16-amplitude kernels' code (140 KiB) does not
-    // stay in the instruction cache.  16 qubits, 8 layers: 160 us on 11-qubit
-    // tiles against 204 on 12-qubit ones and 209 on one-wave 9-qubit ones; 20
-    // qubits: 377 us on 512 threads against 414 (11-qubit tiles) and 474 (12, 16
-    // amplitudes per thread), which win from 23 qubits on (27: 21.6 ms against
-    // 22.4).  Up to 12 qubits (reverse sweeps 11) the whole state is one tile, so
-    // a plan is one pass (12 qubits: 96 us against 104 in passes of 11).
-    if (!chosen && pp.fp32) {
-        if (n < k + 6) {
-            tlog = 6;
-            k = 10;
-        }
-    } else if (!chosen && (!given || n < k + 6) && n <= (adjoint ? 24 : 20)) {
-        k = adjoint || (n > 12 && n < 20) ? std::min(n, 11) : std::min(n, 12);
-        tlog = k <= 9 ? 6 : (k == 12 ? 9 : 8);
-    }
+    if (!chosen && (!given || n < k + 6))
+        default_shape(n, dtype, adjoint, &k, &tlog);
     if (k > n)
         k = n;
     pp.k = k;

@@ -17,7 +17,7 @@ namespace dmv {
 struct TuneChoice {
     int k = 0;        // tile qubits
     int tlog = 0;     // log2 threads per workgroup
-    int max_gen = 0;  // general 2x2 ops per fused pass
+    int max_gen = 0;  // general 2x2 ops per fused pass (of a set choice, 0: no budget, plans by cost)
     int nt = -1;      // forward passes: nontemporal loads and stores (0/1)
     int wgs = 0;      // batched kernel: workgroups per CU
     double ms = 0.0;  // measured time of the choice
@@ -139,6 +139,8 @@ StateLayout default_layout(int n, int dtype);
 // over states of the given layout.  Each field comes from the first of: the
 // circuit's own choice `pin` (may be null), the tunables set by
 // dmv_tune_set or DMV_<NAME>, the tuning table, the defaults.
+// The tile shape where nothing is set, measured or tuned.
+void default_shape(int n, int dtype, bool adjoint, int *k, int *tlog);
 PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const TuneChoice *pin = nullptr);
 // States of up to this many qubits take the whole-state kernels.
 inline int small_qubits(int dtype, bool adjoint)

@@ -4,8 +4,8 @@
 // by timing the candidates on the caller's workload, kept in a process-wide
 // table and in an optional JSON-lines cache file (DMV_TUNE_CACHE), and
 // applied per circuit:
-//  * forward: tile qubits, threads per workgroup, GEN budget per pass and
-//    streaming stores of the fused passes;
+//  * forward: tile qubits, threads per workgroup, GEN budget per pass (or none)
+//    and streaming stores of the fused passes;
 //  * adjoint: tile qubits, threads and GEN budget of the reverse sweep;
 //  * batch: tile shape.
 #include <algorithm>
@@ -199,14 +199,22 @@ struct Plan1 {
 };
 
 // Candidate tile shapes (tile qubits, log2 threads) with kernels in this
-// library, largest first.
-std::vector<std::pair<int, int>> shapes(int dtype, bool adjoint)
+// library: the default shape of the size, then others of at most n - 3 qubits.
+std::vector<std::pair<int, int>> shapes(int n, int dtype, bool adjoint)
 {
+    int k, tlog;
+    default_shape(n, dtype, adjoint, &k, &tlog);
+    std::vector<std::pair<int, int>> out{{k, tlog}}, all;
     if (adjoint)
-        return dtype == DMV_C64 ? std::vector<std::pair<int, int>>{{12, 8}, {11, 8}, {10, 6}, {9, 6}}
-                                : std::vector<std::pair<int, int>>{{11, 8}, {10, 8}, {9, 6}};
-    return dtype == DMV_C64 ? std::vector<std::pair<int, int>>{{13, 8}, {12, 8}, {11, 8}, {10, 6}, {9, 6}}
-                            : std::vector<std::pair<int, int>>{{12, 8}, {12, 9}, {11, 8}, {11, 7}, {10, 8}, {9, 6}};
+        all = dtype == DMV_C64 ? std::vector<std::pair<int, int>>{{12, 8}, {11, 8}, {10, 6}, {9, 6}}
+                               : std::vector<std::pair<int, int>>{{11, 8}, {10, 8}, {9, 6}};
+    else
+        all = dtype == DMV_C64 ? std::vector<std::pair<int, int>>{{13, 8}, {12, 8}, {11, 8}, {10, 6}, {9, 6}}
+                               : std::vector<std::pair<int, int>>{{12, 8}, {12, 9}, {11, 8}, {11, 7}, {10, 8}, {9, 6}};
+    for (const auto &shape : all)
+        if (shape.first + 3 <= n && shape != out[0])
+            out.push_back(shape);
+    return out;
 }
 
 // Times `run` on the library stream: the smaller of two runs after a warm-up.
@@ -248,10 +256,8 @@ int autotune_forward(dmv_circuit *c, dmv_state *s, int *chosen)
     const std::vector<HostOp> ops = forward_ops(c->gates);
     TuneChoice best;
     float best_ms = 1e30f;
-    for (auto [k, tlog] : shapes(s->dtype, false)) {
-        if (k + 3 > s->n)
-            continue;
-        for (int gen : {6, 8, 12, 16}) {
+    for (auto [k, tlog] : shapes(s->n, s->dtype, false)) {
+        for (int gen : {0, 6, 8, 12, 16}) {  // 0: no budget, as without tuning
             TuneChoice cand;
             cand.k = k;
             cand.tlog = tlog;
@@ -266,11 +272,6 @@ int autotune_forward(dmv_circuit *c, dmv_state *s, int *chosen)
                 best = cand;
             }
         }
-    }
-    if (!best.set()) {
-        if (chosen)
-            *chosen = 0;
-        return DMV_OK;
     }
     {  // streaming loads and stores on the best shape
         TuneChoice cand = best;
@@ -311,10 +312,8 @@ int autotune_adjoint(dmv_circuit *c, int dtype, int *chosen)
     obs.a = a.data();
     TuneChoice best;
     float best_ms = 1e30f;
-    for (auto [k, tlog] : shapes(dtype, true)) {
-        if (k + 3 > c->n)
-            continue;
-        for (int gen : {8, 16}) {
+    for (auto [k, tlog] : shapes(c->n, dtype, true)) {
+        for (int gen : {0, 8, 16}) {
             TuneChoice cand;
             cand.k = k;
             cand.tlog = tlog;
@@ -331,11 +330,6 @@ int autotune_adjoint(dmv_circuit *c, int dtype, int *chosen)
                 best = cand;
             }
         }
-    }
-    if (!best.set()) {
-        if (chosen)
-            *chosen = 0;
-        return DMV_OK;
     }
     best.ms = best_ms;
     c->tune_adj = best;

@@ -172,3 +172,53 @@ for _ in range(2):
     c.set_parameters(np.zeros(c.num_parameters))
 assert S.stand_in_bad_launches() == 0
 """, str(mib))
+
+
+@pytest.mark.parametrize("n,layers,dtype", [(30, 5, "complex128"), (20, 4, "complex128"), (14, 4, "complex128"),
+                                            (10, 2, "complex128"), (20, 3, "complex64")])
+def test_autotuner_can_keep_the_default(stand_in, tmp_path, n, layers, dtype):
+    """Where every launch takes as long, tuning chooses no plan with more launches than the default's, and another
+    process that reads the choice from the file makes that plan."""
+    run(stand_in, r"""
+import os
+n, layers, dtype = int(sys.argv[2]), int(sys.argv[3]), sys.argv[4]
+gates = wl.layered_circuit(n, layers, 1)
+
+def forward_launches(c):
+    before = S.stand_in_launches()
+    c.forward()
+    return S.stand_in_launches() - before
+
+default = forward_launches(build(n, gates, dtype))
+os.environ["DMV_TUNE_CACHE"] = sys.argv[5]
+N.call("dmv_tune_forget")
+c = build(n, gates, dtype)
+k = c.autotune()
+shape = c.tile_shape()
+assert k == shape["tile_qubits"] and k <= n
+tuned = forward_launches(c)
+assert tuned <= default, (tuned, default, shape)
+N.call("dmv_tune_forget")
+fresh = build(n, gates, dtype)
+assert fresh.tile_shape() == shape and forward_launches(fresh) == tuned
+""", str(n), str(layers), dtype, str(tmp_path / "tune.jsonl"))
+
+
+@pytest.mark.parametrize("n,dtype", [(23, "complex128"), (13, "complex128"), (10, "complex128"), (12, "complex64")])
+def test_adjoint_autotuner_can_keep_the_default(stand_in, n, dtype):
+    run(stand_in, r"""
+n, dtype = int(sys.argv[2]), sys.argv[3]
+gates = wl.layered_circuit(n, 4, 1)
+
+def launches(c):
+    c.gradient(np.ones(n))
+    before = S.stand_in_launches()
+    c.gradient(np.ones(n))
+    return S.stand_in_launches() - before
+
+default = launches(build(n, gates, dtype))
+c = build(n, gates, dtype)
+k = c.autotune(adjoint=True)
+assert k == c.tile_shape(adjoint=True)["tile_qubits"] and 9 <= k <= n
+assert launches(c) <= default, (launches(c), default)
+""", str(n), dtype)
