@@ -524,7 +524,7 @@ PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const
         nt = pin->nt >= 0 ? pin->nt : nt;
         chosen = true;
     }
-    if (!chosen && (!given || n < k + 6))
+    if (k > n || (!chosen && (!given || n < k + 6)))  // (a shape of larger states does not fit this one)
         default_shape(n, dtype, adjoint, &k, &tlog);
     if (k > n)
         k = n;

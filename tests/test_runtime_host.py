@@ -222,3 +222,19 @@ k = c.autotune(adjoint=True)
 assert k == c.tile_shape(adjoint=True)["tile_qubits"] and 9 <= k <= n
 assert launches(c) <= default, (launches(c), default)
 """, str(n), dtype)
+
+
+@pytest.mark.parametrize("n", [9, 10, 11])
+def test_tuning_entry_larger_than_the_state(stand_in, tmp_path, n):
+    """An entry whose tile is larger than the state does not apply (it never did at these sizes)."""
+    (tmp_path / "tune.jsonl").write_text("".join(
+        '{"key": "gfx950/n%d/c128/%s", "tile_qubits": 12, "threads_log2": 8, "max_gen_per_pass": 8}\n' % (n, kind)
+        for kind in ("forward", "adjoint")))
+    run(stand_in, r"""
+import os
+os.environ["DMV_TUNE_CACHE"] = sys.argv[2]
+n = int(sys.argv[3])
+c = build(n, wl.layered_circuit(n, 2, 1))
+c.forward()
+c.gradient(np.ones(n))
+""", str(tmp_path / "tune.jsonl"), str(n))
