@@ -362,10 +362,13 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
         C.adj_ops = n_ops + T.pf->ops.size();
         n_ops += T.pf->ops.size() + T.pa->ops.size();
     }
-    // Circuits run in groups whose states and partials fit kPoolBytes (one
-    // circuit at least); with the default tiles the 4096-circuit 12-18 qubit
-    // batch in complex128 takes 9.8 + 1.3 GB and is one group.
-    constexpr uint64_t kPoolBytes = uint64_t(16) << 30;
+    // Circuits run in groups whose states and partials fit `limit` bytes (one
+    // circuit at least): 16 GiB, or tunable batch_pool_mib, and half of what a
+    // group took where the device has no room for it.  With the default tiles the
+    // 4096-circuit 12-18 qubit batch in complex128 takes 9.8 + 1.3 GB and is
+    // one group.
+    const int64_t pool_mib = tune_value("batch_pool_mib", 0);
+    uint64_t limit = pool_mib > 0 ? (uint64_t)pool_mib << 20 : uint64_t(16) << 30;
     const uint32_t waves = (1u << tlog) / 64;
     struct Group {
         uint32_t first, count;
@@ -376,48 +379,56 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
     std::vector<Group> groups;
     std::vector<BatchTile> by_fwd, by_adj;
     uint64_t pool_amps = 0, pool_parts = 0, pool_tiles = 0;
-    for (int i = 0; i < count;) {
-        Group G{(uint32_t)i, 0, by_fwd.size(), {}, {}, 0};
-        uint64_t amps = 0, parts = 0, tiles = 0;
-        for (; i < count; i++) {
-            BatchCircuit &C = circ[i];
-            const uint64_t a2 = amps + 2 * C.amps, p2 = parts + (uint64_t)C.n_ip * C.tiles * waves;
-            if (G.count > 0 && a2 * amp_bytes(dtype) + p2 * 8 > kPoolBytes)
-                break;
-            C.state = amps;
-            C.parts = parts;
-            C.tile0 = (uint32_t)tiles;
-            amps = a2;
-            parts = p2;
-            tiles += C.tiles;
-            G.count++;
-        }
-        DMV_CHECK_ARG(tiles <= 0x7FFFFFFFull, "batch too large");
-        G.tiles = (uint32_t)tiles;
-        pool_amps = std::max(pool_amps, amps);
-        pool_parts = std::max(pool_parts, parts);
-        pool_tiles = std::max(pool_tiles, tiles);
-        for (int which = 0; which < 2; which++) {
-            auto levels = [&](uint32_t c) {
-                const Built &T = built[built[c].like];
-                return (which == 0 ? *T.pf : *T.pa).passes.size();
-            };
-            std::vector<uint32_t> order(G.count);
-            for (uint32_t j = 0; j < G.count; j++)
-                order[j] = G.first + j;
-            std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return levels(x) > levels(y); });
-            std::vector<BatchTile> &list = which == 0 ? by_fwd : by_adj;
-            std::vector<uint32_t> &per_level = which == 0 ? G.fwd_tiles : G.adj_tiles;
-            per_level.assign(levels(order[0]), 0);
-            for (uint32_t c : order) {
-                for (uint32_t t = 0; t < circ[c].tiles; t++)
-                    list.push_back({c, t});
-                for (size_t p = 0; p < levels(c); p++)
-                    per_level[p] += circ[c].tiles;
+    auto make_groups = [&]() -> int {
+        groups.clear();
+        by_fwd.clear();
+        by_adj.clear();
+        pool_amps = pool_parts = pool_tiles = 0;
+        for (int i = 0; i < count;) {
+            Group G{(uint32_t)i, 0, by_fwd.size(), {}, {}, 0};
+            uint64_t amps = 0, parts = 0, tiles = 0;
+            for (; i < count; i++) {
+                BatchCircuit &C = circ[i];
+                const uint64_t a2 = amps + 2 * C.amps, p2 = parts + (uint64_t)C.n_ip * C.tiles * waves;
+                if (G.count > 0 && a2 * amp_bytes(dtype) + p2 * 8 > limit)
+                    break;
+                C.state = amps;
+                C.parts = parts;
+                C.tile0 = (uint32_t)tiles;
+                amps = a2;
+                parts = p2;
+                tiles += C.tiles;
+                G.count++;
             }
+            DMV_CHECK_ARG(tiles <= 0x7FFFFFFFull, "batch too large");
+            G.tiles = (uint32_t)tiles;
+            pool_amps = std::max(pool_amps, amps);
+            pool_parts = std::max(pool_parts, parts);
+            pool_tiles = std::max(pool_tiles, tiles);
+            for (int which = 0; which < 2; which++) {
+                auto levels = [&](uint32_t c) {
+                    const Built &T = built[built[c].like];
+                    return (which == 0 ? *T.pf : *T.pa).passes.size();
+                };
+                std::vector<uint32_t> order(G.count);
+                for (uint32_t j = 0; j < G.count; j++)
+                    order[j] = G.first + j;
+                std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return levels(x) > levels(y); });
+                std::vector<BatchTile> &list = which == 0 ? by_fwd : by_adj;
+                std::vector<uint32_t> &per_level = which == 0 ? G.fwd_tiles : G.adj_tiles;
+                per_level.assign(levels(order[0]), 0);
+                for (uint32_t c : order) {
+                    for (uint32_t t = 0; t < circ[c].tiles; t++)
+                        list.push_back({c, t});
+                    for (size_t p = 0; p < levels(c); p++)
+                        per_level[p] += circ[c].tiles;
+                }
+            }
+            groups.push_back(std::move(G));
         }
-        groups.push_back(std::move(G));
-    }
+        return DMV_OK;
+    };
+    DMV_TRY(make_groups());
 
     // host work and argument checks are done: only now touch the device
     DMV_TRY(ensure_device());
@@ -427,21 +438,34 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
 
     // One device buffer: what the host fills in first, so that it goes over in
     // one copy, then the results, partials and states.
-    Arena A;
-    const uint64_t o_circ = A.part(circ.size() * sizeof(BatchCircuit));
-    const uint64_t o_fwd = A.part(by_fwd.size() * sizeof(BatchTile));
-    const uint64_t o_adj = A.part(by_adj.size() * sizeof(BatchTile));
-    const uint64_t o_passes = A.part(passes.size() * sizeof(DevPass));
-    const uint64_t o_phases = A.part(phases.size() * sizeof(DevPhase));
-    const uint64_t o_ops = A.part(n_ops * sizeof(DevOp));
-    const uint64_t o_slots = A.part(slots.size() * sizeof(int));
-    const uint64_t o_coef = A.part((uint64_t)coef_len * sizeof(double));
-    const uint64_t o_energy = A.part((uint64_t)count * sizeof(double) + (uint64_t)total_params * sizeof(double));
-    const uint64_t o_grad = o_energy + (uint64_t)count * sizeof(double);
-    const uint64_t o_eparts = A.part(pool_tiles * sizeof(double));
-    const uint64_t o_parts = A.part(pool_parts * sizeof(double));
-    const uint64_t o_pool = A.part(pool_amps * (uint64_t)amp_bytes(dtype));
-    DMV_TRY(A.get(o_energy));
+    std::unique_ptr<Arena> arena;
+    uint64_t o_circ, o_fwd, o_adj, o_passes, o_phases, o_ops, o_slots, o_coef, o_energy, o_grad, o_eparts, o_parts, o_pool;
+    for (;;) {
+        arena.reset();
+        arena.reset(new Arena);
+        Arena &A = *arena;
+        o_circ = A.part(circ.size() * sizeof(BatchCircuit));
+        o_fwd = A.part(by_fwd.size() * sizeof(BatchTile));
+        o_adj = A.part(by_adj.size() * sizeof(BatchTile));
+        o_passes = A.part(passes.size() * sizeof(DevPass));
+        o_phases = A.part(phases.size() * sizeof(DevPhase));
+        o_ops = A.part(n_ops * sizeof(DevOp));
+        o_slots = A.part(slots.size() * sizeof(int));
+        o_coef = A.part((uint64_t)coef_len * sizeof(double));
+        o_energy = A.part((uint64_t)count * sizeof(double) + (uint64_t)total_params * sizeof(double));
+        o_grad = o_energy + (uint64_t)count * sizeof(double);
+        o_eparts = A.part(pool_tiles * sizeof(double));
+        o_parts = A.part(pool_parts * sizeof(double));
+        o_pool = A.part(pool_amps * (uint64_t)amp_bytes(dtype));
+        const int rc = A.get(o_energy);
+        if (rc == DMV_OK)
+            break;
+        if (rc != DMV_ERR_MEMORY || groups.size() == (size_t)count)
+            return rc;
+        limit = std::min(limit, pool_amps * (uint64_t)amp_bytes(dtype) + pool_parts * sizeof(double)) / 2;
+        DMV_TRY(make_groups());
+    }
+    Arena &A = *arena;
     char *filled = A.host();
     std::memcpy(filled + o_circ, circ.data(), circ.size() * sizeof(BatchCircuit));
     std::memcpy(filled + o_fwd, by_fwd.data(), by_fwd.size() * sizeof(BatchTile));

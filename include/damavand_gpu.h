@@ -352,7 +352,9 @@ int dmv_synchronize(void);
  * "adjoint_partial_kib" (gradient partials of one reverse pass, which bound
  * its parametrised gates; default a KiB per 1024 amplitudes, 256 MiB at least),
  * "gate_pairs_per_thread" (1, 2, 4), "batch_tile_qubits",
- * "batch_threads_log2", "batch_wgs_per_cu" (1..16, without
+ * "batch_threads_log2", "batch_pool_mib" (states and gradient partials of
+ * the circuits of a batch that run together; default 16384, less where the
+ * device has no room for it), "batch_wgs_per_cu" (1..16, without
  * effect: a batch's launches fill the chip), "graph" (0/1: replay forward
  * passes from a captured hipGraph), "half_lds" (0/1, default 1: forward
  * passes of the default tile shapes split their LDS transposes in two

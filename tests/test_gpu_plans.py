@@ -134,3 +134,18 @@ def test_threads_share_plans(native):
     for t in ts:
         t.join(timeout=100)
     assert not any(t.is_alive() for t in ts) and not bad, bad
+
+
+@pytest.mark.parametrize("mib", [1, 2, 6])
+def test_batch_in_groups(native, mib):
+    """Groups of one circuit, of a few and of all of them: the same results to the bit."""
+    print(f"case batch groups {mib} MiB", flush=True)
+    circuits = wl.batch_workload(24, 97, n_range=(9, 14), layer_range=(1, 3))
+    want = batch_forward_adjoint(circuits)
+    native.tune_set("batch_pool_mib", mib)
+    try:
+        got = batch_forward_adjoint(circuits)
+    finally:
+        native.tune_set("batch_pool_mib", -1)
+    assert np.array_equal(got[0], want[0])
+    assert all(np.array_equal(x, y) for x, y in zip(got[1], want[1]))

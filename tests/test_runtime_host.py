@@ -238,3 +238,26 @@ c = build(n, wl.layered_circuit(n, 2, 1))
 c.forward()
 c.gradient(np.ones(n))
 """, str(tmp_path / "tune.jsonl"), str(n))
+
+
+def test_batch_takes_the_memory_there_is(stand_in):
+    """64 circuits that take 20 MiB together, with more and more left on the device."""
+    run(stand_in, r"""
+from damavand_amd import batch_forward_adjoint
+circuits = wl.batch_workload(64, 5, n_range=(12, 14), layer_range=(2, 4))
+N.synchronize()
+S.stand_in_capacity(1 << 18)  # not even room for one circuit
+try:
+    batch_forward_adjoint(circuits)
+    assert False
+except N.OutOfDeviceMemory:
+    pass
+launches = []
+for mib in (3, 8, 16, 64):
+    S.stand_in_capacity(mib << 20)
+    before = S.stand_in_launches()
+    batch_forward_adjoint(circuits)
+    launches.append(S.stand_in_launches() - before)
+assert S.stand_in_bad_launches() == 0
+assert launches[0] > launches[1] > launches[2] > launches[3], launches
+""")
