@@ -10,6 +10,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <unordered_map>
 #include <vector>
@@ -264,7 +265,7 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
                           kBatchMaxIp);
         return DMV_OK;
     };
-    // fn(i) for i < total, on up to 16 threads taking `grain` at a time or more
+    // fn(i) for i < total, on up to 16 threads with `grain` of them each or more
     auto on_threads = [](int total, int grain, const std::function<void(int)> &fn) {
         const int hw = (int)std::max(1u, std::thread::hardware_concurrency());
         const int nthreads = std::max(1, std::min({hw, 16, total / grain}));
@@ -274,8 +275,12 @@ int batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_of
                 fn(i);
         };
         std::vector<std::thread> pool;
-        for (int t = 1; t < nthreads; t++)
-            pool.emplace_back(worker);
+        try {
+            for (int t = 1; t < nthreads; t++)
+                pool.emplace_back(worker);
+        } catch (const std::system_error &) {
+            // no more threads to be had: the work is shared by those there are
+        }
         worker();
         for (std::thread &t : pool)
             t.join();

@@ -261,3 +261,23 @@ for mib in (3, 8, 16, 64):
 assert S.stand_in_bad_launches() == 0
 assert launches[0] > launches[1] > launches[2] > launches[3], launches
 """)
+
+
+def test_batch_without_threads():
+    """The host threads of a batch are a matter of speed: none can be made here, since their stacks exceed the address
+    space that is left.  (No stand-in: the call ends when it finds no GPU.)"""
+    code = r"""
+import resource
+from damavand_amd import _native as N, workloads as wl, batch_forward_adjoint
+circuits = wl.batch_workload(64, 5, n_range=(3, 5), layer_range=(1, 2))
+N.device_count()
+size = next(int(l.split()[1]) for l in open("/proc/self/status") if l.startswith("VmSize")) << 10
+resource.setrlimit(resource.RLIMIT_AS, (size + (6 << 20),) * 2)
+try:
+    batch_forward_adjoint(circuits)
+except N.NoDeviceError:
+    pass
+"""
+    r = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, PYTHONPATH=ROOT, HIP_VISIBLE_DEVICES="-1"),
+                       capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
