@@ -99,3 +99,48 @@ def test_reverse_plan_within_its_partials(kib, most):
     assert sorted(s for p in per_pass for s in p) == list(range(sum(g[0] in wl.PARAMETRIC for g in gates)))
     want = TileEmulator(free).reverse(psi, lam)[2]
     np.testing.assert_allclose(TileEmulator(plan).reverse(psi, lam)[2], want, atol=1e-11)
+
+
+def exact_amplitudes(n, ops):
+    """State after (matrix, control mask, target) ops, in 80 bits."""
+    v = np.zeros(1 << n, dtype=np.clongdouble)
+    v[0] = 1
+    idx = np.arange(1 << n)
+    for m, ctrl, target in ops:
+        m = np.asarray(m, dtype=np.clongdouble)
+        w = v.reshape(-1, 2, 1 << target)
+        x, y = w[:, 0], w[:, 1]
+        out = np.stack([m[0, 0] * x + m[0, 1] * y, m[1, 0] * x + m[1, 1] * y], axis=1).reshape(-1)
+        v = np.where((idx & ctrl) == ctrl, out, v) if ctrl else out
+    return v
+
+
+def exact_u3(th, ph, la):
+    def e(x):
+        return np.cos(np.longdouble(x)) + 1j * np.sin(np.longdouble(x))
+
+    c, s = np.cos(np.longdouble(th) / 2), np.sin(np.longdouble(th) / 2)
+    return [[c, -e(la) * s], [e(ph) * s, e(np.longdouble(ph) + np.longdouble(la)) * c]]
+
+
+def test_special_unitary_matrices_lose_nothing():
+    """U3 gates (any determinant) and CNOTs.  The matrices of complex128 plans, phases taken out and put back, against
+    the merged gates as they are (the ops of complex64 plans): they are no further from the exact state, on the
+    geometric mean of eight circuits."""
+    ratios = []
+    for seed in range(8):
+        n, rng = 9 + seed % 3, np.random.default_rng(40 + seed)
+        gates = []
+        for _ in range(3 + 2 * seed):
+            gates += [(wl.GATE_U3, -1, q, tuple(rng.uniform(0, 2 * math.pi, 3))) for q in range(n)]
+            gates += [(wl.GATE_CNOT, q, q + 1, ()) for q in range(0, n - 1, 2)]
+        want = exact_amplitudes(n, [([[0, 1], [1, 0]], 1 << c, t) if k == wl.GATE_CNOT else (exact_u3(*p), 0, t)
+                                    for k, c, t, p in gates])
+        nc = NativeCircuit(n, gates)
+        error = []
+        for dtype in (N.C128, N.C64):
+            _, target, ctrl, m, _ = nc.plan_ops(dtype=dtype)
+            got = exact_amplitudes(n, [(x, int(c), int(t)) for x, c, t in zip(m, ctrl, target)])
+            error.append(np.sqrt((np.abs(got - want) ** 2).sum()))
+        ratios.append(float(error[0] / error[1]))
+    assert np.exp(np.log(ratios).mean()) <= 1.0, ratios
