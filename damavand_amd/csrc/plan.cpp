@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <unordered_map>
 
@@ -741,47 +742,63 @@ static int phases_cost(const std::vector<Ph> &phs, const std::vector<HostOp> &lo
     return c;
 }
 
-// Phases in op order: registers go to the first targets that come along.
-static void first_fit_phases(const std::vector<HostOp> &loc, const PlanParams &pp, std::vector<Ph> *out)
+// Phases in op order: registers go to the first targets that come along.  A
+// phase looks only at the next op of every bit (the oldest first): what lies behind one that
+// does not fit cannot run either.  (A walk over all ops left, once per phase,
+// took 0.5 s for a 10-qubit circuit of 98000 gates, which is one pass.)
+static void first_fit_phases(const std::vector<SchedOp> &ops, const PlanParams &pp, std::vector<Ph> *out)
 {
+    Frontier F;
+    F.build(ops, pp.k);
+    auto ready = [&](int i) {
+        for (uint64_t m = ops[(size_t)i].bits; m; m &= m - 1)
+            if (F.next(F.at, __builtin_ctzll(m)) != i)
+                return false;
+        return true;
+    };
     out->clear();
-    std::vector<char> used(loc.size(), 0);
-    size_t left = loc.size(), first = 0;
-    while (left > 0) {
-        Ph ph{0u, {}};
-        uint64_t blocked = 0;
-        for (size_t i = first; i < loc.size(); i++) {
-            if (used[i])
-                continue;
-            const uint64_t qs = op_qubits(loc[i]), tb = uint64_t(1) << loc[i].target;
-            const bool reg = op_needs_register(loc[i].kind);
-            if ((qs & blocked) || (reg && !(ph.rs & tb) && popcount64(ph.rs) >= pp.rlog)) {
-                blocked |= qs;
-                continue;
+    std::vector<int> heap;  // ops that come next on all their bits
+    auto offer = [&](uint64_t bits) {
+        for (uint64_t m = bits; m; m &= m - 1) {
+            const int q = __builtin_ctzll(m), i = F.next(F.at, q);
+            if (i >= 0 && (ops[(size_t)i].bits & bits & ((uint64_t(1) << q) - 1)) == 0 && ready(i)) {
+                heap.push_back(i);
+                std::push_heap(heap.begin(), heap.end(), std::greater<int>());
             }
-            if (reg)
-                ph.rs |= (uint32_t)tb;
-            ph.ops.push_back((int)i);
-            used[i] = 1;
-            left--;
         }
-        while (first < loc.size() && used[first])
-            first++;
+    };
+    for (size_t left = ops.size(); left > 0;) {
+        Ph ph{0u, {}};
+        offer((uint64_t(1) << pp.k) - 1);
+        while (!heap.empty()) {
+            std::pop_heap(heap.begin(), heap.end(), std::greater<int>());
+            const int i = heap.back();
+            heap.pop_back();
+            const SchedOp &op = ops[(size_t)i];
+            if (op_needs_register(op.kind)) {
+                const uint32_t tb = 1u << op.target;
+                if (!(ph.rs & tb) && popcount64(ph.rs) >= pp.rlog)
+                    continue;
+                ph.rs |= tb;
+            }
+            ph.ops.push_back(i);
+            left--;
+            for (uint64_t m = op.bits; m; m &= m - 1)
+                F.at[__builtin_ctzll(m)]++;
+            offer(op.bits);
+        }
         out->push_back(std::move(ph));
     }
 }
 
-static bool split_phases(const std::vector<HostOp> &loc, const PlanParams &pp, bool renames_only, bool high_first,
+static bool split_phases(const std::vector<SchedOp> &so, const PlanParams &pp, bool renames_only, bool high_first,
                          std::vector<Ph> *out)
 {
-    std::vector<SchedOp> so(loc.size());
-    for (size_t i = 0; i < loc.size(); i++)
-        so[i] = SchedOp{op_qubits(loc[i]), loc[i].ctrl, loc[i].target, loc[i].kind, op_weight(loc[i]), 0};
     Frontier F;
     F.build(so, pp.k);
     const SchedLimits none;
     const uint64_t all = (uint64_t(1) << pp.k) - 1, low = (uint64_t(1) << pp.low_bits) - 1;
-    size_t left = loc.size();
+    size_t left = so.size();
     out->clear();
     while (left > 0) {
         const uint64_t allowed = out->empty() && high_first ? all & ~low : all;
@@ -807,8 +824,8 @@ static bool split_phases(const std::vector<HostOp> &loc, const PlanParams &pp, b
         // register bits that no pair op of the phase needs are free again
         uint32_t used = 0;
         for (int i : ph.ops)
-            if (op_needs_register(loc[(size_t)i].kind))
-                used |= (uint32_t)(op_qubits(loc[(size_t)i]) & t.bits);
+            if (op_needs_register(so[(size_t)i].kind))
+                used |= (uint32_t)(so[(size_t)i].bits & t.bits);
         ph.rs = used;
         out->push_back(std::move(ph));
     }
@@ -856,11 +873,14 @@ static int cut_pass(uint64_t Q, const std::vector<HostOp> &ops, const std::vecto
     // they only relabel, or done in place; the first phase's registers off the
     // low bits, which saves the load's transpose, or anywhere).
     const uint32_t lowmask = (1u << pp.low_bits) - 1;
-    first_fit_phases(C.loc, pp, &C.phs);
+    std::vector<SchedOp> so(C.loc.size());
+    for (size_t i = 0; i < C.loc.size(); i++)
+        so[i] = SchedOp{op_qubits(C.loc[i]), C.loc[i].ctrl, C.loc[i].target, C.loc[i].kind, op_weight(C.loc[i]), 0};
+    first_fit_phases(so, pp, &C.phs);
     C.cost = phases_cost(C.phs, C.loc, lowmask);
     std::vector<Ph> trial;
     for (int way = 0; way < 4 && !first_fit; way++) {
-        if (!split_phases(C.loc, pp, (way & 1) == 0, (way & 2) != 0, &trial))
+        if (!split_phases(so, pp, (way & 1) == 0, (way & 2) != 0, &trial))
             continue;
         const int c = phases_cost(trial, C.loc, lowmask);
         if (c < C.cost) {

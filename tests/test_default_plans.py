@@ -2,6 +2,7 @@
 with their global phase, shapes by size, complex64 forwards in gate order),
 emulated on the CPU against the oracle."""
 import math
+import time
 
 import numpy as np
 import pytest
@@ -144,3 +145,17 @@ def test_special_unitary_matrices_lose_nothing():
             error.append(np.sqrt((np.abs(got - want) ** 2).sum()))
         ratios.append(float(error[0] / error[1]))
     assert np.exp(np.log(ratios).mean()) <= 1.0, ratios
+
+
+def test_planning_time_grows_with_the_gates():
+    """A state of one tile is one pass, however long the circuit: ten times the gates take about ten times as long to plan."""
+    n, best = 10, []
+    for layers in (200, 2000):
+        nc = NativeCircuit(n, wl.ansatz_circuit(n, layers, 3)[0])
+        times = []
+        for _ in range(3):
+            t = time.perf_counter()
+            assert nc.plan_stats()[0] == 1
+            times.append(time.perf_counter() - t)
+        best.append(min(times))
+    assert best[1] < 40 * best[0], best
