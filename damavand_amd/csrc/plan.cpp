@@ -726,19 +726,26 @@ struct Ph {
 // phase, a load or store transpose where the low qubits must leave the
 // registers, and an X or CNOT whose control is a thread bit (per-lane selects
 // of every register).
-static int phases_cost(const std::vector<Ph> &phs, const std::vector<HostOp> &loc, uint32_t lowmask)
+constexpr int kPhaseCost = 13, kTransposeCost = 13, kFarSwapCost = 6;
+
+static int phase_cost(const Ph &ph, const std::vector<SchedOp> &ops)
+{
+    int c = kPhaseCost;
+    for (int i : ph.ops)
+        if (ops[(size_t)i].kind == OP_SWAP && (ops[(size_t)i].ctrl & ~(uint64_t)ph.rs))
+            c += kFarSwapCost;
+    return c;
+}
+
+static int phases_cost(const std::vector<Ph> &phs, const std::vector<SchedOp> &ops, uint32_t lowmask)
 {
     int c = 0;
-    for (const Ph &ph : phs) {
-        c += 13;
-        for (int i : ph.ops)
-            if (loc[(size_t)i].kind == OP_SWAP && (loc[(size_t)i].ctrl & ~(uint64_t)ph.rs))
-                c += 6;
-    }
+    for (const Ph &ph : phs)
+        c += phase_cost(ph, ops);
     if (phs.front().rs & lowmask)
-        c += 13;
+        c += kTransposeCost;
     if (phs.back().rs & lowmask)
-        c += 13;
+        c += kTransposeCost;
     return c;
 }
 
@@ -746,10 +753,9 @@ static int phases_cost(const std::vector<Ph> &phs, const std::vector<HostOp> &lo
 // phase looks only at the next op of every bit (the oldest first): what lies behind one that
 // does not fit cannot run either.  (A walk over all ops left, once per phase,
 // took 0.5 s for a 10-qubit circuit of 98000 gates, which is one pass.)
-static void first_fit_phases(const std::vector<SchedOp> &ops, const PlanParams &pp, std::vector<Ph> *out)
+static void first_fit_phases(Frontier F, const PlanParams &pp, std::vector<Ph> *out)
 {
-    Frontier F;
-    F.build(ops, pp.k);
+    const std::vector<SchedOp> &ops = *F.ops;
     auto ready = [&](int i) {
         for (uint64_t m = ops[(size_t)i].bits; m; m &= m - 1)
             if (F.next(F.at, __builtin_ctzll(m)) != i)
@@ -791,14 +797,15 @@ static void first_fit_phases(const std::vector<SchedOp> &ops, const PlanParams &
     }
 }
 
-static bool split_phases(const std::vector<SchedOp> &so, const PlanParams &pp, bool renames_only, bool high_first,
+// Phases searched for (false: there are none, or they cost `limit` or more).
+static bool split_phases(Frontier F, const PlanParams &pp, bool renames_only, bool high_first, int limit,
                          std::vector<Ph> *out)
 {
-    Frontier F;
-    F.build(so, pp.k);
+    const std::vector<SchedOp> &so = *F.ops;
     const SchedLimits none;
     const uint64_t all = (uint64_t(1) << pp.k) - 1, low = (uint64_t(1) << pp.low_bits) - 1;
     size_t left = so.size();
+    int cost = 0;
     out->clear();
     while (left > 0) {
         const uint64_t allowed = out->empty() && high_first ? all & ~low : all;
@@ -808,12 +815,8 @@ static bool split_phases(const std::vector<SchedOp> &so, const PlanParams &pp, b
             only = false;  // only swaps with controls far away are left to run
             t = pick_bits<true>(F, none, false, pp.k, 0, allowed, pp.rlog);
         }
-        if (t.score == 0) {
-            if (high_first && out->empty())
-                return false;
-            set_error("internal: scheduler made no progress");
-            return false;
-        }
+        if (t.score == 0)
+            return false;  // nothing runs without the bits that are not allowed
         Ph ph{(uint32_t)t.bits, {}};
         Trial done;
         done.bits = t.bits;
@@ -827,6 +830,9 @@ static bool split_phases(const std::vector<SchedOp> &so, const PlanParams &pp, b
             if (op_needs_register(so[(size_t)i].kind))
                 used |= (uint32_t)(so[(size_t)i].bits & t.bits);
         ph.rs = used;
+        cost += phase_cost(ph, so) + (out->empty() && (used & low) ? kTransposeCost : 0);
+        if (cost >= limit)
+            return false;
         out->push_back(std::move(ph));
     }
     return true;
@@ -874,15 +880,22 @@ static int cut_pass(uint64_t Q, const std::vector<HostOp> &ops, const std::vecto
     // low bits, which saves the load's transpose, or anywhere).
     const uint32_t lowmask = (1u << pp.low_bits) - 1;
     std::vector<SchedOp> so(C.loc.size());
-    for (size_t i = 0; i < C.loc.size(); i++)
+    bool far_swaps = false;
+    for (size_t i = 0; i < C.loc.size(); i++) {
         so[i] = SchedOp{op_qubits(C.loc[i]), C.loc[i].ctrl, C.loc[i].target, C.loc[i].kind, op_weight(C.loc[i]), 0};
-    first_fit_phases(so, pp, &C.phs);
-    C.cost = phases_cost(C.phs, C.loc, lowmask);
+        far_swaps = far_swaps || (so[i].kind == OP_SWAP && so[i].ctrl);
+    }
+    Frontier F;
+    F.build(so, pp.k);
+    first_fit_phases(F, pp, &C.phs);
+    C.cost = phases_cost(C.phs, so, lowmask);
     std::vector<Ph> trial;
     for (int way = 0; way < 4 && !first_fit; way++) {
-        if (!split_phases(so, pp, (way & 1) == 0, (way & 2) != 0, &trial))
+        if ((way & 1) && !far_swaps)
+            continue;  // without such swaps this is the way before
+        if (!split_phases(F, pp, (way & 1) == 0, (way & 2) != 0, C.cost, &trial))
             continue;
-        const int c = phases_cost(trial, C.loc, lowmask);
+        const int c = phases_cost(trial, so, lowmask);
         if (c < C.cost) {
             C.cost = c;
             C.phs.swap(trial);
@@ -928,6 +941,7 @@ static int make_pass(const PassCut &C, const PlanParams &pp, Plan *plan)
     // the gapped state layout).
     const uint32_t default_rs = pad_regs(0u, pp, avoid);
     const bool mem_order = tune_value("memory_layouts", 0) != 0;
+    const bool renaming = tune_value("register_renaming", 1) != 0;
     const bool first_coalesced = (phs.front().rs & lowmask) == 0;
     const bool last_coalesced = (phs.back().rs & lowmask) == 0;
     P.lay_ld = make_layout(first_coalesced && !mem_order ? phs.front().rs : default_rs, pp, true, top);
@@ -995,7 +1009,7 @@ static int make_pass(const PassCut &C, const PlanParams &pp, Plan *plan)
                 return DMV_ERR_STATE;
             }
             // relabel-only X / CNOT: the map stays affine with at most one register control
-            if (h.kind == OP_SWAP && cthr == 0 && popcount64(creg) <= 1 && tune_value("register_renaming", 1)) {
+            if (h.kind == OP_SWAP && cthr == 0 && popcount64(creg) <= 1 && renaming) {
                 for (int q = 0; q < NR; q++)
                     if ((tab[q] & creg) == creg)
                         tab[q] ^= 1u << J;
@@ -1335,12 +1349,14 @@ int build_plan(const std::vector<HostOp> &given, const PlanParams &pp, Plan *out
     // against 532 us).  A CNOT ring, whose next layer waits for the whole ring,
     // takes as many passes either way.
     constexpr int kInOrder = 8;
+    const auto gens = std::count_if(so.begin(), so.end(), [](const SchedOp &op) { return op.kind == OP_GEN; });
     std::vector<PassCut> cuts;
     if (pp.fp32) {
         if (pp.gen_auto)
             DMV_TRY(in_order_budget(ops, pp, &lim.max_gen));
         DMV_TRY(first_fit_passes(ops, so, lim, pp, &cuts));
-    } else if (pp.gen_auto || pp.max_gen_per_pass <= kInOrder) {
+    } else if (pp.gen_auto ? pp.n > pp.k || gens <= kInOrder : pp.max_gen_per_pass <= kInOrder) {
+        // (not for a state of one tile if it takes passes in order: searched, it is one)
         if (pp.gen_auto)
             lim.max_gen = kInOrder;
         DMV_TRY(first_fit_passes(ops, so, lim, pp, &cuts));
