@@ -41,8 +41,14 @@ constexpr int kMaxQubits = 33;      // 2^33 complex128 = 128 GiB, one MI355X
 constexpr int kMaxRegs = 32;        // amplitudes per thread in a tile kernel
 constexpr int kMaxThreadBits = 9;   // up to 512 threads per tile workgroup
 constexpr int kMaxTileQubits = 13;  // 2^13 * 8 B (c64) or 2^12 * 16 B (c128) = 64 KiB of LDS
-constexpr int kSmallMaxQubits = 8;       // whole-state kernels: an amplitude per thread, in LDS
-constexpr int kSmallMaxQubitsFp32 = 13;  // ... of FP32 forward plans (64 KiB of LDS)
+// Whole-state kernels, the state in LDS: reverse sweeps with an amplitude per
+// thread, FP32 forward plans up to 64 KiB.  Complex128 forwards up to 10 qubits:
+// a tile plan runs them as fast or little faster (10 qubits, 4 layers: 50-57 us
+// either way; 20 layers: 185-212 us against 223) but has to be made first (4 layers:
+// 225 us for the first forward against 82).
+constexpr int kSmallMaxQubits = 8;
+constexpr int kSmallMaxQubitsFp32 = 13;
+constexpr int kSmallMaxQubitsFp64 = 10;
 
 inline int amp_bytes(int dtype) { return dtype == DMV_C64 ? 8 : 16; }
 // Low qubits a tile always keeps in lanes so that 8 consecutive lanes read one
@@ -268,7 +274,7 @@ inline DMV_HD uint64_t elem(uint64_t i, StateLayout L)
     return e;
 }
 
-static_assert(kSmallMaxQubits <= 17 && kSmallMaxQubitsFp32 <= 18,
+static_assert(kSmallMaxQubits <= 17 && kSmallMaxQubitsFp64 <= 17 && kSmallMaxQubitsFp32 <= 18,
               "whole-state kernels index states of the plain layout");
 static_assert(kMaxQubits - 17 <= 16, "span index wider than the swizzle");
 

@@ -13,7 +13,7 @@ __global__ void __launch_bounds__(kSmallThreads)
 k_small(typename Cplx<R>::T *__restrict__ state, uint32_t n, const DevOp *__restrict__ ops, uint32_t n_ops)
 {
     using V = typename Cplx<R>::T;
-    constexpr int CAP = 1 << (sizeof(V) == 8 ? kSmallMaxQubitsFp32 : kSmallMaxQubits);
+    constexpr int CAP = 1 << (sizeof(V) == 8 ? kSmallMaxQubitsFp32 : kSmallMaxQubitsFp64);
     __shared__ V s[CAP];
     const uint32_t n_amp = 1u << n;
     for (uint32_t i = threadIdx.x; i < n_amp; i += blockDim.x)
@@ -64,7 +64,7 @@ k_small_adjoint(typename Cplx<R>::T *__restrict__ psi, typename Cplx<R>::T *__re
 
 int launch_small(int dtype, void *state, int n, const DevOp *ops, uint32_t n_ops)
 {
-    const int cap = dtype == DMV_C64 ? kSmallMaxQubitsFp32 : kSmallMaxQubits;
+    const int cap = dtype == DMV_C64 ? kSmallMaxQubitsFp32 : kSmallMaxQubitsFp64;
     DMV_CHECK_ARG(n >= 1 && n <= cap, "whole-state kernel holds at most %d qubits", cap);
     if (dtype == DMV_C64)
         hipLaunchKernelGGL(k_small<float>, dim3(1), dim3(kSmallThreads), 0, stream(), (c64 *)state, (uint32_t)n, ops,

@@ -145,7 +145,7 @@ PlanParams tile_params(int n, int dtype, bool adjoint, StateLayout layout, const
 // States of up to this many qubits take the whole-state kernels.
 inline int small_qubits(int dtype, bool adjoint)
 {
-    return dtype == DMV_C64 && !adjoint ? kSmallMaxQubitsFp32 : kSmallMaxQubits;
+    return adjoint ? kSmallMaxQubits : dtype == DMV_C64 ? kSmallMaxQubitsFp32 : kSmallMaxQubitsFp64;
 }
 // How many IP ops a pass of a reverse sweep may hold.  Each takes a partial, a
 // double, per tile and wave: 16 MiB an op at 30 qubits.  A byte an amplitude (a

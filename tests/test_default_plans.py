@@ -149,8 +149,8 @@ def test_special_unitary_matrices_lose_nothing():
 
 def test_planning_time_grows_with_the_gates():
     """A state of one tile is one pass, however long the circuit: ten times the gates take about ten times as long to plan."""
-    n, best = 10, []
-    for layers in (200, 2000):
+    n, best = 12, []
+    for layers in (150, 1500):
         nc = NativeCircuit(n, wl.ansatz_circuit(n, layers, 3)[0])
         times = []
         for _ in range(3):
@@ -159,3 +159,10 @@ def test_planning_time_grows_with_the_gates():
             times.append(time.perf_counter() - t)
         best.append(min(times))
     assert best[1] < 40 * best[0], best
+
+
+@pytest.mark.parametrize("n,dtype,whole", [(10, N.C128, True), (11, N.C128, False), (13, N.C64, True), (14, N.C64, False)])
+def test_small_forwards_need_no_plan(n, dtype, whole):
+    """Up to 10 qubits (complex64 13) a forward is one launch that takes the ops in order."""
+    passes, phases, _, _ = NativeCircuit(n, wl.layered_circuit(n, 4, 1)).plan_stats(dtype=dtype)
+    assert ((passes, phases) == (1, 1)) == whole
