@@ -445,27 +445,43 @@ int max_ip_per_pass(const PlanParams &pp)
 void default_shape(int n, int dtype, bool adjoint, int *k, int *tlog)
 {
     const bool fp32 = dtype == DMV_C64 && !adjoint;
-    // 256 threads; k = 12 forward (FP32: 13), 11 for reverse sweeps, which hold
-    // psi and lambda in registers together
+    // large states: 256 threads; k = 12 forward (FP32: 13), 11 for reverse sweeps,
+    // which hold psi and lambda in registers together
     *k = adjoint ? 11 : (fp32 ? 13 : 12);
     *tlog = 8;
-    // Small states run 8 amplitudes per thread on every thread that their tiles
-    // have: with one tile a CU or fewer a pass is a chain of latencies, which
-    // more waves overlap, and the 16-amplitude kernels' code (140 KiB) does not
-    // stay in the instruction cache.  16 qubits, 8 layers: 160 us on 11-qubit
-    // tiles against 204 on 12-qubit ones and 209 on one-wave 9-qubit ones; 20
-    // qubits: 377 us on 512 threads against 414 (11-qubit tiles) and 474 (12, 16
-    // amplitudes per thread), which win from 23 qubits on (27: 21.6 ms against
-    // 22.4).  Up to 12 qubits (reverse sweeps 11) the whole state is one tile, so
-    // a plan is one pass (12 qubits: 96 us against 104 in passes of 11).
     if (fp32) {
         if (n < 19) {
             *tlog = 6;
             *k = 10;
         }
-    } else if (n <= (adjoint ? 24 : 20)) {
-        *k = adjoint || (n > 12 && n < 20) ? std::min(n, 11) : std::min(n, 12);
-        *tlog = *k <= 9 ? 6 : (*k == 12 ? 9 : 8);
+        return;
+    }
+    // Small states run 8 amplitudes per thread on every thread that their tiles
+    // have: with one tile a CU or fewer a pass is a chain of latencies, which
+    // more waves overlap, and the 16-amplitude kernels' code (140 KiB) does not
+    // stay in the instruction cache.  Up to 12 qubits (reverse sweeps 11) the
+    // whole state is one tile, so a plan is one pass (12 qubits: 96 us against 104
+    // in passes of 11).  With fewer 12-qubit tiles than the chip has CUs, 11-qubit
+    // ones keep more of them busy; with one a CU, 12-qubit ones take fewer
+    // passes.  6 layers of the layered, ansatz and random circuits, us:
+    //   qubits   11 on 256       12 on 512       12 on 256 threads
+    //     18     100  147   87   120  155   88   135  171  108
+    //     19     116  191  101   137  199  103   151  217  128
+    //     20     210  304  173   215  273  169   205  291  203
+    //     21     236  302  188   193  304  175   223  332  207
+    //     22     391  590  360   384  584  352   374  572  392
+    //     24    1334 1817 1183  1534 1852 1230  1299 1710 1124
+    // From 21 qubits on the shape is 12 on 256 threads, the documented default of
+    // large states, though 512 are faster at 21.
+    constexpr int kCusLog2 = 8;
+    const int most = adjoint ? 11 : 12;
+    if (n <= most) {
+        *k = n;
+        *tlog = n <= 9 ? 6 : (n == 12 ? 9 : 8);
+    } else if (!adjoint && n - 12 < kCusLog2) {
+        *k = 11;
+    } else if (!adjoint && n - 12 == kCusLog2) {
+        *tlog = 9;
     }
 }
 

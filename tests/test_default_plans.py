@@ -166,3 +166,14 @@ def test_small_forwards_need_no_plan(n, dtype, whole):
     """Up to 10 qubits (complex64 13) a forward is one launch that takes the ops in order."""
     passes, phases, _, _ = NativeCircuit(n, wl.layered_circuit(n, 4, 1)).plan_stats(dtype=dtype)
     assert ((passes, phases) == (1, 1)) == whole
+
+
+def test_default_forward_plan_of_a_large_state():
+    """21 qubits: 16 amplitudes a thread, passes searched with and without a bit to split their transposes by."""
+    n = 21
+    gates = random_gates(np.random.default_rng(21), n, 90)
+    nc = NativeCircuit(n, gates)
+    plan = plan_json(nc.h)
+    assert (plan["k"], plan["tlog"]) == (12, 8)
+    got = TileEmulator(plan).forward(zero_state(n))
+    np.testing.assert_allclose(got, oracle.run_gates(n, gates).amp, atol=1e-12)
