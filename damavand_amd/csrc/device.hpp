@@ -139,6 +139,5 @@ int check_launch(const char *what);
 int64_t tune_value(const char *name, int64_t dflt);
 int gate_pairs_per_thread();
 bool gate_nontemporal(uint32_t target, int dtype);
-int device_cus();  // compute units of the current device
 
 }  // namespace dmv

@@ -12,7 +12,7 @@ namespace dmv {
 
 // The pass `level` of a circuit's forward, over its tiles.  Level 0 starts from
 // |0> in registers instead of reading it.  complex64 (S = float) is computed in
-// FP64 as in the other tile kernels.
+// FP64, as in reverse sweeps (see tile_body).
 template <class S, int RLOG, int TLOG, bool STREAM>
 __global__ void __launch_bounds__(1 << TLOG)
 k_batch_forward(const BatchCircuit *__restrict__ circ, const BatchTile *__restrict__ tiles, uint32_t level,
@@ -87,7 +87,6 @@ k_batch_obs(const BatchCircuit *__restrict__ circ, const BatchTile *__restrict__
 
 // One partial per (IP op of the circuit, tile, wave).
 struct BatchSink {
-    static constexpr bool kPerWave = true;
     double *parts;  // of the pass's first IP op, at this tile
     uint64_t per_ip;
     __device__ void operator()(const DevOp *op, double v, uint32_t wave) const
@@ -105,15 +104,14 @@ k_batch_reverse(const BatchCircuit *__restrict__ circ, const BatchTile *__restri
 {
     constexpr uint32_t W = (1u << TLOG) / 64;
     __shared__ c128 lds[1 << (RLOG + TLOG)];
-    __shared__ double red[W];
     const BatchTile T = tiles[blockIdx.x];
     const BatchCircuit *C = circ + T.circuit;
     const DevPass *P = passes + C->adj_begin + level;
     const uint64_t per_ip = (uint64_t)C->tiles * W;
     BatchSink sink{parts + C->parts + P->ip_begin * per_ip + (uint64_t)T.tile * W, per_ip};
     typename Cplx<S>::T *psi = pool + C->state;
-    tile_body_adjoint<S, double, RLOG, TLOG, STREAM>(psi, psi + C->amps, P, phases, ops + C->adj_ops, T.tile, lds, red,
-                                                     sink, kPlainLayout);
+    tile_body_adjoint<S, double, RLOG, TLOG, STREAM>(psi, psi + C->amps, P, phases, ops + C->adj_ops, T.tile, lds, sink,
+                                                     kPlainLayout);
 }
 
 // A circuit's gradient entries and energy: a wave per IP op, in a fixed order.

@@ -10,7 +10,6 @@ namespace dmv {
 // among them): one value per wave of every tile, reduced by the host's
 // per-pass slot sums, so the buffer holds one pass's IP ops only.
 struct PartialSink {
-    static constexpr bool kPerWave = true;
     double *partials;
     uint64_t per_ip, base;  // per_ip = tiles x waves, base = tile x waves
     __device__ void operator()(const DevOp *op, double v, uint32_t wave) const
@@ -27,10 +26,9 @@ k_tile_adjoint(typename Cplx<S>::T *__restrict__ psi, typename Cplx<S>::T *__res
 {
     using V = typename Cplx<R>::T;
     __shared__ V lds[1 << (RLOG + TLOG)];
-    __shared__ double red[(1 << TLOG) / 64];
     constexpr uint32_t W = (1u << TLOG) / 64;
     PartialSink sink{partials, (uint64_t)gridDim.x * W, (uint64_t)blockIdx.x * W};
-    tile_body_adjoint<S, R, RLOG, TLOG, NT>(psi, lam, passes + pass_idx, phases, ops, blockIdx.x, lds, red, sink, L);
+    tile_body_adjoint<S, R, RLOG, TLOG, NT>(psi, lam, passes + pass_idx, phases, ops, blockIdx.x, lds, sink, L);
 }
 
 // complex64 states are computed in FP64 as in the forward passes (tile_body).

@@ -28,8 +28,9 @@ int launch_small(int dtype, void *state, int n, const DevOp *ops, uint32_t n_ops
 int launch_small_adjoint(int dtype, void *psi, void *lam, int n, const DevOp *ops, uint32_t n_ops,
                          double *partials);
 // Batched circuits (k_batch.hip): launches over the tiles of all circuits.
-// IP ops (gradient outputs) of one reverse pass of a circuit of more qubits than
-// a tile; the host rejects plans with more.
+// IP ops (gradient outputs) of one reverse pass of a circuit of at least a tile's
+// qubits: the interface's limit.  The host plans for it and rejects a run of more
+// on one qubit, which stays together.
 constexpr uint32_t kBatchMaxIp = 128;
 struct BatchCircuit {
     uint32_t n;

@@ -106,21 +106,6 @@ int ensure_device()
 
 hipStream_t stream() { return t_capture ? t_capture : ctx().stream; }
 
-int device_cus()
-{
-    static std::atomic<int> cus{0};
-    int c = cus.load(std::memory_order_relaxed);
-    if (c == 0) {
-        hipDeviceProp_t prop;
-        if (hipGetDeviceProperties(&prop, ctx().device) == hipSuccess && prop.multiProcessorCount > 0)
-            c = prop.multiProcessorCount;
-        else
-            c = 256;
-        cus.store(c, std::memory_order_relaxed);
-    }
-    return c;
-}
-
 int check_launch(const char *what)
 {
     hipError_t e = hipGetLastError();

@@ -774,8 +774,8 @@ __device__ __forceinline__ void ip_sums(const V (&p)[1 << RLOG], const V (&l)[1 
 }
 
 // One tile of a reverse-sweep pass over psi and lambda.  For every IP op the
-// sum over each wave (Sink::kPerWave) or over the workgroup is handed to
-// sink(op, value, wave) by the first lane of the wave / thread 0.  The ops
+// sum over each wave is handed to sink(op, value, wave) by the wave's first
+// lane: lane moves only, no workgroup barrier.  The ops
 // are applied in place, to psi and then to lambda: an out-of-place loop over
 // two states (four register arrays, or three with one run of ops per state
 // between IP ops) needed more registers or twice the code and ran slower.
@@ -785,11 +785,11 @@ __device__ __forceinline__ void tile_body_adjoint(typename Cplx<S>::T *__restric
                                                   typename Cplx<S>::T *__restrict__ lam, const DevPass *P,
                                                   const DevPhase *__restrict__ phases,
                                                   const DevOp *__restrict__ ops, uint64_t tile,
-                                                  typename Cplx<R>::T *lds, double *red, Sink sink, StateLayout L)
+                                                  typename Cplx<R>::T *lds, Sink sink, StateLayout L)
 {
     using V = typename Cplx<R>::T;
     using ST = typename Cplx<S>::T;
-    constexpr int NR = 1 << RLOG, K = RLOG + TLOG, NT = 1 << TLOG;
+    constexpr int NR = 1 << RLOG, K = RLOG + TLOG;
     const uint32_t tid = threadIdx.x;
     const uint64_t g = tile_base<K>(P, tile);
     const uint64_t gl = g | thread_global_offset<TLOG>(P->gthr_ld, tid);
@@ -813,17 +813,9 @@ __device__ __forceinline__ void tile_body_adjoint(typename Cplx<S>::T *__restric
             if (op_is_ip(op->kind)) {
                 if (!op->plain)
                     ip_sums<V, RLOG>(p, l, op, tid, sx, sy, sz);
-                const double v = op->m[0] * sx + op->m[1] * sy + op->m[2] * sz;
-                if constexpr (Sink::kPerWave) {
-                    // one partial per wave: lane moves only, no workgroup barrier
-                    const double w = wave_sum_rows(v);
-                    if ((tid & 63) == 0)
-                        sink(op, w, tid >> 6);
-                } else {
-                    const double s = block_sum<NT>(v, red);
-                    if (tid == 0)
-                        sink(op, s, 0);
-                }
+                const double w = wave_sum_rows(op->m[0] * sx + op->m[1] * sy + op->m[2] * sz);
+                if ((tid & 63) == 0)
+                    sink(op, w, tid >> 6);
                 continue;
             }
             const bool hold = thread_controls_hold(op, tid);

@@ -308,8 +308,9 @@ int dmv_circuit_plan_json(dmv_circuit *c, int dtype, int adjoint, int tile_qubit
  * must be the exclusive prefix sum of the circuits' parameter counts
  * (param_offset[0] = 0), so grad holds sum_i (parameters of circuit i)
  * values; anything else returns DMV_ERR_ARG before the device is touched.
- * Circuits have 2 to 24 qubits, and a circuit's reverse sweep may hold at
- * most 128 parametrised gates in one fused pass; a batch with more returns DMV_ERR_ARG. */
+ * Circuits have 2 to 24 qubits.  A circuit of as many qubits as a tile (11 by
+ * default) or more may have at most 128 parametrised gates on one qubit between
+ * two of its two-qubit gates; a batch with more returns DMV_ERR_ARG. */
 int dmv_batch_forward_adjoint(int count, int dtype, const int *n, const int *gate_offset,
                               const int *gate_kind, const int *gate_control,
                               const int *gate_target, const double *gate_param,
@@ -377,12 +378,13 @@ int dmv_tune_get(const char *name, int64_t *value);
  *    defaults.
  * The candidates run on scratch states the call allocates (the caller's
  * states are left as they were) and no tunable is changed. */
-/* Times the fused forward of `c` for tile shapes x GEN budgets per pass
- * (then streaming stores on the best); writes the chosen tile qubits. */
+/* Times the fused forward of `c` for tile shapes x GEN budgets per pass (and
+ * none, the default), then streaming stores on the best; writes the chosen
+ * tile qubits. */
 int dmv_autotune(dmv_circuit *c, dmv_state *s, int *chosen_tile_qubits);
 /* The same for the reverse sweep of dmv_circuit_adjoint in `dtype`. */
 int dmv_autotune_adjoint(dmv_circuit *c, int dtype, int *chosen_tile_qubits);
-/* Times the batched kernel (tile shape x workgroups per CU) on this batch
+/* Times the batched kernels' tile shapes on this batch
  * (arguments as dmv_batch_forward_adjoint) and keeps the fastest in the
  * table under the qubits of its largest circuit. */
 int dmv_batch_autotune(int count, int dtype, const int *n, const int *gate_offset, const int *gate_kind,
@@ -393,7 +395,10 @@ int dmv_batch_autotune(int count, int dtype, const int *n, const int *gate_offse
  * Circuits keep their own choices. */
 int dmv_tune_forget(void);
 /* The tile shape the next forward (adjoint = 0) or reverse-sweep plan of `c`
- * in `dtype` will use, after the precedence above.  No device needed. */
+ * in `dtype` will use, after the precedence above.  No device needed.
+ * max_gen_per_pass is the budget that is set, or 0 for a tuned choice without
+ * one.  Where nothing is set it is what the gates in their order would take (8
+ * or 12; reverse sweeps 8), though complex128 passes are searched for without. */
 int dmv_circuit_tile_shape(dmv_circuit *c, int dtype, int adjoint, int *tile_qubits, int *threads_log2,
                            int *max_gen_per_pass, int *nontemporal);
 
