@@ -696,6 +696,7 @@ int dmv_circuit_clear(dmv_circuit *c)
     c->version++;
     c->tune_fwd = TuneChoice();  // tuned for the gates just removed
     c->tune_adj = TuneChoice();
+    c->max_ip = 0;
     return DMV_OK;
 }
 
