@@ -42,13 +42,15 @@ constexpr int kMaxRegs = 32;        // amplitudes per thread in a tile kernel
 constexpr int kMaxThreadBits = 9;   // up to 512 threads per tile workgroup
 constexpr int kMaxTileQubits = 13;  // 2^13 * 8 B (c64) or 2^12 * 16 B (c128) = 64 KiB of LDS
 // Whole-state kernels, the state in LDS: reverse sweeps with an amplitude per
-// thread, FP32 forward plans up to 64 KiB.  Complex128 forwards up to 10 qubits:
-// a tile plan runs them as fast or little faster (10 qubits, 4 layers: 50-57 us
-// either way; 20 layers: 185-212 us against 223) but has to be made first (4 layers:
-// 225 us for the first forward against 82).
+// thread, FP32 forward plans up to 64 KiB.  Complex128 forwards up to 9 qubits:
+// a tile plan is no faster there (4 layers: 42-45 us against 42) and has to be made
+// first (178 us for the first forward against 56).  At 10 qubits the plan's kernel
+// takes 40 us where gate by gate takes 45 (4 layers), 20 layers 185-212 us against
+// 224, so that a training step there is 2-5% shorter; its first forward takes 225 us
+// for 71.
 constexpr int kSmallMaxQubits = 8;
 constexpr int kSmallMaxQubitsFp32 = 13;
-constexpr int kSmallMaxQubitsFp64 = 10;
+constexpr int kSmallMaxQubitsFp64 = 9;
 
 inline int amp_bytes(int dtype) { return dtype == DMV_C64 ? 8 : 16; }
 // Low qubits a tile always keeps in lanes so that 8 consecutive lanes read one

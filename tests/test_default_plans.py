@@ -161,9 +161,9 @@ def test_planning_time_grows_with_the_gates():
     assert best[1] < 40 * best[0], best
 
 
-@pytest.mark.parametrize("n,dtype,whole", [(10, N.C128, True), (11, N.C128, False), (13, N.C64, True), (14, N.C64, False)])
+@pytest.mark.parametrize("n,dtype,whole", [(9, N.C128, True), (10, N.C128, False), (13, N.C64, True), (14, N.C64, False)])
 def test_small_forwards_need_no_plan(n, dtype, whole):
-    """Up to 10 qubits (complex64 13) a forward is one launch that takes the ops in order."""
+    """Up to 9 qubits (complex64 13) a forward is one launch that takes the ops in order."""
     passes, phases, _, _ = NativeCircuit(n, wl.layered_circuit(n, 4, 1)).plan_stats(dtype=dtype)
     assert ((passes, phases) == (1, 1)) == whole
 
